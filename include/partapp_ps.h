@@ -286,8 +286,9 @@ int ps_find_local_max(const float *grids_dev, const long long *offsets, const in
  * major: image = Tig * grid) by nearest scatter (interpolate = 0, TM_DIRECT)
  * or bilinear gather (TM_BILINEAR), with NO_CLASS_VALUE 0 where nothing
  * lands; then scores < 0 become 1e-4 and the log is taken (0 -> LOG_ZERO).
- * Writes log_unary_dev [n][height][width].  Allocates a workspace (8 bytes
- * per output cell for the scatter); synchronous. */
+ * Writes log_unary_dev [n][height][width].  Synchronous.  Allocates device
+ * memory only for more than 1440 slices (their warps) and for nearest warps
+ * that cannot be inverted or shrink extremely (8 bytes per output cell). */
 int ps_ingest_scores(const float *score_grid_dev, int n, int grid_height, int grid_width, const double *Tig,
                      int interpolate, int height, int width, float *log_unary_dev, void *stream);
 

@@ -11,6 +11,7 @@
 //   findObjectImageRotJoints does (objectdetect_findrot.cpp:834-845).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cfloat>
 #include <cmath>
 #include <string>
@@ -26,6 +27,7 @@ extern thread_local std::string g_last_error;
 namespace {
 
 constexpr int kIngThreads = 256;
+constexpr double kIngSlack = 1e-3;  // cells added around a pixel's preimage for rounding
 
 // clip_scores_fill then computeLogGrid of one value
 __device__ __forceinline__ float clip_log(float v) {
@@ -77,43 +79,190 @@ __global__ __launch_bounds__(kIngThreads) void k_ingest_finish(const unsigned lo
   }
 }
 
-// TM_BILINEAR: output pixel (x3, y3) samples its slice at inverse(Tig) (x3, y3)
-// (within 10 float epsilons of a grid point: that point; last row / column
-// and outside: NO_CLASS_VALUE)
-__global__ __launch_bounds__(kIngThreads) void k_ingest_gather(const float *__restrict__ grid,
-                                                               const double *__restrict__ mats, int n, int gh,
-                                                               int gw, int H, int W, float *__restrict__ out) {
-  const long long cells = (long long)H * W;
-  const long long total = n * cells;
-  const float eps10 = 10.0f * FLT_EPSILON;
-  for (long long i = (long long)blockIdx.x * kIngThreads + threadIdx.x; i < total;
-       i += (long long)gridDim.x * kIngThreads) {
-    const int s = (int)(i / cells);
-    const int rem = (int)(i - s * cells);
-    const int y3 = rem / W;
-    const int x3 = rem - y3 * W;
-    const double *m = mats + 6 * s;
-    const double x1 = m[0] * (double)x3 + m[1] * (double)y3 + m[2];
-    const double y1 = m[3] * (double)x3 + m[4] * (double)y3 + m[5];
-    const int ix = (int)floor(x1);
-    const int iy = (int)floor(y1);
-    float r = 0.0f;
-    if (ix >= 0 && ix < gw && iy >= 0 && iy < gh) {
-      const float a = (float)(x1 - (double)ix);
-      const float b = (float)(y1 - (double)iy);
-      const float *p = grid + (long long)s * gh * gw + (long long)iy * gw + ix;
-      if (a < eps10 && b < eps10) {
-        r = p[0];
-      } else if (ix < gw - 1 && iy < gh - 1) {
-        const float t0 = (1.0f - b) * (1.0f - a) * p[0];
-        const float t1 = (1.0f - b) * a * p[1];
-        const float t2 = b * (1.0f - a) * p[gw];
-        const float t3 = b * a * p[gw + 1];
-        r = t0 + t1 + t2 + t3;
+// A slice's warp, rows 0-1: grid -> image for TM_DIRECT, image -> grid for
+// TM_BILINEAR.
+struct IngestWarp {
+  double m[6];
+};
+// The warps of one launch, passed by value: no table in device memory to
+// allocate, fill and free around a call of some 100 us.
+struct IngestSlices {
+  static constexpr int kMax = 80;  // 48 bytes each, below the 4 KB of kernel arguments
+  IngestWarp one[kMax];
+};
+
+constexpr int kTile = 32;                    // output pixels per side of a block
+constexpr int kPix = kTile * kTile / kIngThreads;  // pixels of a thread, kTile / kPix rows apart
+
+// the inverse of a grid -> image warp, rows 0-1
+__host__ __device__ __forceinline__ void ingest_inverse(const double (&m)[6], double (&a)[6]) {
+  const double D = m[0] * m[4] - m[3] * m[1];
+  a[0] = m[4] / D;
+  a[1] = -m[1] / D;
+  a[3] = -m[3] / D;
+  a[4] = m[0] / D;
+  a[2] = -(a[0] * m[2] + a[1] * m[5]);
+  a[5] = -(a[3] * m[2] + a[4] * m[5]);
+}
+
+enum IngestMode : int { kIngBilinear = 0, kIngDirect = 1, kIngDirect4 = 2 };
+
+// One block per 32 x 32 output pixels of a slice, four rows of pixels per
+// thread, so that the cells a rotated block reads (46 x 46 at 45 degrees) stay
+// in its CU's cache; the blocks of a slice run behind one L2 (xcd_block).
+//
+// Direct (TM_DIRECT): the reference scatters source cell (x1, y1) to the
+// nearest pixel of Tig (x1, y1), the last cell of the x-outer, y-inner scan
+// staying.  Here pixel (ix, iy) looks for that cell itself: the cells that can
+// land on it lie in the box of half widths ex, ey about its preimage
+// (ingest_gather bounds both roundings), walked from the scan's end, and each
+// is tested with the scatter's own double arithmetic, so the same cell is
+// found.  Direct4: no box of the launch holds more than 2 x 2 cells (every
+// warp that does not shrink): the cells of all four pixels are tested and
+// their loads issued before any is used.  Bilinear (TM_BILINEAR): the sample
+// at inverse(Tig) (ix, iy) (within 10 float epsilons of a grid point: that
+// point; last row / column and outside: NO_CLASS_VALUE).
+//
+// Every cell is read once from HBM and every pixel written once: 240 slices of
+// 425 x 425 cells onto 300 x 300 pixels in 92 us (2.8 TB/s; a large copy
+// reaches 5.2), the rest being vector work on the warp (147 us with every test
+// in double).  The scatter into 64-bit keys took 575 us, with clearing and
+// reading the keys 646 us, and several ms of allocating 172 MB for them.
+template <int MODE>
+__global__ __launch_bounds__(kIngThreads) void k_ingest_tile(const float *__restrict__ grid, IngestSlices sl,
+                                                             const IngestWarp *__restrict__ tab, int first, int gh,
+                                                             int gw, int H, int W, int tile0, int xtiles,
+                                                             float *__restrict__ out) {
+  unsigned bx, by;
+  xcd_block(bx, by);
+  IngestWarp S;  // from the arguments, or from the table where a call has very many slices
+  if (tab) S = tab[by];
+  else S = sl.one[by];
+  const int s = first + (int)by;
+  const int ty = (tile0 + (int)bx) / xtiles;
+  const unsigned x = (unsigned)(tile0 + (int)bx - ty * xtiles) * kTile + (threadIdx.x & 31);
+  const unsigned y0 = (unsigned)ty * kTile + (threadIdx.x >> 5);
+  if (x >= (unsigned)W) return;
+  const float *src = grid + (long long)s * gh * gw;
+  float *dst = out + (long long)s * H * W + x;
+  const double m0 = S.m[0], m1 = S.m[1], m2 = S.m[2], m3 = S.m[3], m4 = S.m[4], m5 = S.m[5];
+  const double xd = (double)x;
+  if (MODE != kIngBilinear) {
+    double a[6];
+    ingest_inverse(S.m, a);
+    const double ex = 0.5 * (fabs(a[0]) + fabs(a[1])) + kIngSlack, ey = 0.5 * (fabs(a[3]) + fabs(a[4])) + kIngSlack;
+    // floor(x3 + 0.5) == x and floor(y3 + 0.5) == y of cell (x1, y1)
+    auto lands = [&](double p, double q, double y1, double yd) {
+      const double tx = (p + m1 * y1 + m2) + 0.5, t3 = (q + m4 * y1 + m5) + 0.5;
+      return tx >= xd && tx < xd + 1.0 && t3 >= yd && t3 < yd + 1.0;
+    };
+    if (MODE == kIngDirect4) {
+      // a cell's landing point relative to the pixel's centre, in float from
+      // the fractions of the double preimage: off by less than tol, so only a
+      // cell that close to the pixel's edge takes the double test
+      const float n0 = (float)m0, n1 = (float)m1, n3 = (float)m3, n4 = (float)m4;
+      const float tolx = 1e-6f * (1.0f + fabsf(n0) + fabsf(n1)), toly = 1e-6f * (1.0f + fabsf(n3) + fabsf(n4));
+      float c[kPix][4];
+#pragma unroll
+      for (int k = 0; k < kPix; ++k) {
+        const double yd = (double)(y0 + k * (kTile / kPix));
+        const double cx = a[0] * xd + a[1] * yd + a[2], cy = a[3] * xd + a[4] * yd + a[5];
+        const double xh = floor(cx + ex), yh = floor(cy + ey);  // the box's last column and row
+        const float fx = (float)(xh - cx), fy = (float)(yh - cy);
+        const int xi = (int)xh, yi = (int)yh;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int x1 = xi - (j >> 1), y1 = yi - (j & 1);
+          const float u = fx - (float)(j >> 1), w = fy - (float)(j & 1);
+          const float dx = fabsf(n0 * u + n1 * w) - 0.5f, dy = fabsf(n3 * u + n4 * w) - 0.5f;
+          c[k][j] = 0.0f;
+          if ((unsigned)x1 < (unsigned)gw && (unsigned)y1 < (unsigned)gh && dx < tolx && dy < toly) {
+            bool hit = true;
+            if (dx > -tolx || dy > -toly) hit = lands(m0 * (double)x1, m3 * (double)x1, (double)y1, yd);
+            if (hit) c[k][j] = src[(long long)y1 * gw + x1];
+          }
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < kPix; ++k) {
+        const unsigned y = y0 + k * (kTile / kPix);
+        // NO_CLASS_VALUE is not written
+        const float v = c[k][0] != 0.0f ? c[k][0] : c[k][1] != 0.0f ? c[k][1] : c[k][2] != 0.0f ? c[k][2] : c[k][3];
+        if (y < (unsigned)H) dst[(long long)y * W] = clip_log(v);
+      }
+    } else {
+      for (int k = 0; k < kPix; ++k) {
+        const unsigned y = y0 + k * (kTile / kPix);
+        if (y >= (unsigned)H) break;
+        const double yd = (double)y;
+        const double cx = a[0] * xd + a[1] * yd + a[2], cy = a[3] * xd + a[4] * yd + a[5];
+        const int x_hi = (int)fmin(floor(cx + ex), (double)(gw - 1)), x_lo = (int)fmax(ceil(cx - ex), 0.0);
+        const int y_hi = (int)fmin(floor(cy + ey), (double)(gh - 1)), y_lo = (int)fmax(ceil(cy - ey), 0.0);
+        float v = 0.0f;
+        for (int x1 = x_hi; x1 >= x_lo && v == 0.0f; --x1) {
+          const double p = m0 * (double)x1, q = m3 * (double)x1;
+          for (int y1 = y_hi; y1 >= y_lo; --y1)
+            if (lands(p, q, (double)y1, yd)) {
+              v = src[(long long)y1 * gw + x1];
+              if (v != 0.0f) break;
+            }
+        }
+        dst[(long long)y * W] = clip_log(v);
       }
     }
-    out[i] = clip_log(r);
+  } else {
+    const float eps10 = 10.0f * FLT_EPSILON;
+#pragma unroll
+    for (int k = 0; k < kPix; ++k) {
+      const unsigned y = y0 + k * (kTile / kPix);
+      if (y >= (unsigned)H) break;
+      const double x1 = m0 * xd + m1 * (double)y + m2;
+      const double y1 = m3 * xd + m4 * (double)y + m5;
+      const int ix = (int)floor(x1);
+      const int iy = (int)floor(y1);
+      float r = 0.0f;
+      if (ix >= 0 && ix < gw && iy >= 0 && iy < gh) {
+        const float a = (float)(x1 - (double)ix);
+        const float b = (float)(y1 - (double)iy);
+        const float *p = src + (long long)iy * gw + ix;
+        if (a < eps10 && b < eps10) {
+          r = p[0];
+        } else if (ix < gw - 1 && iy < gh - 1) {
+          const float t0 = (1.0f - b) * (1.0f - a) * p[0];
+          const float t1 = (1.0f - b) * a * p[1];
+          const float t2 = b * (1.0f - a) * p[gw];
+          const float t3 = b * a * p[gw + 1];
+          r = t0 + t1 + t2 + t3;
+        }
+      }
+      dst[(long long)y * W] = clip_log(r);
+    }
   }
+}
+
+// Whether the scatter of a slice with warp m (grid -> image) can be taken as
+// a gather; four: its boxes hold at most 2 x 2 cells.  The cells of a pixel lie within
+// half the absolute row sums of the inverse about its preimage, plus what
+// rounding adds: of the inverse (cancellation in its determinant) and of the
+// forward map, both bounded here and required to stay far below the slack
+// that the kernel adds.  A test costs some 0.3 ps of the chip and an atomic of
+// the scatter 14-30 ps, and a pixel has |det a| atomics: the gather takes
+// boxes of up to 64 cells per atomic (beyond, an extreme shear), and of at
+// most 4096 (a thread's serial walk).  Measured on 48 slices onto 300 x 300
+// pixels, scatter against gather: 120 and 21 us without shrinking, 2.4 ms and 89 us at
+// 1 / 4, 9.8 ms and 109 us at 1 / 8 (boxes of some 130 cells).
+bool ingest_gather(const double (&m)[6], int gh, int gw, int H, int W, bool &four) {
+  double a[6];
+  ingest_inverse(m, a);
+  const double D = std::fabs(m[0] * m[4] - m[3] * m[1]);
+  const double cancel = std::fabs(m[0] * m[4]) + std::fabs(m[3] * m[1]);
+  const double ax = std::fabs(a[0]) + std::fabs(a[1]), ay = std::fabs(a[3]) + std::fabs(a[4]);
+  const double reach = (double)W + (double)H + std::fabs(m[2]) + std::fabs(m[5]) + 2.0;
+  const double fwd = (std::fabs(m[0]) + std::fabs(m[3]) + 1.0) * gw + (std::fabs(m[1]) + std::fabs(m[4]) + 1.0) * gh;
+  const double err = 32.0 * 2.220446049250313e-16 * (ax + ay) * (reach * (1.0 + cancel / D) + fwd);
+  const double box = (ax + 2.0) * (ay + 2.0);
+  four = std::max(ax, ay) + 2.0 * kIngSlack < 2.0;
+  return std::isfinite(err) && err < 0.01 * kIngSlack && box <= 64.0 * (1.0 + 1.0 / D) && box <= 4096.0;
 }
 
 }  // namespace ps
@@ -140,11 +289,55 @@ extern "C" int ps_ingest_scores(const float *score_grid_dev, int n, int grid_hei
   std::vector<double> mats(6 * (size_t)n);
   for (int s = 0; s < n; ++s) warp_matrix(Tig + 9 * s, interpolate != 0, mats.data() + 6 * s);
   hipStream_t st = static_cast<hipStream_t>(stream);
+  std::vector<IngestWarp> warps(n);
+  for (int s = 0; s < n; ++s) std::copy(&mats[6 * (size_t)s], &mats[6 * (size_t)s] + 6, warps[s].m);
+  bool gather = true, four = true;
+  for (int s = 0; s < n && !interpolate && gather; ++s) {
+    bool f = false;
+    gather = ingest_gather(warps[s].m, grid_height, grid_width, height, width, f);
+    four = four && f;
+  }
+  if (gather) {
+    // up to 1440 slices (10 parts x 3 scales x 48 rotations) ride in the
+    // arguments of at most 18 launches; more come from a table
+    IngestWarp *tab = nullptr;
+    hipError_t eg = hipSuccess;
+    if (n > 18 * IngestSlices::kMax) {
+      if (hipMalloc(&tab, sizeof(IngestWarp) * n) != hipSuccess)
+        return set_error(PS_ERR_OUT_OF_MEMORY, "ingest workspace");
+      eg = hipMemcpyAsync(tab, warps.data(), sizeof(IngestWarp) * n, hipMemcpyHostToDevice, st);
+    }
+    const int xtiles = (width + kTile - 1) / kTile, step = tab ? 32768 : IngestSlices::kMax;
+    const long long tiles = (long long)xtiles * ((height + kTile - 1) / kTile);
+    constexpr long long kTiles = 1ll << 22;  // tiles of one launch
+    for (int s0 = 0; s0 < n; s0 += step) {
+      IngestSlices sl;
+      const int ns = std::min(n - s0, step);
+      if (!tab) std::copy(warps.begin() + s0, warps.begin() + s0 + ns, sl.one);
+      for (long long t0 = 0; t0 < tiles && eg == hipSuccess; t0 += kTiles) {
+        const dim3 grid((unsigned)std::min(kTiles, tiles - t0), (unsigned)ns), blk(kIngThreads);
+        const IngestWarp *t = tab ? tab + s0 : nullptr;
+        auto launch = [&](auto kernel) {
+          hipLaunchKernelGGL(kernel, grid, blk, 0, st, score_grid_dev, sl, t, s0, grid_height, grid_width, height,
+                             width, (int)t0, xtiles, log_unary_dev);
+        };
+        if (interpolate) launch(k_ingest_tile<kIngBilinear>);
+        else if (four) launch(k_ingest_tile<kIngDirect4>);
+        else launch(k_ingest_tile<kIngDirect>);
+        eg = hipGetLastError();
+      }
+    }
+    if (eg == hipSuccess) eg = hipStreamSynchronize(st);
+    if (tab) (void)hipFree(tab);
+    if (eg != hipSuccess) return set_error(PS_ERR_HIP, std::string("ingest: ") + hipGetErrorString(eg));
+    return PS_OK;
+  }
+  // some slice's warp is singular, too ill-conditioned or shrinks too much
+  // for the gather: scatter with last-writer keys
   const long long out_n = (long long)n * height * width;
   const size_t mat_bytes = (mats.size() * sizeof(double) + 255) & ~(size_t)255;
-  const size_t key_bytes = interpolate ? 0 : (size_t)out_n * sizeof(unsigned long long);
   void *ws = nullptr;
-  hipError_t e = hipMalloc(&ws, mat_bytes + key_bytes);
+  hipError_t e = hipMalloc(&ws, mat_bytes + (size_t)out_n * sizeof(unsigned long long));
   if (e != hipSuccess) return set_error(PS_ERR_OUT_OF_MEMORY, "ingest workspace");
   double *mats_dev = static_cast<double *>(ws);
   unsigned long long *keys = reinterpret_cast<unsigned long long *>(static_cast<char *>(ws) + mat_bytes);
@@ -154,17 +347,11 @@ extern "C" int ps_ingest_scores(const float *score_grid_dev, int n, int grid_hei
     return (unsigned)(g < 8192 ? (g < 1 ? 1 : g) : 8192);
   };
   if (e == hipSuccess) {
-    if (interpolate) {
-      hipLaunchKernelGGL(k_ingest_gather, dim3(blocks(out_n)), dim3(kIngThreads), 0, st, score_grid_dev, mats_dev, n,
-                         grid_height, grid_width, height, width, log_unary_dev);
-    } else {
-      const long long in_n = (long long)n * grid_height * grid_width;
-      hipLaunchKernelGGL(k_ingest_clear, dim3(blocks(out_n)), dim3(kIngThreads), 0, st, keys, out_n);
-      hipLaunchKernelGGL(k_ingest_scatter, dim3(blocks(in_n)), dim3(kIngThreads), 0, st, score_grid_dev, mats_dev, n,
-                         grid_height, grid_width, height, width, keys);
-      hipLaunchKernelGGL(k_ingest_finish, dim3(blocks(out_n)), dim3(kIngThreads), 0, st, keys, out_n,
-                         log_unary_dev);
-    }
+    const long long in_n = (long long)n * grid_height * grid_width;
+    hipLaunchKernelGGL(k_ingest_clear, dim3(blocks(out_n)), dim3(kIngThreads), 0, st, keys, out_n);
+    hipLaunchKernelGGL(k_ingest_scatter, dim3(blocks(in_n)), dim3(kIngThreads), 0, st, score_grid_dev, mats_dev, n,
+                       grid_height, grid_width, height, width, keys);
+    hipLaunchKernelGGL(k_ingest_finish, dim3(blocks(out_n)), dim3(kIngThreads), 0, st, keys, out_n, log_unary_dev);
     e = hipGetLastError();
   }
   if (e == hipSuccess) e = hipStreamSynchronize(st);
@@ -183,51 +370,71 @@ extern "C" int ps_ingest_scores(const float *score_grid_dev, int n, int grid_hei
 namespace ps {
 namespace {
 
-// setTorsoPosPrior (objectdetect_icps.cpp:137-191): one thread per pixel
-// forms the clipped log prior once, then adds it to every slice.
+// Slices per thread of the two adds below: a thread forms its pixel's term
+// once for kAddSlices slices, whose loads are all in flight together (one
+// thread per pixel with every slice in turn waits for each load: 8.5 and 11.9
+// us per 24 x 300 x 300 grid, now 7.0 and 6.7).
+constexpr int kAddSlices = 6;
+
+// setTorsoPosPrior (objectdetect_icps.cpp:137-191): the clipped log prior of a
+// pixel, added to its slices.
 __global__ __launch_bounds__(kIngThreads) void k_torso_prior(float *g, int n_slices, int H, int W, float mu_x,
                                                              float mu_y, float var_x, float var_y, float weight) {
   const long long hw = (long long)H * W;
   const long long i = (long long)blockIdx.x * kIngThreads + threadIdx.x;
   if (i >= hw) return;
-  const int iy = (int)(i / W), ix = (int)(i - (long long)iy * W);
-  const float img_c_x = (float)(0.5 * W), img_c_y = (float)(0.5 * H);
-  const float ix_rel = img_c_x - (float)ix;
-  const float iy_rel = img_c_y - (float)iy;
-  // pow(d, 2) of a float d is exact in double
-  const double dx = (double)(ix_rel - mu_x), dy = (double)(iy_rel - mu_y);
-  const float score_x = (float)exp(-0.5 * (dx * dx) / (double)var_x);
-  const float score_y = (float)exp(-0.5 * (dy * dy) / (double)var_y);
-  float score = weight * score_x * score_y;
-  if ((double)score < 1e-4) score = 1e-4f;
-  const double pred = (double)logf(score);
-  for (int k = 0; k < n_slices; ++k) {
-    float *p = g + (long long)k * hw + i;
-    *p = (float)((double)*p + pred);
+  for (int k0 = (int)blockIdx.y * kAddSlices; k0 < n_slices; k0 += (int)gridDim.y * kAddSlices) {
+    float v[kAddSlices];
+#pragma unroll
+    for (int j = 0; j < kAddSlices; ++j) v[j] = g[(long long)min(k0 + j, n_slices - 1) * hw + i];
+    const int iy = (int)(i / W), ix = (int)(i - (long long)iy * W);
+    const float img_c_x = (float)(0.5 * W), img_c_y = (float)(0.5 * H);
+    const float ix_rel = img_c_x - (float)ix;
+    const float iy_rel = img_c_y - (float)iy;
+    // pow(d, 2) of a float d is exact in double
+    const double dx = (double)(ix_rel - mu_x), dy = (double)(iy_rel - mu_y);
+    const float score_x = (float)exp(-0.5 * (dx * dx) / (double)var_x);
+    const float score_y = (float)exp(-0.5 * (dy * dy) / (double)var_y);
+    float score = weight * score_x * score_y;
+    if ((double)score < 1e-4) score = 1e-4f;
+    const double pred = (double)logf(score);
+#pragma unroll
+    for (int j = 0; j < kAddSlices; ++j)
+      if (k0 + j < n_slices) g[(long long)(k0 + j) * hw + i] = (float)((double)v[j] + pred);
   }
 }
 
 // addLoadDPMScore's accumulation (:469-484, raw scores), addDPMScore
 // (:490-524, log grids) and the torso path's computeLogGrid + addDPMScore
-// (objectdetect_findrot.cpp:896-903): one thread per pixel, all slices
+// (objectdetect_findrot.cpp:896-903)
 __global__ __launch_bounds__(kIngThreads) void k_dpm_add(float *g, int S, int R, int H, int W, const float *dpm,
                                                          int n_dpm, float weight, int mode, double log_clip) {
   const long long hw = (long long)H * W;
   const long long i = (long long)blockIdx.x * kIngThreads + threadIdx.x;
   if (i >= hw) return;
-  for (int s = 0; s < S; ++s)
-    for (int r = 0; r < R; ++r) {
-      float *p = g + ((long long)s * R + r) * hw + i;
+  const bool per_r = mode == PS_DPM_RAW ? n_dpm == R : n_dpm > 1;
+  const int n = S * R;
+  for (int k0 = (int)blockIdx.y * kAddSlices; k0 < n; k0 += (int)gridDim.y * kAddSlices) {
+    float v[kAddSlices], d[kAddSlices];
+#pragma unroll
+    for (int j = 0; j < kAddSlices; ++j) {
+      const int k = min(k0 + j, n - 1);
+      v[j] = g[(long long)k * hw + i];
+      d[j] = dpm[(long long)(per_r ? k % R : 0) * hw + i];
+    }
+#pragma unroll
+    for (int j = 0; j < kAddSlices; ++j) {
+      if (k0 + j >= n) break;
+      float *p = g + (long long)(k0 + j) * hw + i;
       if (mode == PS_DPM_RAW) {
-        const float val = dpm[(long long)(n_dpm == R ? r : 0) * hw + i];
-        const double add = (double)val > 1e-4 ? (double)(weight * logf(val)) : log_clip;
-        *p = (float)((double)*p + add);
+        const double add = (double)d[j] > 1e-4 ? (double)(weight * logf(d[j])) : log_clip;
+        *p = (float)((double)v[j] + add);
       } else {
-        float lv = dpm[(long long)(n_dpm > 1 ? r : 0) * hw + i];
-        if (mode == PS_DPM_LOG_OF_RAW) lv = lv == 0.0f ? kLogZero : logf(lv);
-        *p = *p + weight * lv;
+        const float lv = mode == PS_DPM_LOG_OF_RAW ? (d[j] == 0.0f ? kLogZero : logf(d[j])) : d[j];
+        *p = v[j] + weight * lv;
       }
     }
+  }
 }
 
 // addExtraUnary (:526-548)
@@ -236,7 +443,10 @@ __global__ __launch_bounds__(kIngThreads) void k_add_scaled(float *g, const floa
     g[i] = g[i] + weight * e[i];
 }
 
-unsigned pixel_blocks(long long hw) { return (unsigned)((hw + kIngThreads - 1) / kIngThreads); }
+dim3 pixel_blocks(long long hw, long long n_slices) {
+  return dim3((unsigned)((hw + kIngThreads - 1) / kIngThreads),
+              (unsigned)std::min<long long>((n_slices + kAddSlices - 1) / kAddSlices, 65535));
+}
 
 }  // namespace
 }  // namespace ps
@@ -247,7 +457,7 @@ extern "C" int ps_add_torso_pos_prior(float *root_unary_dev, int n_slices, int h
   if (n_slices < 1 || height < 1 || width < 1) return set_error(PS_ERR_INVALID_ARG, "counts and sizes must be >= 1");
   if ((long long)height * width >= (1ll << 40)) return set_error(PS_ERR_UNSUPPORTED, "grid too large");
   hipStream_t st = static_cast<hipStream_t>(stream);
-  hipLaunchKernelGGL(k_torso_prior, dim3(pixel_blocks((long long)height * width)), dim3(kIngThreads), 0, st,
+  hipLaunchKernelGGL(k_torso_prior, pixel_blocks((long long)height * width, n_slices), dim3(kIngThreads), 0, st,
                      root_unary_dev, n_slices, height, width, (float)params[0], (float)params[1], (float)params[2],
                      (float)params[3], weight);
   hipError_t e = hipGetLastError();
@@ -267,7 +477,7 @@ extern "C" int ps_add_dpm_score(float *part_unary_dev, int S, int R, int height,
     if (n_dpm > 1 && n_dpm < R) return set_error(PS_ERR_INVALID_ARG, "a rotation-dependent DPM prior needs R grids");
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
-  hipLaunchKernelGGL(k_dpm_add, dim3(pixel_blocks((long long)height * width)), dim3(kIngThreads), 0, st,
+  hipLaunchKernelGGL(k_dpm_add, pixel_blocks((long long)height * width, (long long)S * R), dim3(kIngThreads), 0, st,
                      part_unary_dev, S, R, height, width, dpm_dev, n_dpm, weight, mode, std::log(1e-4));
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return set_error(PS_ERR_HIP, std::string("dpm score: ") + hipGetErrorString(e));
