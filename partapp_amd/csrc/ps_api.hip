@@ -36,8 +36,10 @@ hipError_t launch_rowpass(const Bases &b, const MsgJob *jobs, int n_jobs, const 
 size_t colpass_lds_bytes(int ky, int rows);
 hipError_t launch_colpass(const Bases &b, const MsgJob *jobs, int n_jobs, const float *taps, const int *shifts,
                           int R, int epi_hi, int max_w, size_t lds_bytes_16, hipStream_t s, int rows, bool split);
+void od_extent(OdExtent &e, int R, const MsgJob &j);
+hipError_t od_set_lds_limit(const OdExtent &ext);
 hipError_t launch_offdiag(const Bases &b, const MsgJob *jobs, int n_jobs, const float *taps, const int *shifts, int R,
-                          long long max_cells, long long max_hw, hipStream_t s);
+                          const OdExtent &ext, hipStream_t s);
 hipError_t launch_root(const Bases &b, const RootJob *jobs, int n_jobs, int k, int R, int max_hw, bool lse64,
                        hipStream_t s);
 size_t rowpass_mfma_lds_bytes(int R, int W, int kx, int KK, int terms);
@@ -102,7 +104,7 @@ struct Level {
   std::vector<WidthClass> col_classes;  // column passes: the same split further by epilogue kind
   size_t lds = 0;      // row pass
   size_t col_lds = 0;  // column pass
-  long long od_cells = 0, od_hw = 0;  // max R*th*tw and H*W of the off-diagonal jobs
+  OdExtent od_ext;     // launches of the off-diagonal jobs' eigenbasis stages
   bool mfma_ok = false;                // every diagonal job fits the BF16 Toeplitz passes
   size_t mfma_row_lds[3] = {0, 0, 0};  // 1, 2 and 3 terms
   size_t mfma_col_lds[3] = {0, 0, 0};
@@ -804,8 +806,7 @@ extern "C" int ps_plan_create(const ps_model *model, const ps_instance *instance
         L.max_w = std::max(L.max_w, j.W);
         L.lds = std::max(L.lds, rowpass_lds_bytes(R, j.W, j.kx));
         if (j.od) {
-          L.od_cells = std::max(L.od_cells, (long long)R * j.th * j.tw);
-          L.od_hw = std::max(L.od_hw, (long long)j.H * j.W);
+          od_extent(L.od_ext, R, j);
         } else {
           ++L.n_diag;
           L.col_lds = std::max(L.col_lds, colpass_lds_bytes(j.ky, 16));
@@ -954,6 +955,9 @@ extern "C" int ps_plan_create(const ps_model *model, const ps_instance *instance
         mcol = std::max(mcol, std::max(L.mfma_col_lds[2], L.mfma_col16_lds));
       }
   if (e == hipSuccess) e = mfma_set_lds_limit(mrow, mcol);
+  for (auto *lv : {&pl->up, &pl->down})
+    for (auto &L : *lv)
+      if (e == hipSuccess) e = od_set_lds_limit(L.od_ext);
   if (e != hipSuccess) {
     ps_plan_destroy(pl);
     return hip_error(e, "hipFuncSetAttribute");
@@ -1219,7 +1223,7 @@ static hipError_t sweep(ps_plan *pl, const Bases &b, int terms, int col_terms, p
     // the column pass class also times the eigenbasis stages
     if (e == hipSuccess && n_od > 0) {
       const long ev2 = profile_begin(pp, 3, s);
-      e = launch_offdiag(b, jobs + L.n_diag, n_od, pl->taps, pl->shifts, pl->R, L.od_cells, L.od_hw, s);
+      e = launch_offdiag(b, jobs + L.n_diag, n_od, pl->taps, pl->shifts, pl->R, L.od_ext, s);
       profile_end(pp, ev2, s);
     }
   };
@@ -1335,8 +1339,7 @@ static hipError_t sweep_subset(ps_plan *pl, const Bases &b, ps_map *map_dev, hip
     }
     if (e == hipSuccess && ls.od_col.count > 0) {
       const long ev2 = profile_begin(pp, 3, s);
-      e = launch_offdiag(b, jobs + ls.od_col.start, ls.od_col.count, pl->taps, pl->shifts, pl->R, L.od_cells,
-                         L.od_hw, s);
+      e = launch_offdiag(b, jobs + ls.od_col.start, ls.od_col.count, pl->taps, pl->shifts, pl->R, L.od_ext, s);
       profile_end(pp, ev2, s);
     }
   };
@@ -1562,7 +1565,7 @@ int message_prepare(const ps_model *model, int height, int width, const double o
   ms.W = width;
   ms.od = mp.od != 0;
   ms.split = mp.split;
-  ms.od_cells = mp.od ? (long long)R * mp.th * mp.tw : 0;
+  if (mp.od) od_extent(ms.od_ext, R, mj);
   ms.lds = rowpass_lds_bytes(R, width, mj.kx);
   ms.col_lds = mp.od ? 0 : colpass_lds_bytes(mp.ky, 16);
   if (ms.lds > kLdsLimit || ms.col_lds > kLdsLimit)
@@ -1622,14 +1625,14 @@ int message_enqueue(const MessageSetup &ms, char *mem, const float *child_dev, f
   const float *td = reinterpret_cast<const float *>(mem + ms.o_taps);
   const int *sd = reinterpret_cast<const int *>(mem + ms.o_sh);
   if (e == hipSuccess) e = rowpass_set_lds_limit(ms.lds);
-  if (e == hipSuccess && !ms.od) e = colpass_set_lds_limit(ms.col_lds);
+  if (e == hipSuccess) e = ms.od ? od_set_lds_limit(ms.od_ext) : colpass_set_lds_limit(ms.col_lds);
   if (e == hipSuccess) e = launch_reset(b, 1, 1, 1, nullptr, 0, s);
   if (e == hipSuccess)
     e = launch_max(b, reinterpret_cast<const MaxJob *>(mem + ms.o_max), 1, ms.R, ms.H * ms.W, s);
   if (e == hipSuccess) e = launch_rowpass(b, jd, 1, td, sd, ms.R, ms.H, ms.W, ms.lds, s, 0, ms.split);
   if (e == hipSuccess) {
     if (ms.od)
-      e = launch_offdiag(b, jd, 1, td, sd, ms.R, ms.od_cells, (long long)ms.H * ms.W, s);
+      e = launch_offdiag(b, jd, 1, td, sd, ms.R, ms.od_ext, s);
     else
       e = launch_colpass(b, jd, 1, td, sd, ms.R, ms.epi, ms.W, ms.col_lds, s, 0, ms.split);
   }

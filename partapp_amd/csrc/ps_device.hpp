@@ -106,6 +106,71 @@ __device__ __forceinline__ bool masked(const UnaryMask &m, int r, int x, int W) 
   return ((m.rot_bits >> r) & 1ull) || x < m.strip || x >= W - m.strip;
 }
 
+// The nearest scatter (TM_DIRECT, multi_array_transform.hpp:122-239) seen from
+// an output cell: which source cells (x1, y1) have
+// floor(m (x1, y1) + 0.5) = (x, y).  They lie within half the absolute row
+// sums of the inverse about the cell's preimage; kCellSlack covers what
+// rounding adds (the callers make sure that it does).
+constexpr double kCellSlack = 1e-3;
+
+// the inverse of an affine map, rows 0-1
+__host__ __device__ __forceinline__ void affine_inverse(const double *m, double (&a)[6]) {
+  const double D = m[0] * m[4] - m[3] * m[1];
+  a[0] = m[4] / D;
+  a[1] = -m[1] / D;
+  a[3] = -m[3] / D;
+  a[4] = m[0] / D;
+  a[2] = -(a[0] * m[2] + a[1] * m[5]);
+  a[5] = -(a[3] * m[2] + a[4] * m[5]);
+}
+
+struct CellWarp {
+  double m[6], a[6], ex, ey;
+  __device__ __forceinline__ explicit CellWarp(const double *map) {
+#pragma unroll
+    for (int i = 0; i < 6; ++i) m[i] = map[i];
+    affine_inverse(m, a);
+    ex = 0.5 * (fabs(a[0]) + fabs(a[1])) + kCellSlack;
+    ey = 0.5 * (fabs(a[3]) + fabs(a[4])) + kCellSlack;
+  }
+  // the scatter's own test of cell (x1, y1): p = m0 x1, q = m3 x1
+  __device__ __forceinline__ bool lands(double p, double q, double y1, double xd, double yd) const {
+    const double tx = (p + m[1] * y1 + m[2]) + 0.5, ty = (q + m[4] * y1 + m[5]) + 0.5;
+    return tx >= xd && tx < xd + 1.0 && ty >= yd && ty < yd + 1.0;
+  }
+  // Where the box holds at most 2 x 2 cells: their values (0 for a cell that
+  // does not land on (x, y) or lies outside), the scan's last first.  A
+  // cell's landing point relative to the output cell's centre is formed in
+  // float from the fractions of the double preimage, off by less than tol, so
+  // only a cell that close to the edge takes the double test.
+  __device__ __forceinline__ void load4(int x, int y, int gw, int gh, const float *src, int pitch,
+                                        float (&c)[4]) const {
+    const float n0 = (float)m[0], n1 = (float)m[1], n3 = (float)m[3], n4 = (float)m[4];
+    const float tolx = 1e-6f * (1.0f + fabsf(n0) + fabsf(n1)), toly = 1e-6f * (1.0f + fabsf(n3) + fabsf(n4));
+    const double xd = (double)x, yd = (double)y;
+    const double cx = a[0] * xd + a[1] * yd + a[2], cy = a[3] * xd + a[4] * yd + a[5];
+    const double xh = floor(cx + ex), yh = floor(cy + ey);  // the box's last column and row
+    const float fx = (float)(xh - cx), fy = (float)(yh - cy);
+    const int xi = (int)xh, yi = (int)yh;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int x1 = xi - (j >> 1), y1 = yi - (j & 1);
+      const float u = fx - (float)(j >> 1), w = fy - (float)(j & 1);
+      const float dx = fabsf(n0 * u + n1 * w) - 0.5f, dy = fabsf(n3 * u + n4 * w) - 0.5f;
+      c[j] = 0.0f;
+      if ((unsigned)x1 < (unsigned)gw && (unsigned)y1 < (unsigned)gh && dx < tolx && dy < toly) {
+        bool hit = true;
+        if (dx > -tolx || dy > -toly) hit = lands(m[0] * (double)x1, m[3] * (double)x1, (double)y1, xd, yd);
+        if (hit) c[j] = src[(long long)y1 * pitch + x1];
+      }
+    }
+  }
+};
+// the value that stays: the last of the scan that is not 0 (which is not written)
+__device__ __forceinline__ float last_cell(const float (&c)[4]) {
+  return c[0] != 0.0f ? c[0] : c[1] != 0.0f ? c[1] : c[2] != 0.0f ? c[2] : c[3];
+}
+
 // log of a filter response, 0 -> LOG_ZERO (multi_array_op.hpp:154-166), on
 // the hardware log2 (v_log_f32, about 1 ulp): a response the hardware takes
 // for 0 (below 2^-126 where it flushes) is LOG_ZERO too
@@ -237,19 +302,28 @@ __device__ __forceinline__ void dst_store(const MsgJob &J, float *dst, float *ds
   }
 }
 
+// Raise a key to v where it is lower: most waves only read it (same-address
+// atomics of a level's thousands of waves queue up at one cache line).
+__device__ __forceinline__ void raise_key(unsigned *k, unsigned v) {
+  if (__hip_atomic_load(k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < v) atomicMax(k, v);
+}
+__device__ __forceinline__ void raise_key(unsigned long long *k, unsigned long long v) {
+  if (__hip_atomic_load(k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < v) atomicMax(k, v);
+}
+
 // Wave reductions of DstAcc and one atomic per wave; every lane of the wave
 // calls it.
 __device__ __forceinline__ void dst_flush(const Bases &b, const MsgJob &J, bool has_dst2, DstAcc &a, int lane) {
   if (J.dst_kind == kDstUpNode) {
     const unsigned v = wave_max_u32(a.kmax1);
-    if (lane == 0 && v) atomicMax(b.max_keys + J.dst_key, v);
+    if (lane == 0 && v) raise_key(b.max_keys + J.dst_key, v);
   } else if (J.dst_kind == kDstDown) {
     const unsigned long long m = wave_max_u64(a.amax);
-    if (lane == 0 && m) atomicMax(b.map_keys + J.map_slot, m);
+    if (lane == 0 && m) raise_key(b.map_keys + J.map_slot, m);
     if (b.top2_keys) top2_flush(b.top2_keys + J.map_slot, (unsigned)(a.amax >> 32), a.second, lane);
     if (has_dst2) {
       const unsigned v = wave_max_u32(a.kmax2);
-      if (lane == 0 && v) atomicMax(b.max_keys + J.dst2_key, v);
+      if (lane == 0 && v) raise_key(b.max_keys + J.dst2_key, v);
     }
   }
 }

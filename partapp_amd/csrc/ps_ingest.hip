@@ -27,7 +27,6 @@ extern thread_local std::string g_last_error;
 namespace {
 
 constexpr int kIngThreads = 256;
-constexpr double kIngSlack = 1e-3;  // cells added around a pixel's preimage for rounding
 
 // clip_scores_fill then computeLogGrid of one value
 __device__ __forceinline__ float clip_log(float v) {
@@ -94,17 +93,6 @@ struct IngestSlices {
 constexpr int kTile = 32;                    // output pixels per side of a block
 constexpr int kPix = kTile * kTile / kIngThreads;  // pixels of a thread, kTile / kPix rows apart
 
-// the inverse of a grid -> image warp, rows 0-1
-__host__ __device__ __forceinline__ void ingest_inverse(const double (&m)[6], double (&a)[6]) {
-  const double D = m[0] * m[4] - m[3] * m[1];
-  a[0] = m[4] / D;
-  a[1] = -m[1] / D;
-  a[3] = -m[3] / D;
-  a[4] = m[0] / D;
-  a[2] = -(a[0] * m[2] + a[1] * m[5]);
-  a[5] = -(a[3] * m[2] + a[4] * m[5]);
-}
-
 enum IngestMode : int { kIngBilinear = 0, kIngDirect = 1, kIngDirect4 = 2 };
 
 // One block per 32 x 32 output pixels of a slice, four rows of pixels per
@@ -147,68 +135,35 @@ __global__ __launch_bounds__(kIngThreads) void k_ingest_tile(const float *__rest
   float *dst = out + (long long)s * H * W + x;
   const double m0 = S.m[0], m1 = S.m[1], m2 = S.m[2], m3 = S.m[3], m4 = S.m[4], m5 = S.m[5];
   const double xd = (double)x;
-  if (MODE != kIngBilinear) {
-    double a[6];
-    ingest_inverse(S.m, a);
-    const double ex = 0.5 * (fabs(a[0]) + fabs(a[1])) + kIngSlack, ey = 0.5 * (fabs(a[3]) + fabs(a[4])) + kIngSlack;
-    // floor(x3 + 0.5) == x and floor(y3 + 0.5) == y of cell (x1, y1)
-    auto lands = [&](double p, double q, double y1, double yd) {
-      const double tx = (p + m1 * y1 + m2) + 0.5, t3 = (q + m4 * y1 + m5) + 0.5;
-      return tx >= xd && tx < xd + 1.0 && t3 >= yd && t3 < yd + 1.0;
-    };
-    if (MODE == kIngDirect4) {
-      // a cell's landing point relative to the pixel's centre, in float from
-      // the fractions of the double preimage: off by less than tol, so only a
-      // cell that close to the pixel's edge takes the double test
-      const float n0 = (float)m0, n1 = (float)m1, n3 = (float)m3, n4 = (float)m4;
-      const float tolx = 1e-6f * (1.0f + fabsf(n0) + fabsf(n1)), toly = 1e-6f * (1.0f + fabsf(n3) + fabsf(n4));
-      float c[kPix][4];
+  if (MODE == kIngDirect4) {
+    const CellWarp cell(S.m);
+    float c[kPix][4];
 #pragma unroll
-      for (int k = 0; k < kPix; ++k) {
-        const double yd = (double)(y0 + k * (kTile / kPix));
-        const double cx = a[0] * xd + a[1] * yd + a[2], cy = a[3] * xd + a[4] * yd + a[5];
-        const double xh = floor(cx + ex), yh = floor(cy + ey);  // the box's last column and row
-        const float fx = (float)(xh - cx), fy = (float)(yh - cy);
-        const int xi = (int)xh, yi = (int)yh;
+    for (int k = 0; k < kPix; ++k) cell.load4((int)x, (int)(y0 + k * (kTile / kPix)), gw, gh, src, gw, c[k]);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int x1 = xi - (j >> 1), y1 = yi - (j & 1);
-          const float u = fx - (float)(j >> 1), w = fy - (float)(j & 1);
-          const float dx = fabsf(n0 * u + n1 * w) - 0.5f, dy = fabsf(n3 * u + n4 * w) - 0.5f;
-          c[k][j] = 0.0f;
-          if ((unsigned)x1 < (unsigned)gw && (unsigned)y1 < (unsigned)gh && dx < tolx && dy < toly) {
-            bool hit = true;
-            if (dx > -tolx || dy > -toly) hit = lands(m0 * (double)x1, m3 * (double)x1, (double)y1, yd);
-            if (hit) c[k][j] = src[(long long)y1 * gw + x1];
+    for (int k = 0; k < kPix; ++k) {
+      const unsigned y = y0 + k * (kTile / kPix);
+      if (y < (unsigned)H) dst[(long long)y * W] = clip_log(last_cell(c[k]));
+    }
+  } else if (MODE == kIngDirect) {
+    const CellWarp cell(S.m);
+    for (int k = 0; k < kPix; ++k) {
+      const unsigned y = y0 + k * (kTile / kPix);
+      if (y >= (unsigned)H) break;
+      const double yd = (double)y;
+      const double cx = cell.a[0] * xd + cell.a[1] * yd + cell.a[2], cy = cell.a[3] * xd + cell.a[4] * yd + cell.a[5];
+      const int x_hi = (int)fmin(floor(cx + cell.ex), (double)(gw - 1)), x_lo = (int)fmax(ceil(cx - cell.ex), 0.0);
+      const int y_hi = (int)fmin(floor(cy + cell.ey), (double)(gh - 1)), y_lo = (int)fmax(ceil(cy - cell.ey), 0.0);
+      float v = 0.0f;
+      for (int x1 = x_hi; x1 >= x_lo && v == 0.0f; --x1) {
+        const double p = m0 * (double)x1, q = m3 * (double)x1;
+        for (int y1 = y_hi; y1 >= y_lo; --y1)
+          if (cell.lands(p, q, (double)y1, xd, yd)) {
+            v = src[(long long)y1 * gw + x1];
+            if (v != 0.0f) break;  // NO_CLASS_VALUE is not written
           }
-        }
       }
-#pragma unroll
-      for (int k = 0; k < kPix; ++k) {
-        const unsigned y = y0 + k * (kTile / kPix);
-        // NO_CLASS_VALUE is not written
-        const float v = c[k][0] != 0.0f ? c[k][0] : c[k][1] != 0.0f ? c[k][1] : c[k][2] != 0.0f ? c[k][2] : c[k][3];
-        if (y < (unsigned)H) dst[(long long)y * W] = clip_log(v);
-      }
-    } else {
-      for (int k = 0; k < kPix; ++k) {
-        const unsigned y = y0 + k * (kTile / kPix);
-        if (y >= (unsigned)H) break;
-        const double yd = (double)y;
-        const double cx = a[0] * xd + a[1] * yd + a[2], cy = a[3] * xd + a[4] * yd + a[5];
-        const int x_hi = (int)fmin(floor(cx + ex), (double)(gw - 1)), x_lo = (int)fmax(ceil(cx - ex), 0.0);
-        const int y_hi = (int)fmin(floor(cy + ey), (double)(gh - 1)), y_lo = (int)fmax(ceil(cy - ey), 0.0);
-        float v = 0.0f;
-        for (int x1 = x_hi; x1 >= x_lo && v == 0.0f; --x1) {
-          const double p = m0 * (double)x1, q = m3 * (double)x1;
-          for (int y1 = y_hi; y1 >= y_lo; --y1)
-            if (lands(p, q, (double)y1, yd)) {
-              v = src[(long long)y1 * gw + x1];
-              if (v != 0.0f) break;
-            }
-        }
-        dst[(long long)y * W] = clip_log(v);
-      }
+      dst[(long long)y * W] = clip_log(v);
     }
   } else {
     const float eps10 = 10.0f * FLT_EPSILON;
@@ -253,7 +208,7 @@ __global__ __launch_bounds__(kIngThreads) void k_ingest_tile(const float *__rest
 // 1 / 4, 9.8 ms and 109 us at 1 / 8 (boxes of some 130 cells).
 bool ingest_gather(const double (&m)[6], int gh, int gw, int H, int W, bool &four) {
   double a[6];
-  ingest_inverse(m, a);
+  affine_inverse(m, a);
   const double D = std::fabs(m[0] * m[4] - m[3] * m[1]);
   const double cancel = std::fabs(m[0] * m[4]) + std::fabs(m[3] * m[1]);
   const double ax = std::fabs(a[0]) + std::fabs(a[1]), ay = std::fabs(a[3]) + std::fabs(a[4]);
@@ -261,8 +216,8 @@ bool ingest_gather(const double (&m)[6], int gh, int gw, int H, int W, bool &fou
   const double fwd = (std::fabs(m[0]) + std::fabs(m[3]) + 1.0) * gw + (std::fabs(m[1]) + std::fabs(m[4]) + 1.0) * gh;
   const double err = 32.0 * 2.220446049250313e-16 * (ax + ay) * (reach * (1.0 + cancel / D) + fwd);
   const double box = (ax + 2.0) * (ay + 2.0);
-  four = std::max(ax, ay) + 2.0 * kIngSlack < 2.0;
-  return std::isfinite(err) && err < 0.01 * kIngSlack && box <= 64.0 * (1.0 + 1.0 / D) && box <= 4096.0;
+  four = std::max(ax, ay) + 2.0 * kCellSlack < 2.0;
+  return std::isfinite(err) && err < 0.01 * kCellSlack && box <= 64.0 * (1.0 + 1.0 / D) && box <= 4096.0;
 }
 
 }  // namespace ps

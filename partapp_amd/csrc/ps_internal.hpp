@@ -114,7 +114,7 @@ struct MsgJob {
   int kxe, kye;    // half widths of the eigenbasis filters
   int taps_xe;     // offsets into the tap pool
   int taps_ye;
-  GridRef od_buf;  // floats: A[R][th][tw] (scatter keys: 2 floats per cell), then X[R][th][tw]
+  GridRef od_buf;  // floats: A[R][th][od_pitch(tw)], then X likewise
   // pruned execution: the destination part's keep flags, [R][keep_ty][keep_tx]
   // tiles of 64 x 64 starting at keep_off (bytes) in Bases::keep
   long long keep_off;
@@ -149,8 +149,20 @@ constexpr int f16_tap_copy_len(int KK) {
   return (256 * ((2 * (16 * KK + 32) - 64 + 255) / 256) + 64) / 2;
 }
 
-// floats of the eigenbasis scratch of one message
-inline long long od_scratch_floats(int R, int th, int tw) { return 3ll * R * th * tw; }
+// row pitch of an eigenbasis grid (16-byte rows where that costs at most the
+// scratch of three dense grids, i.e. not for a few columns)
+#if defined(__HIPCC__)
+__host__ __device__
+#endif
+inline int od_pitch(int tw) { return tw < 6 ? tw : (tw + 3) & ~3; }
+// floats of the eigenbasis scratch of one message: the filtered grid and the
+// x-filtered one
+inline long long od_scratch_floats(int R, int th, int tw) { return 2ll * R * th * od_pitch(tw); }
+// The largest launch of each eigenbasis stage over a set of jobs.
+struct OdExtent {
+  long long x_blocks = 0, y_blocks = 0, b_blocks = 0;
+  size_t x_lds = 0;
+};
 // row pitch of the row-pass output and of the plan's own grids: rows start
 // on 128-byte boundaries
 inline int t_pitch(int W) { return (W + 31) & ~31; }

@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "../../include/partapp_ps.h"
+#include "ps_internal.hpp"
 
 namespace ps {
 
@@ -18,7 +19,7 @@ struct MessageSetup {
   int R = 0, H = 0, W = 0;
   bool od = false;          // off-diagonal covariance: eigenbasis stages instead of the column pass
   bool split = false;       // a warp whose offset changes along an axis (MsgJob::split)
-  long long od_cells = 0;   // R * th * tw of the eigenbasis grid
+  OdExtent od_ext;          // launches of the eigenbasis stages
   size_t lds = 0, col_lds = 0;
   // byte offsets in the block: job, max job, taps, shifts, max key, argmax key, grids
   size_t o_job = 0, o_max = 0, o_taps = 0, o_sh = 0, o_key = 0, o_mk = 0, o_T = 0;
