@@ -354,6 +354,11 @@ enum { PS_JOINT_POS_GAUSSIAN = 1, PS_JOINT_ROT_GAUSSIAN = 2 };
 int ps_load_joint_mat(const char *path, int flip, ps_joint *out, int *type);
 
 /* --------------------------------------------------------------- utilities */
+/* The library keeps up to 1 GiB per device of the memory that destroyed plans
+ * and finished calls held, for the next ones (and gives it back by itself when
+ * an allocation of its own fails).  This frees what it keeps on the current
+ * device.  No reference counterpart. */
+int ps_release_memory(void);
 const char *ps_last_error_string(void);
 const char *ps_version(void);
 

@@ -149,6 +149,7 @@ SIGNATURES = {
     "ps_synth_unary_dev": (ctypes.c_int, [ctypes.c_ulonglong, ctypes.c_int, ctypes.c_int, ctypes.c_int,
                                           ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]),
     "ps_last_error_string": (ctypes.c_char_p, []),
+    "ps_release_memory": (ctypes.c_int, []),
     "ps_version": (ctypes.c_char_p, []),
     "ps_debug_message_plan": (ctypes.c_int, [ctypes.POINTER(ps_exp_param), ctypes.c_int, ctypes.c_int, c_double_p,
                                              c_double_p, c_double_p, ctypes.c_double, ctypes.c_double,

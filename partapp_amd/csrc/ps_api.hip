@@ -13,17 +13,21 @@
 #include <cmath>
 #include <cstdint>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <vector>
 
 #include "ps_internal.hpp"
 #include "ps_message.hpp"
 #include "ps_plan.hpp"
+#include "ps_pool.hpp"
 
 namespace ps {
 extern thread_local std::string g_last_error;
 hipError_t launch_reset(const Bases &b, int n_keys, int n_map, int n_inst, unsigned *flags, int n_flags,
                         hipStream_t s);
+hipError_t launch_upload(void *dst, const void *src, size_t bytes, hipStream_t s);
+hipError_t launch_fragments(const MsgJob *jobs, int n_jobs, const float *taps, int R, uint4 *frags, hipStream_t s);
 hipError_t launch_invert_flags(const unsigned *in, unsigned *out, int n, hipStream_t s);
 hipError_t launch_certify(const unsigned long long *top2, int n_map, int n_inst, float tau, unsigned *flags,
                           hipStream_t s);
@@ -113,19 +117,6 @@ struct Level {
   bool split = false;                  // some job's warp changes its offset along an axis
 };
 
-// Host bf16 of a float, round to nearest even (finite inputs).
-uint16_t bf16_rne(float f) {
-  uint32_t u;
-  std::memcpy(&u, &f, 4);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (uint16_t)(u >> 16);
-}
-float bf16_float(uint16_t h) {
-  const uint32_t u = (uint32_t)h << 16;
-  float f;
-  std::memcpy(&f, &u, 4);
-  return f;
-}
 // k-steps of 16 of a 32-wide Toeplitz tile with half width k
 int mfma_kk(int k) { return (32 + 2 * k + 15) / 16; }
 
@@ -139,11 +130,18 @@ int check_device(int &device) {
   int n = 0;
   if (hipGetDeviceCount(&n) != hipSuccess || n == 0) return set_error(PS_ERR_NO_DEVICE, "no HIP device");
   if (hipGetDevice(&device) != hipSuccess) return set_error(PS_ERR_NO_DEVICE, "hipGetDevice failed");
+  // the architecture of a device does not change: asked once per device (the
+  // properties take some 10 us to query)
+  static std::mutex mu;
+  static std::vector<int> known;  // devices seen to be gfx950
+  std::lock_guard<std::mutex> lock(mu);
+  if (std::find(known.begin(), known.end(), device) != known.end()) return PS_OK;
   hipDeviceProp_t prop;
   if (hipGetDeviceProperties(&prop, device) != hipSuccess)
     return set_error(PS_ERR_NO_DEVICE, "hipGetDeviceProperties failed");
   if (std::strncmp(prop.gcnArchName, "gfx950", 6) != 0)
     return set_error(PS_ERR_NO_DEVICE, std::string("library is built for gfx950, device is ") + prop.gcnArchName);
+  known.push_back(device);
   return PS_OK;
 }
 
@@ -170,7 +168,8 @@ struct ps_plan {
   MapJob *maps = nullptr;
   float *taps = nullptr;
   int *shifts = nullptr;
-  uint4 *frags = nullptr;
+  uint4 *frags = nullptr;  // formed when a BF16 method is first chosen
+  size_t frag_units = 0;
   int terms = 0;      // x pass: 0 FP32, else the BF16 Toeplitz terms (1, 2, 3)
   int col_terms = 0;  // y pass
   int mfma_rows = 4;  // output rows per block of the BF16 x pass (tunable)
@@ -271,92 +270,12 @@ struct Builder {
   std::vector<MapJob> maps;
   std::vector<float> taps;
   std::vector<int> shifts;
-  std::vector<uint16_t> frags;  // bf16 Toeplitz fragments, 8 per 16-byte unit
+  size_t frag_units = 0;  // 16-byte units of the fragment tables (k_fragments)
   explicit Builder(const Model &mm) : m(mm) {}
 
-  // Fragment tables of one filter for the BF16 passes: lane l at step kk holds
-  // f[16 kk + 8 (l / 32) + t - l % 32], t = 0..7 (zero off the band); the
-  // bf16 hi parts, then the lo parts (f - hi).  Returns the offset in 16-byte units.
-  int add_frags(const std::vector<float> &f, int KK) {
-    const int off = (int)(frags.size() / 8);
-    const int L = (int)f.size();
-    std::vector<uint16_t> lo;
-    lo.reserve((size_t)KK * 64 * 8);
-    for (int kk = 0; kk < KK; ++kk)
-      for (int l = 0; l < 64; ++l)
-        for (int t = 0; t < 8; ++t) {
-          const int i = 16 * kk + 8 * (l / 32) + t - l % 32;
-          const float v = (i >= 0 && i < L) ? f[i] : 0.0f;
-          const uint16_t hi = bf16_rne(v);
-          frags.push_back(hi);
-          lo.push_back(bf16_rne(v - bf16_float(hi)));
-        }
-    frags.insert(frags.end(), lo.begin(), lo.end());
-    return off;
-  }
-
-  // The y taps in fp16 (hi, then lo = f - hi) for the column pass that runs
-  // on the fp16 MFMA, as the 8 shifted copies of f16_tap_copy_len: part p,
-  // copy j, element e holds tap j + e - 32 (zero outside the filter).
-  int add_taps16(const std::vector<float> &f, int KK) {
-    const int off = (int)(frags.size() / 8);
-    const int L = (int)f.size(), Q = f16_tap_copy_len(KK);
-    std::vector<uint16_t> lo;
-    for (int j = 0; j < 8; ++j)
-      for (int e = 0; e < Q; ++e) {
-        const int i = j + e - 32;
-        const float v = (i >= 0 && i < L) ? f[i] : 0.0f;
-        const _Float16 hi = (_Float16)v;
-        const _Float16 lv = (_Float16)(v - (float)hi);
-        frags.push_back(__builtin_bit_cast(uint16_t, hi));
-        lo.push_back(__builtin_bit_cast(uint16_t, lv));
-      }
-    frags.insert(frags.end(), lo.begin(), lo.end());
-    return off;
-  }
-
-  // Rotation filter of a message as the A operand of the row pass's second
-  // GEMM, whose B operand is the x-filter accumulator itself: B position
-  // p = 16 kk + 8 h + t (lane half h, element t) holds slice
-  // 16 kk + 8 (t / 4) + 4 h + t % 4, so lane l, step kk, element t of the
-  // table is F[l % 32][that slice] with F[ro][s] the weight of source slice s
-  // in output slice ro (circular taps, objectdetect_findrot.cpp:377-420);
-  // zero for slices >= R.  The hi block, then the lo block.  With 48 slices
-  // there are two output tiles (ro = 32 mt + l % 32) and three k-steps: step
-  // ks reads the accumulator of slice tile ks / 2, so its B position holds
-  // slice 32 (ks / 2) + 16 (ks % 2) + 8 (t / 4) + 4 h + t % 4; the table is
-  // [mt][ks] per block.
-  int add_rot_frags(const MessagePlan &mp, int R, bool f16 = false) {
-    const int off = (int)(frags.size() / 8);
-    std::vector<float> F((size_t)R * R, 0.0f);
-    if (mp.rot_mode == kRotFilter) {
-      const int LR = (int)mp.rot_taps.size();
-      const int n = (LR - 1) / 2;
-      for (int ro = 0; ro < R; ++ro)
-        for (int j = 0; j < LR; ++j) F[(size_t)ro * R + (((ro - n + j) % R) + R) % R] += mp.rot_taps[j];
-    } else if (mp.rot_mode == kRotCopy) {
-      for (int ro = 0; ro < R; ++ro) F[(size_t)ro * R + ro] = 1.0f;
-    }
-    std::vector<uint16_t> lo;
-    const int MT = (R + 31) / 32, KS = (R + 15) / 16;
-    for (int mt = 0; mt < MT; ++mt)
-      for (int ks = 0; ks < KS; ++ks)
-        for (int l = 0; l < 64; ++l)
-          for (int t = 0; t < 8; ++t) {
-            const int ro = 32 * mt + l % 32, h = l / 32;
-            const int sl = 32 * (ks / 2) + 16 * (ks % 2) + 8 * (t / 4) + 4 * h + t % 4;
-            const float v = (ro < R && sl < R) ? F[(size_t)ro * R + sl] : 0.0f;
-            if (f16) {  // fp16 hi + lo
-              const _Float16 hi = (_Float16)v;
-              frags.push_back(__builtin_bit_cast(uint16_t, hi));
-              lo.push_back(__builtin_bit_cast(uint16_t, (_Float16)(v - (float)hi)));
-            } else {
-              const uint16_t hi = bf16_rne(v);
-              frags.push_back(hi);
-              lo.push_back(bf16_rne(v - bf16_float(hi)));
-            }
-          }
-    frags.insert(frags.end(), lo.begin(), lo.end());
+  int add_frags(int units) {
+    const int off = (int)frag_units;
+    frag_units += (size_t)units;
     return off;
   }
 
@@ -401,11 +320,15 @@ struct Builder {
       J.kk_x = mfma_kk(mp.kx);
       J.kk_y = mfma_kk(mp.ky);
       if (J.kk_x <= kMfmaMaxKK && J.kk_y <= kMfmaMaxKK) {
-        J.frag_x = add_frags(mp.fx, J.kk_x);
-        J.frag_y = add_frags(mp.fy, J.kk_y);
-        J.frag_y16 = add_taps16(mp.fy, J.kk_y);
-        J.frag_r = (R == 24 || R == 48) ? add_rot_frags(mp, R) : 0;
-        J.frag_r16 = (R == 24 || R == 48) ? add_rot_frags(mp, R, true) : 0;
+        // hi and lo parts of each table
+        J.frag_x = add_frags(2 * J.kk_x * 64);
+        J.frag_y = add_frags(2 * J.kk_y * 64);
+        J.frag_y16 = add_frags(2 * f16_tap_copy_len(J.kk_y));
+        if (R == 24 || R == 48) {
+          const int rot = 2 * ((R + 31) / 32) * ((R + 15) / 16) * 64;
+          J.frag_r = add_frags(rot);
+          J.frag_r16 = add_frags(rot);
+        }
         // the row-pass output is at most (sum of x taps) (largest row sum of
         // the rotation filter) times max exp(b - M) = 1; its fp16 copy holds
         // it scaled by 2^t16_shift, that bound (with margin) near 2^14
@@ -877,14 +800,13 @@ extern "C" int ps_plan_create(const ps_model *model, const ps_instance *instance
   size_t o_maps = align(o_maxes + B.maxes.size() * sizeof(MaxJob));
   size_t o_taps = align(o_maps + B.maps.size() * sizeof(MapJob));
   size_t o_shifts = align(o_taps + B.taps.size() * sizeof(float));
-  size_t o_frags = align(o_shifts + B.shifts.size() * sizeof(int));
-  size_t o_keys = align(o_frags + B.frags.size() * sizeof(uint16_t));
+  size_t o_keys = align(o_shifts + B.shifts.size() * sizeof(int));
   size_t o_mkeys = align(o_keys + (size_t)pl->n_keys * sizeof(unsigned));
   size_t o_top2 = align(o_mkeys + (size_t)pl->n_map * sizeof(unsigned long long));
   size_t o_flags = align(o_top2 + (size_t)pl->n_map * sizeof(unsigned long long));
   size_t o_nfb = align(o_flags + (size_t)n_instances * sizeof(unsigned));
   size_t total = align(o_nfb + (size_t)n_instances * sizeof(unsigned));
-  hipError_t e = hipMalloc(&pl->tables, total);
+  hipError_t e = pool_get(&pl->tables, total);
   if (e != hipSuccess) {
     delete pl;
     return set_error(PS_ERR_OUT_OF_MEMORY, "tables: " + std::string(hipGetErrorString(e)));
@@ -896,7 +818,7 @@ extern "C" int ps_plan_create(const ps_model *model, const ps_instance *instance
   pl->maps = reinterpret_cast<MapJob *>(base + o_maps);
   pl->taps = reinterpret_cast<float *>(base + o_taps);
   pl->shifts = reinterpret_cast<int *>(base + o_shifts);
-  pl->frags = reinterpret_cast<uint4 *>(base + o_frags);
+  pl->frag_units = B.frag_units;
   pl->keys = reinterpret_cast<unsigned *>(base + o_keys);
   pl->map_keys = reinterpret_cast<unsigned long long *>(base + o_mkeys);
   pl->top2 = reinterpret_cast<unsigned long long *>(base + o_top2);
@@ -909,29 +831,18 @@ extern "C" int ps_plan_create(const ps_model *model, const ps_instance *instance
   std::memcpy(host.data() + o_maps, B.maps.data(), B.maps.size() * sizeof(MapJob));
   std::memcpy(host.data() + o_taps, B.taps.data(), B.taps.size() * sizeof(float));
   std::memcpy(host.data() + o_shifts, B.shifts.data(), B.shifts.size() * sizeof(int));
-  std::memcpy(host.data() + o_frags, B.frags.data(), B.frags.size() * sizeof(uint16_t));
   e = hipMemcpy(pl->tables, host.data(), total, hipMemcpyHostToDevice);
   if (e == hipSuccess && pl->scratch_elems) {
-    e = hipMalloc(&pl->scratch, pl->scratch_elems * sizeof(float));
+    e = pool_get(&pl->scratch, pl->scratch_elems * sizeof(float));
     if (e != hipSuccess) {
-      (void)hipFree(pl->tables);
+      pool_put(pl->tables, true);
       delete pl;
-      return set_error(PS_ERR_OUT_OF_MEMORY, "scratch (" + std::to_string(pl->scratch_elems * 4) + " bytes): " + hipGetErrorString(e));
+      return set_error(PS_ERR_OUT_OF_MEMORY, "scratch (" + std::to_string(scratch_off * 4) + " bytes): " + hipGetErrorString(e));
     }
   }
-  if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void **>(&pl->flags_host), sizeof(unsigned) * n_instances);
-  // room for every job twice (row-pass and column-pass classes list the same
-  // jobs) and every root, max and map job, each part 256-byte aligned
-  pl->cbytes = align(2 * B.jobs.size() * sizeof(MsgJob)) + align(B.roots.size() * sizeof(RootJob)) +
-               align(B.maxes.size() * sizeof(MaxJob)) + align(B.maps.size() * sizeof(MapJob));
-  if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void **>(&pl->cstage), pl->cbytes);
-  if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&pl->ctables), pl->cbytes);
   if (e != hipSuccess) {
-    if (pl->ctables) (void)hipFree(pl->ctables);
-    if (pl->cstage) (void)hipHostFree(pl->cstage);
-    if (pl->flags_host) (void)hipHostFree(pl->flags_host);
-    if (pl->scratch) (void)hipFree(pl->scratch);
-    (void)hipFree(pl->tables);
+    pool_put(pl->scratch, false);
+    pool_put(pl->tables, false);
     delete pl;
     return hip_error(e, "plan upload");
   }
@@ -966,6 +877,55 @@ extern "C" int ps_plan_create(const ps_model *model, const ps_instance *instance
   return PS_OK;
 }
 
+namespace {
+// makes a plan's device current for a scope
+struct OnDevice {
+  int before = -1;
+  explicit OnDevice(int dev) {
+    if (hipGetDevice(&before) != hipSuccess || before == dev || hipSetDevice(dev) != hipSuccess) before = -1;
+  }
+  ~OnDevice() {
+    if (before >= 0) (void)hipSetDevice(before);
+  }
+};
+
+// the operand tables of the BF16 passes, complete on return (the plan may be
+// executed on any stream)
+int ensure_fragments(ps_plan *pl) {
+  if (pl->frags || pl->frag_units == 0) return PS_OK;
+  OnDevice on(pl->device);
+  uint4 *f = nullptr;
+  if (pool_get(&f, pl->frag_units * 16) != hipSuccess)
+    return set_error(PS_ERR_OUT_OF_MEMORY, "fragment tables (" + std::to_string(pl->frag_units * 16) + " bytes)");
+  hipError_t e = launch_fragments(pl->jobs, (int)pl->h_jobs.size(), pl->taps, pl->R, f, nullptr);
+  if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+  if (e != hipSuccess) {
+    pool_put(f, false);
+    return hip_error(e, "fragment tables");
+  }
+  pl->frags = f;
+  return PS_OK;
+}
+
+// what the MAP guard's eager re-sweep needs: a pinned copy of the flags, and a
+// staging block and its device twin with room for every job twice (row-pass
+// and column-pass classes list the same jobs) and every root, max and map
+// job, each part 256-byte aligned
+int ensure_guard(ps_plan *pl) {
+  if (pl->ctables) return PS_OK;
+  OnDevice on(pl->device);
+  auto align = [](size_t v) { return (v + 255) & ~(size_t)255; };
+  pl->cbytes = align(2 * pl->h_jobs.size() * sizeof(MsgJob)) + align(pl->h_roots.size() * sizeof(RootJob)) +
+               align(pl->h_maxes.size() * sizeof(MaxJob)) + align(pl->h_maps.size() * sizeof(MapJob));
+  hipError_t e = hipSuccess;
+  if (!pl->flags_host) e = hipHostMalloc(reinterpret_cast<void **>(&pl->flags_host), sizeof(unsigned) * pl->n_inst);
+  if (e == hipSuccess && !pl->cstage) e = hipHostMalloc(reinterpret_cast<void **>(&pl->cstage), pl->cbytes);
+  if (e == hipSuccess) e = pool_get(&pl->ctables, pl->cbytes);
+  if (e != hipSuccess) return set_error(PS_ERR_OUT_OF_MEMORY, std::string("MAP guard: ") + hipGetErrorString(e));
+  return PS_OK;
+}
+}  // namespace
+
 extern "C" int ps_plan_set_method(ps_plan *plan, int method) {
   if (!plan) return set_error(PS_ERR_INVALID_ARG, "plan is NULL");
   int terms, col_terms;
@@ -976,6 +936,10 @@ extern "C" int ps_plan_set_method(ps_plan *plan, int method) {
     case PS_METHOD_BF16X3: terms = col_terms = 3; break;
     case PS_METHOD_BF16_MIXED: terms = 1; col_terms = 3; break;
     default: return set_error(PS_ERR_INVALID_ARG, "unknown method " + std::to_string(method));
+  }
+  if (terms != 0) {
+    const int st = ensure_fragments(plan);
+    if (st != PS_OK) return st;
   }
   if ((terms != plan->terms || col_terms != plan->col_terms) && plan->gexec) {
     (void)hipGraphExecDestroy(plan->gexec);
@@ -989,6 +953,10 @@ extern "C" int ps_plan_set_method(ps_plan *plan, int method) {
 extern "C" int ps_plan_set_map_guard(ps_plan *plan, float tau) {
   if (!plan) return set_error(PS_ERR_INVALID_ARG, "plan is NULL");
   if (!(tau >= 0.0f) || !std::isfinite(tau)) return set_error(PS_ERR_INVALID_ARG, "tau must be finite and >= 0");
+  if (tau > 0.0f) {
+    const int st = ensure_guard(plan);
+    if (st != PS_OK) return st;
+  }
   if (tau != plan->guard_tau && plan->gexec) {
     (void)hipGraphExecDestroy(plan->gexec);
     plan->gexec = nullptr;
@@ -1152,13 +1120,17 @@ extern "C" int ps_plan_read_profile(ps_plan *plan, double ms[6], int launches[6]
 
 extern "C" void ps_plan_destroy(ps_plan *plan) {
   if (!plan) return;
+  OnDevice on(plan->device);
+  // executions may still be running on any stream: as freeing the memory
+  // would, wait for the device before it goes back to the pool
+  const bool idle = hipDeviceSynchronize() == hipSuccess;
   for (hipEvent_t e : plan->events) (void)hipEventDestroy(e);
   if (plan->gexec) (void)hipGraphExecDestroy(plan->gexec);
-  if (plan->scratch) (void)hipFree(plan->scratch);
-  if (plan->tables) (void)hipFree(plan->tables);
   if (plan->flags_host) (void)hipHostFree(plan->flags_host);
   if (plan->cstage) (void)hipHostFree(plan->cstage);
-  if (plan->ctables) (void)hipFree(plan->ctables);
+  for (void *p : {static_cast<void *>(plan->scratch), plan->tables, static_cast<void *>(plan->frags),
+                  static_cast<void *>(plan->ctables)})
+    pool_put(p, idle);
   delete plan;
 }
 
@@ -1515,7 +1487,7 @@ extern "C" int ps_marginals(const ps_model *model, const ps_instance *instances,
   hipStream_t s = static_cast<hipStream_t>(stream);
   ps_map *map_dev = nullptr;
   if (map_host) {
-    hipError_t e = hipMalloc(&map_dev, sizeof(ps_map) * pl->n_map);
+    hipError_t e = pool_get(&map_dev, sizeof(ps_map) * pl->n_map);
     if (e != hipSuccess) {
       ps_plan_destroy(pl);
       return set_error(PS_ERR_OUT_OF_MEMORY, "map buffer");
@@ -1530,7 +1502,7 @@ extern "C" int ps_marginals(const ps_model *model, const ps_instance *instances,
     hipError_t e = hipStreamSynchronize(s);
     if (e != hipSuccess) st = hip_error(e, "hipStreamSynchronize");
   }
-  if (map_dev) (void)hipFree(map_dev);
+  pool_put(map_dev, st == PS_OK);
   ps_plan_destroy(pl);
   return st;
 }
@@ -1608,9 +1580,9 @@ int message_prepare(const ps_model *model, int height, int width, const double o
 }
 
 // Upload the tables into `mem` (at least ms.total bytes of device memory),
-// run the message and wait for it.  The two keys are cleared by a kernel.
+// run the message and wait for it.
 int message_enqueue(const MessageSetup &ms, char *mem, const float *child_dev, float *parent_dev, hipStream_t s) {
-  hipError_t e = hipMemcpyAsync(mem, ms.host.data(), ms.o_T, hipMemcpyHostToDevice, s);
+  hipError_t e = launch_upload(mem, ms.host.data(), ms.o_T, s);  // the keys among it, zero
   Bases b;
   b.unary = child_dev;
   b.marginal = parent_dev;
@@ -1626,7 +1598,6 @@ int message_enqueue(const MessageSetup &ms, char *mem, const float *child_dev, f
   const int *sd = reinterpret_cast<const int *>(mem + ms.o_sh);
   if (e == hipSuccess) e = rowpass_set_lds_limit(ms.lds);
   if (e == hipSuccess) e = ms.od ? od_set_lds_limit(ms.od_ext) : colpass_set_lds_limit(ms.col_lds);
-  if (e == hipSuccess) e = launch_reset(b, 1, 1, 1, nullptr, 0, s);
   if (e == hipSuccess)
     e = launch_max(b, reinterpret_cast<const MaxJob *>(mem + ms.o_max), 1, ms.R, ms.H * ms.W, s);
   if (e == hipSuccess) e = launch_rowpass(b, jd, 1, td, sd, ms.R, ms.H, ms.W, ms.lds, s, 0, ms.split);
@@ -1636,8 +1607,7 @@ int message_enqueue(const MessageSetup &ms, char *mem, const float *child_dev, f
     else
       e = launch_colpass(b, jd, 1, td, sd, ms.R, ms.epi, ms.W, ms.col_lds, s, 0, ms.split);
   }
-  // the caller's tables live in pageable host memory and the block may be
-  // reused right after: the call is synchronous
+  // the block may be reused right after: the call is synchronous
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) return hip_error(e, "message");
   return PS_OK;
@@ -1653,9 +1623,9 @@ extern "C" int ps_message(const ps_model *model, const float *child_dev, float *
   int st = message_prepare(model, height, width, offset_c, offset_p, C, rot_mean, rot_sigma, scale, is_sparse, ms);
   if (st != PS_OK) return st;
   void *mem = nullptr;
-  if (hipMalloc(&mem, ms.total) != hipSuccess) return set_error(PS_ERR_OUT_OF_MEMORY, "message scratch");
+  if (pool_get(&mem, ms.total) != hipSuccess) return set_error(PS_ERR_OUT_OF_MEMORY, "message scratch");
   st = message_enqueue(ms, static_cast<char *>(mem), child_dev, parent_dev, static_cast<hipStream_t>(stream));
-  (void)hipFree(mem);
+  pool_put(mem, st == PS_OK);
   return st;
 }
 

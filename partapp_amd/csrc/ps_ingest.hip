@@ -20,6 +20,7 @@
 #include "../../include/partapp_ps.h"
 #include "ps_device.hpp"
 #include "ps_plan.hpp"
+#include "ps_pool.hpp"
 
 namespace ps {
 extern thread_local std::string g_last_error;
@@ -258,7 +259,7 @@ extern "C" int ps_ingest_scores(const float *score_grid_dev, int n, int grid_hei
     IngestWarp *tab = nullptr;
     hipError_t eg = hipSuccess;
     if (n > 18 * IngestSlices::kMax) {
-      if (hipMalloc(&tab, sizeof(IngestWarp) * n) != hipSuccess)
+      if (pool_get(&tab, sizeof(IngestWarp) * n) != hipSuccess)
         return set_error(PS_ERR_OUT_OF_MEMORY, "ingest workspace");
       eg = hipMemcpyAsync(tab, warps.data(), sizeof(IngestWarp) * n, hipMemcpyHostToDevice, st);
     }
@@ -283,7 +284,7 @@ extern "C" int ps_ingest_scores(const float *score_grid_dev, int n, int grid_hei
       }
     }
     if (eg == hipSuccess) eg = hipStreamSynchronize(st);
-    if (tab) (void)hipFree(tab);
+    pool_put(tab, eg == hipSuccess);
     if (eg != hipSuccess) return set_error(PS_ERR_HIP, std::string("ingest: ") + hipGetErrorString(eg));
     return PS_OK;
   }
@@ -292,7 +293,7 @@ extern "C" int ps_ingest_scores(const float *score_grid_dev, int n, int grid_hei
   const long long out_n = (long long)n * height * width;
   const size_t mat_bytes = (mats.size() * sizeof(double) + 255) & ~(size_t)255;
   void *ws = nullptr;
-  hipError_t e = hipMalloc(&ws, mat_bytes + (size_t)out_n * sizeof(unsigned long long));
+  hipError_t e = pool_get(&ws, mat_bytes + (size_t)out_n * sizeof(unsigned long long));
   if (e != hipSuccess) return set_error(PS_ERR_OUT_OF_MEMORY, "ingest workspace");
   double *mats_dev = static_cast<double *>(ws);
   unsigned long long *keys = reinterpret_cast<unsigned long long *>(static_cast<char *>(ws) + mat_bytes);
@@ -310,7 +311,7 @@ extern "C" int ps_ingest_scores(const float *score_grid_dev, int n, int grid_hei
     e = hipGetLastError();
   }
   if (e == hipSuccess) e = hipStreamSynchronize(st);
-  (void)hipFree(ws);
+  pool_put(ws, e == hipSuccess);
   if (e != hipSuccess) return set_error(PS_ERR_HIP, std::string("ingest: ") + hipGetErrorString(e));
   return PS_OK;
 }

@@ -23,6 +23,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <cstring>
 #include <map>
 #include <mutex>
 #include <utility>
@@ -49,6 +50,31 @@ __global__ void k_reset(Bases b, int n_keys, int n_map, int keys_per_inst, int m
     if (b.top2_keys) b.top2_keys[i] = 0ull;
   }
   if (flags && i < n_flags) flags[i] = 0u;
+}
+
+// ---------------------------------------------------------------- k_upload
+// A small table carried to device memory in a kernel's arguments: a copy from
+// pageable memory costs the call some 20 us, a launch some 4.
+
+struct UploadChunk {
+  static constexpr int kUnits = 240;  // 16 bytes each, below the 4 KB of kernel arguments
+  uint4 d[kUnits];
+};
+__global__ __launch_bounds__(256) void k_upload(UploadChunk c, uint4 *dst, int n) {
+  const int i = threadIdx.x;
+  if (i < n) dst[i] = c.d[i];
+}
+
+// `bytes` (a multiple of 16) of host memory to dst in stream order
+hipError_t launch_upload(void *dst, const void *src, size_t bytes, hipStream_t s) {
+  for (size_t o = 0; o < bytes; o += sizeof(UploadChunk)) {
+    UploadChunk c;
+    const size_t n = std::min(bytes - o, sizeof(UploadChunk));
+    std::memcpy(c.d, static_cast<const char *>(src) + o, n);
+    hipLaunchKernelGGL(k_upload, dim3(1), dim3(256), 0, s, c, reinterpret_cast<uint4 *>(static_cast<char *>(dst) + o),
+                       (int)(n / 16));
+  }
+  return hipGetLastError();
 }
 
 // ------------------------------------------------------------------ k_max

@@ -33,6 +33,7 @@
 #include "../../include/partapp_ps.h"
 #include "ps_device.hpp"
 #include "ps_plan.hpp"
+#include "ps_pool.hpp"
 
 namespace ps {
 
@@ -413,7 +414,7 @@ extern "C" int ps_find_local_max(const float *grids_dev, const long long *offset
   const size_t o_keys = sizeof(LmState) * (size_t)n_grids;
   const size_t o_mask = o_keys + sizeof(unsigned long long) * kCap * (size_t)n_grids;
   void *ws = nullptr;
-  if (hipMalloc(&ws, o_mask + sizeof(unsigned long long) * (size_t)words) != hipSuccess)
+  if (pool_get(&ws, o_mask + sizeof(unsigned long long) * (size_t)words) != hipSuccess)
     return set_error(PS_ERR_OUT_OF_MEMORY, "local max workspace");
   char *base = static_cast<char *>(ws);
   LmState *st = reinterpret_cast<LmState *>(base);
@@ -447,7 +448,7 @@ extern "C" int ps_find_local_max(const float *grids_dev, const long long *offset
     e = hipGetLastError();
   }
   if (e == hipSuccess) e = hipStreamSynchronize(s);
-  (void)hipFree(ws);
+  pool_put(ws, e == hipSuccess);
   if (e != hipSuccess) return set_error(PS_ERR_HIP, std::string("local max: ") + hipGetErrorString(e));
   return PS_OK;
 }

@@ -108,6 +108,95 @@ __host__ __device__ __forceinline__ int mfma_row_pitch(int W, int kx, int KK) {
 __host__ __device__ __forceinline__ int mfma_ring_rows(int KK) { return 32 + 16 * KK; }
 __host__ __device__ __forceinline__ int mfma_ring_pitch(int KK) { return mfma_ring_rows(KK) + 8; }
 
+// -------------------------------------------------------- fragment tables
+// The operands of the MFMA passes, formed on the device from the plan's taps
+// (40 KB per message at half widths of 36: 23 MB of a 32-image batch, which
+// the host took longer to form and copy than to plan everything else).
+
+namespace {
+__device__ __forceinline__ unsigned short f16_bits(float v) { return __builtin_bit_cast(unsigned short, (_Float16)v); }
+// round to nearest even (finite inputs)
+__device__ __forceinline__ unsigned short bf16_rne(float f) {
+  const unsigned u = __float_as_uint(f);
+  return (unsigned short)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
+}
+__device__ __forceinline__ void put_pair(unsigned short *d, int lo, int i, float v, bool f16) {
+  if (f16) {
+    const _Float16 h = (_Float16)v;
+    d[i] = __builtin_bit_cast(unsigned short, h);
+    d[lo + i] = f16_bits(v - (float)h);
+  } else {
+    const unsigned short h = bf16_rne(v);
+    d[i] = h;
+    d[lo + i] = bf16_rne(v - __uint_as_float((unsigned)h << 16));
+  }
+}
+}  // namespace
+
+// One block per message.  Each table is its hi parts, then its lo parts (tap
+// minus hi).
+//   frag_x, frag_y  lane l at step kk holds f[16 kk + 8 (l / 32) + t - l % 32],
+//       t = 0..7 (zero off the band), bf16
+//   frag_y16  the y taps in fp16 as the 8 shifted copies of f16_tap_copy_len:
+//       copy j, element e holds tap j + e - 32
+//   frag_r (bf16), frag_r16 (fp16)  the rotation filter as the A operand of the
+//       row pass's second GEMM, whose B operand is the x-filter accumulator
+//       itself: B position p = 16 kk + 8 h + t (lane half h, element t) holds
+//       slice 16 kk + 8 (t / 4) + 4 h + t % 4, so lane l, step kk, element t is
+//       F[l % 32][that slice], F[ro][s] the weight of source slice s in output
+//       slice ro (circular taps, objectdetect_findrot.cpp:377-420); zero for
+//       slices >= R.  With 48 slices there are two output tiles (ro = 32 mt +
+//       l % 32) and three k-steps: step ks reads the accumulator of slice
+//       tile ks / 2, its B position holds slice 32 (ks / 2) + 16 (ks % 2) +
+//       8 (t / 4) + 4 h + t % 4; the table is [mt][ks] per block.
+__global__ __launch_bounds__(256) void k_fragments(const MsgJob *__restrict__ jobs, const float *__restrict__ taps,
+                                                   int R, uint4 *__restrict__ frags) {
+  const MsgJob &J = jobs[blockIdx.x];
+  if (J.od || J.kk_x < 1 || J.kk_y < 1) return;
+  auto band = [&](int off, int KK, const float *f, int L) {
+    unsigned short *d = reinterpret_cast<unsigned short *>(frags + off);
+    for (int e = threadIdx.x; e < KK * 512; e += blockDim.x) {
+      const int kk = e >> 9, l = (e >> 3) & 63, t = e & 7;
+      const int i = 16 * kk + 8 * (l >> 5) + t - (l & 31);
+      put_pair(d, KK * 512, e, i >= 0 && i < L ? f[i] : 0.0f, false);
+    }
+  };
+  band(J.frag_x, J.kk_x, taps + J.taps_x, 2 * J.kx + 1);
+  band(J.frag_y, J.kk_y, taps + J.taps_y, 2 * J.ky + 1);
+  {
+    unsigned short *d = reinterpret_cast<unsigned short *>(frags + J.frag_y16);
+    const int Q = f16_tap_copy_len(J.kk_y), L = 2 * J.ky + 1;
+    for (int e = threadIdx.x; e < 8 * Q; e += blockDim.x) {
+      const int i = e / Q + e % Q - 32;
+      put_pair(d, 8 * Q, e, i >= 0 && i < L ? taps[J.taps_y + i] : 0.0f, true);
+    }
+  }
+  if (R != 24 && R != 48) return;
+  const int MT = (R + 31) / 32, KS = (R + 15) / 16, n = MT * KS * 512;
+  const float *fr = taps + J.taps_r;
+  for (int e = threadIdx.x; e < n; e += blockDim.x) {
+    const int b = e >> 9, mt = b / KS, ks = b - mt * KS, l = (e >> 3) & 63, t = e & 7;
+    const int ro = 32 * mt + (l & 31), sl = 32 * (ks >> 1) + 16 * (ks & 1) + 8 * (t >> 2) + 4 * (l >> 5) + (t & 3);
+    float v = 0.0f;
+    if (ro < R && sl < R) {
+      if (J.rot_mode == kRotFilter) {
+        const int j = (sl - ro + (J.rot_len - 1) / 2 + R) % R;  // rot_len < R: one tap per pair
+        if (j < J.rot_len) v = fr[j];
+      } else if (J.rot_mode == kRotCopy) {
+        v = ro == sl ? 1.0f : 0.0f;
+      }
+    }
+    put_pair(reinterpret_cast<unsigned short *>(frags + J.frag_r), n, e, v, false);
+    put_pair(reinterpret_cast<unsigned short *>(frags + J.frag_r16), n, e, v, true);
+  }
+}
+
+hipError_t launch_fragments(const MsgJob *jobs, int n_jobs, const float *taps, int R, uint4 *frags, hipStream_t s) {
+  if (n_jobs <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_fragments, dim3((unsigned)n_jobs), dim3(256), 0, s, jobs, taps, R, frags);
+  return hipGetLastError();
+}
+
 // ------------------------------------------------------- row pass (x filter)
 // One block per (message, run of `rows` output rows); wave w gathers columns
 // 64 w .. 64 w + 63 and computes the two 32-wide output tiles over them.  For

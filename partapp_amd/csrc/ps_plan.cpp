@@ -68,9 +68,7 @@ static void gaussian_taps(double sigma, std::vector<double> &f) {
 // with alpha rounded to float (objectdetect_findrot.cpp:348-350, 439-441).
 // uBLAS sums each product from zero; the zero terms of the rotation-scaling
 // matrix leave the two products below unchanged.
-static void rotated_offset(const ps_exp_param &ep, int r, double scale, const double v[2], double &dx, double &dy) {
-  float alpha = rot_from_index(ep, r) * M_PI / 180.0;
-  double ca = std::cos((double)alpha), sa = std::sin((double)alpha);
+static void rotated_offset(double ca, double sa, double scale, const double v[2], double &dx, double &dy) {
   double t00 = ca * scale, t01 = -sa * scale, t10 = sa * scale, t11 = ca * scale;
   double p0 = t00 * v[0];
   double p1 = t01 * v[1];
@@ -88,9 +86,16 @@ static void rotated_offset(const ps_exp_param &ep, int r, double scale, const do
 // 197-205 on a translation): off below index brk, off + d from brk on
 // (brk = n, d = 0 when it is one value); false if it changes more than once
 static bool axis_offset(double shift, int n, int &off, int &brk, int &d) {
-  off = (int)std::floor(shift + 0.5);
+  const double t = shift + 0.5, whole = std::floor(t);
+  off = (int)whole;
   brk = n;
   d = 0;
+  // i + shift + 0.5 is off by at most some 2^-52 (n + |shift| + 1) from the
+  // real sum, so a shift further than that from a half-integer has one offset
+  // (the walk below over every index was most of planning an image: 1.9 ms of
+  // 18 messages at 48 x 300 x 300)
+  const double tol = 1e-15 * ((double)n + std::fabs(shift) + 2.0);
+  if (t - whole > tol && t - whole < 1.0 - tol && std::fabs(shift) < 1e9) return true;
   for (int i = 1; i < n; ++i) {
     const double p = (double)i + shift;
     const int o = (int)std::floor(p + 0.5) - i;
@@ -320,10 +325,12 @@ int build_message_plan(const ps_exp_param &ep, int H, int W, const double offset
   out.inv_yb.assign(R, H);
   for (int r = 0; r < R; ++r) {
     double dx, dy;
-    rotated_offset(ep, r, scale, offset_c, dx, dy);
+    const float alpha = rot_from_index(ep, r) * M_PI / 180.0;
+    const double ca = std::cos((double)alpha), sa = std::sin((double)alpha);
+    rotated_offset(ca, sa, scale, offset_c, dx, dy);
     bool ok = axis_offset(-dx, W, out.fwd_ox[r], out.fwd_xb[r], out.fwd_xd[r]) &&
               axis_offset(-dy, H, out.fwd_oy[r], out.fwd_yb[r], out.fwd_yd[r]);
-    rotated_offset(ep, r, scale, offset_p, dx, dy);
+    rotated_offset(ca, sa, scale, offset_p, dx, dy);
     ok = ok && axis_offset(dx, W, out.inv_ox[r], out.inv_xb[r], out.inv_xd[r]) &&
          axis_offset(dy, H, out.inv_oy[r], out.inv_yb[r], out.inv_yd[r]);
     if (!ok)
