@@ -33,13 +33,17 @@ hipError_t launch_certify(const unsigned long long *top2, int n_map, int n_inst,
                           hipStream_t s);
 hipError_t launch_max(const Bases &b, const MaxJob *jobs, int n_jobs, int R, int max_hw, hipStream_t s);
 size_t rowpass_lds_bytes(int R, int W, int kx);
-hipError_t rowpass_set_lds_limit(size_t bytes);
-hipError_t colpass_set_lds_limit(size_t bytes);
+size_t rowpass4_lds_bytes(int R, int W, int kx);
+hipError_t rowpass_set_lds_limit(size_t bytes, size_t bytes4);
+hipError_t colpass_set_lds_limit(size_t bytes, size_t bytes4);
 hipError_t launch_rowpass(const Bases &b, const MsgJob *jobs, int n_jobs, const float *taps, const int *shifts,
-                          int R, int max_h, int max_w, size_t lds_bytes, hipStream_t s, int threads, bool split);
+                          int R, int max_h, int max_w, size_t lds_bytes, size_t lds4_bytes, hipStream_t s, int threads,
+                          bool split);
 size_t colpass_lds_bytes(int ky, int rows);
+size_t colpass4_lds_bytes(int ky);
 hipError_t launch_colpass(const Bases &b, const MsgJob *jobs, int n_jobs, const float *taps, const int *shifts,
-                          int R, int epi_hi, int max_w, size_t lds_bytes_16, hipStream_t s, int rows, bool split);
+                          int R, int epi_hi, int max_w, size_t lds_bytes_16, size_t lds4_bytes_16, hipStream_t s,
+                          int rows, bool split);
 void od_extent(OdExtent &e, int R, const MsgJob &j);
 hipError_t od_set_lds_limit(const OdExtent &ext);
 hipError_t launch_offdiag(const Bases &b, const MsgJob *jobs, int n_jobs, const float *taps, const int *shifts, int R,
@@ -107,7 +111,9 @@ struct Level {
   std::vector<WidthClass> classes;      // row passes: over the diagonal jobs [0, n_diag)
   std::vector<WidthClass> col_classes;  // column passes: the same split further by epilogue kind
   size_t lds = 0;      // row pass
+  size_t lds4 = 0;     // row pass with its x filter on the matrix cores (0: some row does not fit)
   size_t col_lds = 0;  // column pass
+  size_t col_lds4 = 0; // column pass with its y filter on the matrix cores (0: some filter does not fit)
   OdExtent od_ext;     // launches of the off-diagonal jobs' eigenbasis stages
   bool mfma_ok = false;                // every diagonal job fits the BF16 Toeplitz passes
   size_t mfma_row_lds[3] = {0, 0, 0};  // 1, 2 and 3 terms
@@ -362,15 +368,11 @@ struct Builder {
       const int rs = ro - mp.delta;
       shifts.push_back(rs >= 0 && rs < R ? mp.fwd_oy[rs] : kNoSourceRow);
     }
-    // the same pair packed into one word (x offset in the low, y offset in the
-    // high 16 bits, clamped to +-32767, which no grid of the BF16 passes can
-    // reach; no source: y offset -32768)
+    // the row offsets again for the FP32 passes, where a masked source rotation
+    // fails the bounds test as well (mask_rotations)
     for (int ro = 0; ro < R; ++ro) {
       const int rs = ro - mp.delta;
-      const bool has = rs >= 0 && rs < R;
-      const int ox = has ? std::max(-32767, std::min(32767, mp.fwd_ox[rs])) : 0;
-      const int oy = has ? std::max(-32767, std::min(32767, mp.fwd_oy[rs])) : -32768;
-      shifts.push_back((int)(((unsigned)oy << 16) | ((unsigned)ox & 0xffffu)));
+      shifts.push_back(rs >= 0 && rs < R ? mp.fwd_oy[rs] : kNoSourceRow);
     }
     // the source slice of each output slice clamped into [0, R) (an address
     // inside the grid for a slice without a source, whose loads are discarded)
@@ -392,6 +394,16 @@ struct Builder {
       J.kk_x = J.kk_y = 0;  // the BF16 passes take uniform warps only: FP32
     }
     return PS_OK;
+  }
+
+  // a unary source's masked rotations read as no source: they take the warp's
+  // fill value, exp(LOG_ZERO - M), either way
+  void mask_rotations(const MsgJob &J, int R) {
+    if (J.src_kind != kSrcUnary) return;
+    for (int ro = 0; ro < R; ++ro) {
+      const int rs = ro - J.delta;
+      if (rs >= 0 && rs < R && ((J.src_mask.rot_bits >> rs) & 1ull)) shifts[J.shifts + 6 * R + ro] = kNoSourceRow;
+    }
   }
 };
 
@@ -567,6 +579,7 @@ extern "C" int ps_plan_create(const ps_model *model, const ps_instance *instance
             mj.src_kind = m.is_detect[c] ? kSrcUnary : kSrcZero;
             mj.src = unary(c);
             mj.src_mask = part_mask(m, c, W);
+            B.mask_rotations(mj, R);
           } else {
             mj.src_kind = kSrcGrid;
             mj.src = bel(c);
@@ -728,11 +741,13 @@ extern "C" int ps_plan_create(const ps_model *model, const ps_instance *instance
         L.max_h = std::max(L.max_h, j.H);
         L.max_w = std::max(L.max_w, j.W);
         L.lds = std::max(L.lds, rowpass_lds_bytes(R, j.W, j.kx));
+        L.lds4 = std::max(L.lds4, rowpass4_lds_bytes(R, j.W, j.kx));
         if (j.od) {
           od_extent(L.od_ext, R, j);
         } else {
           ++L.n_diag;
           L.col_lds = std::max(L.col_lds, colpass_lds_bytes(j.ky, 16));
+          L.col_lds4 = std::max(L.col_lds4, colpass4_lds_bytes(j.ky));
           // (the BF16 passes address a row-pass output grid with 32-bit byte offsets)
           if (j.kk_x < 1 || j.kk_y < 1 || j.W > 512 || j.H > 32767 || 4ll * R * j.H * j.tpitch >= (1ll << 32))
             L.mfma_ok = false;
@@ -747,6 +762,8 @@ extern "C" int ps_plan_create(const ps_model *model, const ps_instance *instance
       }
       if (L.mfma_row_lds[2] > kLdsLimit || L.mfma_col_lds[2] > kLdsLimit || L.mfma_col16_lds > kLdsLimit)
         L.mfma_ok = false;
+      if (L.lds4 > kLdsLimit) L.lds4 = 0;
+      if (L.col_lds4 > kLdsLimit) L.col_lds4 = 0;
       if (L.lds > kLdsLimit || L.col_lds > kLdsLimit)
         return set_error(PS_ERR_UNSUPPORTED, "row pass needs " + std::to_string(L.lds) +
                                                  " bytes of LDS (R * width too large for one workgroup)");
@@ -850,14 +867,16 @@ extern "C" int ps_plan_create(const ps_model *model, const ps_instance *instance
   pl->h_roots = B.roots;
   pl->h_maxes = B.maxes;
   pl->h_maps = B.maps;
-  size_t max_lds = 0, max_col_lds = 0;
+  size_t max_lds = 0, max_lds4 = 0, max_col_lds = 0, max_col_lds4 = 0;
   for (auto *lv : {&pl->up, &pl->down})
     for (auto &L : *lv) {
       max_lds = std::max(max_lds, L.lds);
+      max_lds4 = std::max(max_lds4, L.lds4);
       max_col_lds = std::max(max_col_lds, L.col_lds);
+      max_col_lds4 = std::max(max_col_lds4, L.col_lds4);
     }
-  e = rowpass_set_lds_limit(max_lds);
-  if (e == hipSuccess) e = colpass_set_lds_limit(max_col_lds);
+  e = rowpass_set_lds_limit(max_lds, max_lds4);
+  if (e == hipSuccess) e = colpass_set_lds_limit(max_col_lds, max_col_lds4);
   size_t mrow = 0, mcol = 0;
   for (auto *lv : {&pl->up, &pl->down})
     for (auto &L : *lv)
@@ -1166,14 +1185,14 @@ static hipError_t sweep(ps_plan *pl, const Bases &b, int terms, int col_terms, p
                                 c.mfma_rows > 0 ? c.mfma_rows : pl->mfma_rows, c.max_h, c.max_w,
                                 L.mfma_row_lds[ti], c.leaf, s);
       else
-        e = launch_rowpass(b, jobs + c.start, c.count, pl->taps, pl->shifts, pl->R, c.max_h, c.max_w, L.lds, s,
-                           c.row_threads, c.split);
+        e = launch_rowpass(b, jobs + c.start, c.count, pl->taps, pl->shifts, pl->R, c.max_h, c.max_w, L.lds, L.lds4,
+                           s, c.row_threads, c.split);
       profile_end(pp, ev2, s);
     }
     if (e == hipSuccess && n_od > 0) {  // off-diagonal messages: the FP32 row pass, then the eigenbasis stages
       const long ev2 = profile_begin(pp, 2, s);
-      e = launch_rowpass(b, jobs + L.n_diag, n_od, pl->taps, pl->shifts, pl->R, L.max_h, L.max_w, L.lds, s, 0,
-                         L.split);
+      e = launch_rowpass(b, jobs + L.n_diag, n_od, pl->taps, pl->shifts, pl->R, L.max_h, L.max_w, L.lds,
+                         L.lds4, s, 0, L.split);
       profile_end(pp, ev2, s);
     }
     if (e != hipSuccess) return;
@@ -1188,8 +1207,8 @@ static hipError_t sweep(ps_plan *pl, const Bases &b, int terms, int col_terms, p
         e = launch_colpass_mfma(b, jobs + c.start, c.count, pl->frags, pl->shifts, pl->R, col_terms, terms != 3,
                                 c.epi_hi, c.max_w, terms != 3 ? L.mfma_col16_lds : L.mfma_col_lds[tc], c.leaf, s);
       else
-        e = launch_colpass(b, jobs + c.start, c.count, pl->taps, pl->shifts, pl->R, c.epi_hi, c.max_w, L.col_lds, s,
-                           c.col_rows, c.split);
+        e = launch_colpass(b, jobs + c.start, c.count, pl->taps, pl->shifts, pl->R, c.epi_hi, c.max_w, L.col_lds,
+                           L.col_lds4, s, c.col_rows, c.split);
       profile_end(pp, ev2, s);
     }
     // the column pass class also times the eigenbasis stages
@@ -1293,20 +1312,20 @@ static hipError_t sweep_subset(ps_plan *pl, const Bases &b, ps_map *map_dev, hip
       const WidthClass &c = L.classes[k];
       const long ev2 = profile_begin(pp, 2, s);
       e = launch_rowpass(b, jobs + ls.row[k].start, ls.row[k].count, pl->taps, pl->shifts, pl->R, c.max_h, c.max_w,
-                         L.lds, s, c.row_threads, c.split);
+                         L.lds, L.lds4, s, c.row_threads, c.split);
       profile_end(pp, ev2, s);
     }
     if (e == hipSuccess && ls.od_row.count > 0) {
       const long ev2 = profile_begin(pp, 2, s);
       e = launch_rowpass(b, jobs + ls.od_row.start, ls.od_row.count, pl->taps, pl->shifts, pl->R, L.max_h, L.max_w,
-                         L.lds, s, 0, L.split);
+                         L.lds, L.lds4, s, 0, L.split);
       profile_end(pp, ev2, s);
     }
     for (size_t k = 0; k < L.col_classes.size() && e == hipSuccess; ++k) {
       const WidthClass &c = L.col_classes[k];
       const long ev2 = profile_begin(pp, 3, s);
       e = launch_colpass(b, jobs + ls.col[k].start, ls.col[k].count, pl->taps, pl->shifts, pl->R, c.epi_hi, c.max_w,
-                         L.col_lds, s, c.col_rows, c.split);
+                         L.col_lds, L.col_lds4, s, c.col_rows, c.split);
       profile_end(pp, ev2, s);
     }
     if (e == hipSuccess && ls.od_col.count > 0) {
@@ -1539,7 +1558,11 @@ int message_prepare(const ps_model *model, int height, int width, const double o
   ms.split = mp.split;
   if (mp.od) od_extent(ms.od_ext, R, mj);
   ms.lds = rowpass_lds_bytes(R, width, mj.kx);
+  ms.lds4 = rowpass4_lds_bytes(R, width, mj.kx);
+  if (ms.lds4 > kLdsLimit) ms.lds4 = 0;
   ms.col_lds = mp.od ? 0 : colpass_lds_bytes(mp.ky, 16);
+  ms.col_lds4 = mp.od ? 0 : colpass4_lds_bytes(mp.ky);
+  if (ms.col_lds4 > kLdsLimit) ms.col_lds4 = 0;
   if (ms.lds > kLdsLimit || ms.col_lds > kLdsLimit)
     return set_error(PS_ERR_UNSUPPORTED, "message needs more LDS than one workgroup has");
   mj.src_kind = kSrcUnary;  // a plain grid, read through the (empty) mask path
@@ -1596,16 +1619,16 @@ int message_enqueue(const MessageSetup &ms, char *mem, const float *child_dev, f
   const MsgJob *jd = reinterpret_cast<const MsgJob *>(mem + ms.o_job);
   const float *td = reinterpret_cast<const float *>(mem + ms.o_taps);
   const int *sd = reinterpret_cast<const int *>(mem + ms.o_sh);
-  if (e == hipSuccess) e = rowpass_set_lds_limit(ms.lds);
-  if (e == hipSuccess) e = ms.od ? od_set_lds_limit(ms.od_ext) : colpass_set_lds_limit(ms.col_lds);
+  if (e == hipSuccess) e = rowpass_set_lds_limit(ms.lds, ms.lds4);
+  if (e == hipSuccess) e = ms.od ? od_set_lds_limit(ms.od_ext) : colpass_set_lds_limit(ms.col_lds, ms.col_lds4);
   if (e == hipSuccess)
     e = launch_max(b, reinterpret_cast<const MaxJob *>(mem + ms.o_max), 1, ms.R, ms.H * ms.W, s);
-  if (e == hipSuccess) e = launch_rowpass(b, jd, 1, td, sd, ms.R, ms.H, ms.W, ms.lds, s, 0, ms.split);
+  if (e == hipSuccess) e = launch_rowpass(b, jd, 1, td, sd, ms.R, ms.H, ms.W, ms.lds, ms.lds4, s, 0, ms.split);
   if (e == hipSuccess) {
     if (ms.od)
       e = launch_offdiag(b, jd, 1, td, sd, ms.R, ms.od_ext, s);
     else
-      e = launch_colpass(b, jd, 1, td, sd, ms.R, ms.epi, ms.W, ms.col_lds, s, 0, ms.split);
+      e = launch_colpass(b, jd, 1, td, sd, ms.R, ms.epi, ms.W, ms.col_lds, ms.col_lds4, s, 0, ms.split);
   }
   // the block may be reused right after: the call is synchronous
   if (e == hipSuccess) e = hipStreamSynchronize(s);

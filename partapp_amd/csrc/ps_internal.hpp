@@ -73,8 +73,8 @@ struct MsgJob {
   int taps_x;    //   with zeros to a multiple of 16
   int taps_y;
   int shifts;    // offset into the shift pool: fwd_ox[R] fwd_oy[R] inv_ox[R] inv_oy[R] (by source
-                 // slice), then fwd_ox[R] fwd_oy[R] by output slice, then those packed in 16 bits each,
-                 // then the clamped source slice by output slice; split: from 8 R the forward x break,
+                 // slice), then fwd_ox[R] fwd_oy[R] by output slice, then fwd_oy with the masked rotations
+                 // left without a source, then the clamped source slice by output slice; split: from 8 R the forward x break,
                  // x step, y break, y step by output slice, then the inverse ones by slice
   int src_kind;  // SrcKind
   int src_key;   // index of the source's max key

@@ -7,10 +7,10 @@
 //   k_rowpass  one block per (message, row y): gathers the forward-warped
 //              child belief of all R rotation slices (integer shift per
 //              slice), exp(b - M), circular rotation filter, then the
-//              truncated x filter from an LDS row with zero halo.  Writes the
-//              row-filtered grid T.
-//   k_colpass  one block per (message, rotation, 64x64 tile): truncated y
-//              filter of T with a 16-row register window per lane, log,
+//              truncated x filter from an LDS row with zero halo on the
+//              matrix cores.  Writes the row-filtered grid T.
+//   k_colpass  one block per (message, rotation, 64-column strip): truncated y
+//              filter of T on the matrix cores from an LDS ring of rows, log,
 //              +M, the inverse warp folded into the tile origin, and the
 //              caller's accumulation (parent belief, root message slot, or
 //              marginal + next downward source) fused as the epilogue,
@@ -26,6 +26,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <type_traits>
 #include <utility>
 
 #include "ps_device.hpp"
@@ -76,6 +77,43 @@ hipError_t launch_upload(void *dst, const void *src, size_t bytes, hipStream_t s
   }
   return hipGetLastError();
 }
+
+// ------------------------------------------------- FP32 filters on the MFMA
+// v_mfma_f32_4x4x1 holds 16 independent 4 x 4 products of depth 1: lane l =
+// 4 b + n of block b has D[i] += A(lane 4 b + i) B(lane l), i = 0..3, each one
+// fused multiply-add, bit for bit fmaf (checked on the device over 50-step
+// chains with operands down to subnormals).  Four outputs next to each other
+// along a filter of L taps, out[n] = sum_k x[k] f[k - n], therefore take L + 3
+// steps in ascending order, the same sums as the sequential dot product with
+// zero products before and after (0 x + a = a for finite x), at twice the
+// rate of unpacked v_fma_f32 (131 against 65 TFLOP/s measured; the two do not
+// overlap: a loop of both takes the sum of their times).  A zero product with
+// a non-finite value would be a NaN outside the band, so data holding one goes
+// an output at a time over its own taps.
+
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ f32x4_t mfma4(float a, float b, f32x4_t c) {
+  return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 0, 0, 0);
+}
+
+// The taps of such a filter as that operand, in steps of four: copy n (n =
+// lane % 4) holds f[k - n], k = 0 .. 4 chunks - 1 (zero off the filter); the
+// copies' 16-byte units start in different LDS banks (an odd pitch).
+__host__ __device__ __forceinline__ int tap4_chunks(int k) { return (2 * k + 1 + 3 + 3) >> 2; }
+__host__ __device__ __forceinline__ int tap4_pitch(int k) { return 4 * (tap4_chunks(k) | 1); }
+__device__ __forceinline__ void tap4_fill(float *t4, const float *__restrict__ f, int k) {
+  const int L = 2 * k + 1, n4 = 4 * tap4_chunks(k), pitch = tap4_pitch(k);
+  for (int i = threadIdx.x; i < 4 * n4; i += blockDim.x) {
+    const int n = i & 3, e = i >> 2, t = e - n;
+    t4[n * pitch + e] = t >= 0 && t < L ? f[t] : 0.0f;
+  }
+}
+
+// bit patterns from here on (infinities, NaNs, and anything negative, which
+// no filter operand is) are not for the MFMA
+constexpr unsigned kNonFinite = 0x7f800000u;
+__device__ __forceinline__ unsigned max_bits(unsigned m, float v) { return max(m, __float_as_uint(v)); }
 
 // ------------------------------------------------------------------ k_max
 // Max of a leaf's source grid (getMinMax, multi_array_op.hpp:60-77).  Grids
@@ -145,6 +183,88 @@ __global__ __launch_bounds__(256) void k_max(Bases b, const MaxJob *__restrict__
 // two halves 9.7 instead of 8.8 ms per 32 x 300x300x24 sweep)
 __host__ __device__ constexpr int row_groups(int R) { return R >= 48 ? 2 : 1; }
 
+// LDS of the row pass with the x filter on the MFMA: P[position][RG + 1], the
+// RG slices of a column next to each other (written and read at immediate
+// offsets; an odd pitch, so 16 positions 4 apart are 16 different banks), kx
+// zeros before the row and the last tile's window behind it; the tap operand and
+// the flag follow.  24 slices go through at once (12 at a time halve the LDS
+// and cost a second pass over the rotation filter's inputs: 855 against 765 us
+// per launch of 96 messages of 300x300x24), 48 in four groups of 12 (24 beside
+// the 48 values held from group to group spill).
+__host__ __device__ constexpr int row4_slices(int R) { return R == 24 ? 24 : 12; }
+__host__ __device__ __forceinline__ int row4_len(int W, int k) { return ((W + 63) & ~63) + 4 * tap4_chunks(k); }
+__host__ __device__ __forceinline__ size_t row4_floats(int rg, int W, int k) {
+  return ((size_t)row4_len(W, k) * (rg + 1) + 3) & ~(size_t)3;
+}
+__host__ __device__ __forceinline__ size_t row4_lds_bytes(int rg, int W, int k) {
+  return sizeof(float) * (row4_floats(rg, W, k) + 4 * tap4_pitch(k) + 4);
+}
+
+// x filter of the RG rows of P (RG a multiple of 4), row y of T: wave w takes
+// the 64-column tiles w, w + waves, ...; lane 4 b + m reads slice 4 s + m from
+// position 4 b of the tile on, and holds after the last step, in acc[s][i],
+// slice 4 s + i at column `lane`: stores of whole lines.  One LDS read of four
+// steps' taps serves RG / 4 groups of slices.
+template <int RG>
+__device__ __forceinline__ void xfilter4(const float *P, const float *t4, int kx, float *T, int tp, long long plane,
+                                         int y, int W) {
+  static_assert(RG % 4 == 0, "rows in groups of four");
+  constexpr int S = RG / 4, Q = RG + 1;
+  const int lane = threadIdx.x & 63, m = lane & 3;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int NT = tap4_chunks(kx), tiles = (W + 63) >> 6;
+  char *trow = reinterpret_cast<char *>(T + (long long)y * tp);
+  const long long plane_b = plane * 4;
+  for (int j = wave; j < tiles; j += (int)(blockDim.x >> 6)) {
+    const float4 *tv = reinterpret_cast<const float4 *>(t4 + m * tap4_pitch(kx));
+    const float *d = P + (64 * j + (lane & ~3)) * Q + m;
+    f32x4_t acc[S];
+#pragma unroll
+    for (int s = 0; s < S; ++s) acc[s] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int c = 0; c < NT; ++c) {
+      const float4 t = *tv++;
+      float x[4][S];
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int s = 0; s < S; ++s) x[k][s] = d[k * Q + 4 * s];
+      d += 4 * Q;
+#pragma unroll
+      for (int s = 0; s < S; ++s) acc[s] = mfma4(x[0][s], t.x, acc[s]);
+#pragma unroll
+      for (int s = 0; s < S; ++s) acc[s] = mfma4(x[1][s], t.y, acc[s]);
+#pragma unroll
+      for (int s = 0; s < S; ++s) acc[s] = mfma4(x[2][s], t.z, acc[s]);
+#pragma unroll
+      for (int s = 0; s < S; ++s) acc[s] = mfma4(x[3][s], t.w, acc[s]);
+    }
+    const unsigned xo = 64u * (unsigned)j + (unsigned)lane;
+    if ((int)xo < tp) {
+      char *o = trow;
+#pragma unroll
+      for (int s = 0; s < S; ++s)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          *reinterpret_cast<float *>(o + xo * 4u) = acc[s][i];
+          o += plane_b;
+        }
+    }
+  }
+}
+
+// The same filter of rows holding a non-finite value, one output at a time
+// (the taps padded to a multiple of four with zeros, as the pool holds them).
+__device__ __forceinline__ void xfilter_plain(const float *P, int rg, const float *__restrict__ f, int kx, float *T,
+                                              int tp, long long plane, int y, int W) {
+  const int Lp = (2 * kx + 1 + 3) & ~3;
+  for (int i = threadIdx.x; i < rg * W; i += blockDim.x) {
+    const int r = i / W, x = i - r * W;
+    float a = 0.0f;
+    for (int t = 0; t < Lp; ++t) a = fmaf(P[(x + t) * (rg + 1) + r], f[t], a);
+    T[r * plane + (long long)y * tp + x] = a;
+  }
+}
+
 struct RowGeom {
   int Wo;    // groups of 8 outputs per row
   int nch;   // chunks of 8 taps (the last one a half chunk when tail4)
@@ -160,13 +280,13 @@ __host__ __device__ __forceinline__ RowGeom row_geom(int W, int kx) {
   return g;
 }
 
-// zero the halo columns [0, kx) and [kx + W, Pw) of every row of P
-__device__ __forceinline__ void zero_halo(float *P, int R, int W, int kx, const RowGeom &g) {
-  const int per_row = g.Pw - W;
+// zero the halo columns [0, kx) and [kx + W, pitch) of every row of P
+__device__ __forceinline__ void zero_halo(float *P, int R, int W, int kx, int pitch) {
+  const int per_row = pitch - W;
   for (int i = threadIdx.x; i < R * per_row; i += blockDim.x) {
     const int r = i / per_row;
     const int c = i - r * per_row;
-    P[r * g.Pw + (c < kx ? c : c + W)] = 0.0f;
+    P[r * pitch + (c < kx ? c : c + W)] = 0.0f;
   }
 }
 
@@ -295,12 +415,12 @@ __device__ __forceinline__ void xfilter_rows(const float *P, const float *taps_x
 }
 
 // Forward offsets of output slice ro (so = J.shifts + 4 R: the x offsets at
-// so, the y offsets at so + R) at row ys / column x.  SPLIT: the warp's
+// so, the y offsets at so + 2 R) at row ys / column x.  SPLIT: the warp's
 // offset changes once along an axis, by the step at so + 5 R (x) / so + 7 R
 // (y) from the break at so + 4 R / so + 6 R on.
 template <int R, bool SPLIT>
 __device__ __forceinline__ int fwd_oy(const int *__restrict__ shifts, int so, int ro, int ys) {
-  int oy = shifts[so + R + ro];
+  int oy = shifts[so + 2 * R + ro];  // masked rotations have no source row
   if (SPLIT && ys >= shifts[so + 6 * R + ro]) oy += shifts[so + 7 * R + ro];
   return oy;
 }
@@ -311,38 +431,24 @@ __device__ __forceinline__ int fwd_ox(const int *__restrict__ shifts, int so, in
   return ox;
 }
 
-// One column x of the fixed-R row pass for slice group G: the R source
-// values are loaded together, exponentiated and rotation-filtered in
-// registers; the group's output slices G * RG .. (G + 1) * RG - 1 are written
-// to P.
-template <int R, int G, bool SPLIT>
-__device__ __forceinline__ void rowpass_column(const MsgJob &J, const float *__restrict__ taps,
-                                               const int *__restrict__ shifts, const float *src, float negM,
-                                               float e_fill, float *P, int y, const RowGeom &g, const int x) {
-  constexpr int RG = R / row_groups(R);
+// The R raw source values of column x, row y.  Per OUTPUT slice: the source
+// slice is ro - delta (clamped into [0, R) at so + 3 R), read at (y + oyo, x +
+// oxo) with oxo at so, oyo at so + 2 R (so = J.shifts + 4 R); slices without a
+// source, or with a masked one, carry a row offset that fails the bounds test.
+// Forward warp (objectdetect_findrot.cpp:342-359): every load unconditional (a
+// slice without a source reads its clamped slice, a column outside the grid
+// its nearest column), all R of them issued before any is used; the row
+// address on the scalar unit, the column a byte offset from it.  The offsets
+// are read through the scalar cache here and again by rowpass_exp (an empty
+// asm keeps the reads apart) rather than held in scalar registers.
+template <int R, bool SPLIT>
+__device__ __forceinline__ void rowpass_gather(const MsgJob &J, const int *__restrict__ shifts, const float *src, int y,
+                                               const int x, float (&v)[R]) {
   const int H = J.H, W = J.W;
-  const int kx = J.kx;
-  const float *fr = taps + J.taps_r;
-  const int delta = J.delta;
-  const bool zero_src = J.src_kind == kSrcZero;
-  const UnaryMask mk = J.src_mask;
-  const bool use_mask = J.src_kind == kSrcUnary && (mk.rot_bits != 0ull || mk.strip != 0);
   const int Ps = J.src.pitch;
-  int HW = H * Ps;  // R * H * pitch < 2^31 is checked when the plan is built
-  // per OUTPUT slice: the source slice is ro - delta (clamped into [0, R) at
-  // so + 3 R), read at (y + oyo, x + oxo) with oxo at so, oyo at so + R;
-  // slices without a source carry a row offset that fails the bounds test.
-  // The offsets are read through the scalar cache twice (an empty asm keeps
-  // the reads apart) rather than held in scalar registers from the loads to
-  // their use.
-  int so = J.shifts + 4 * R;
+  int HW = __builtin_amdgcn_readfirstlane(H * Ps);  // R * H * pitch < 2^31 is checked when the plan is built
+  int so = __builtin_amdgcn_readfirstlane(J.shifts + 4 * R);
   const int ys = __builtin_amdgcn_readfirstlane(y);  // uniform: the row offsets on the scalar unit
-
-  // forward warp (objectdetect_findrot.cpp:342-359): every load unconditional
-  // (a slice without a source reads its clamped slice, a column outside the
-  // grid its nearest column), all R of them issued before any is used; the
-  // row address on the scalar unit, the column a byte offset from it
-  float v[R];
   asm volatile("" : "+s"(so), "+s"(HW));
   const int x4 = x * 4, xmax4 = (W - 1) * 4;
 #pragma unroll
@@ -352,22 +458,27 @@ __device__ __forceinline__ void rowpass_column(const MsgJob &J, const float *__r
     const int xx4 = min(max(x4 + fwd_ox<R, SPLIT>(shifts, so, ro, x) * 4, 0), xmax4);
     v[ro] = *reinterpret_cast<const float *>(srow + (unsigned)xx4);
   }
-  // masks, then exp(b - M) (:362-365) as 2^((b - M) log2 e) on the hardware
-  // exp2 (values below 2^-126 flush to zero, where the reference's expf
-  // returns subnormals).  A source pixel outside the grid (the warp's
-  // LOG_ZERO fill) and a masked unary state (a masked rotation, or a column
-  // in the masked strips) both take e_fill = exp(LOG_ZERO - M): a masked
-  // rotation fails its row's test, the strips narrow the columns' range.
+}
+
+// Masks, then exp(b - M) (:362-365) as 2^((b - M) log2 e) on the hardware exp2
+// (values below 2^-126 flush to zero, where the reference's expf returns
+// subnormals).  A source pixel outside the grid (the warp's LOG_ZERO fill) and
+// a masked unary state (a masked rotation, or a column in the masked strips)
+// both take e_fill = exp(LOG_ZERO - M): a masked rotation's row offset fails the
+// test, the strips narrow the columns' range.
+template <int R, bool SPLIT>
+__device__ __forceinline__ void rowpass_exp(const MsgJob &J, const int *__restrict__ shifts, float negM, float e_fill,
+                                            int y, const int x, const float (&v)[R], float (&e)[R]) {
+  const int H = J.H, W = J.W;
+  const bool zero_src = J.src_kind == kSrcZero;
+  int so = __builtin_amdgcn_readfirstlane(J.shifts + 4 * R);
+  const int ys = __builtin_amdgcn_readfirstlane(y);
   asm volatile("" : "+s"(so));
-  const int lo = use_mask ? mk.strip : 0;
+  const int lo = J.src_kind == kSrcUnary ? J.src_mask.strip : 0;
   const unsigned span = (unsigned)max(W - 2 * lo, 0);  // columns lo .. W - lo - 1 are read
-  const unsigned long long rot_bits = use_mask ? mk.rot_bits : 0ull;
-  float e[R];
 #pragma unroll
   for (int ro = 0; ro < R; ++ro) {
-    const int rs = ro - delta;
-    const bool row_ok = (unsigned)(ys + fwd_oy<R, SPLIT>(shifts, so, ro, ys)) < (unsigned)H &&
-                        !((unsigned)rs < (unsigned)R && ((rot_bits >> (rs & 63)) & 1ull));
+    const bool row_ok = (unsigned)(ys + fwd_oy<R, SPLIT>(shifts, so, ro, ys)) < (unsigned)H;
     // a leaf without a detector has the zero log posterior (b = 0); the
     // exponential is computed for every lane (an empty asm keeps it out of a
     // branch), then selected
@@ -376,22 +487,105 @@ __device__ __forceinline__ void rowpass_column(const MsgJob &J, const float *__r
     const bool ok = row_ok && (unsigned)(x + fwd_ox<R, SPLIT>(shifts, so, ro, x) - lo) < span;
     e[ro] = ok ? ev : e_fill;
   }
-  float *out = P + kx + x;
+}
+
+// Rotation filter of a column's values: the output slices G * RG .. (G + 1) *
+// RG - 1 are written to out (pitch apart).
+template <int R, int RG, int G, class Pitch>
+__device__ __forceinline__ void rowpass_rotate(const MsgJob &J, const float *__restrict__ taps, const float (&e)[R],
+                                               float *out, Pitch pitch) {
   if (J.rot_mode == kRotFilter) {
-    RotDispatch<R, (R % 2 == 1) ? R - 2 : R - 1, G * RG, (G + 1) * RG>::run(J.rot_len, e, fr, out, g.Pw);
+    RotDispatch<R, (R % 2 == 1) ? R - 2 : R - 1, G * RG, (G + 1) * RG>::run(J.rot_len, e, taps + J.taps_r, out, pitch);
   } else if (J.rot_mode == kRotCopy) {
 #pragma unroll
-    for (int k = 0; k < RG; ++k) out[k * g.Pw] = e[G * RG + k];
+    for (int k = 0; k < RG; ++k) out[k * pitch] = e[G * RG + k];
   } else {
 #pragma unroll
-    for (int k = 0; k < RG; ++k) out[k * g.Pw] = 0.0f;
+    for (int k = 0; k < RG; ++k) out[k * pitch] = 0.0f;
   }
 }
 
 // Row pass for a rotation count fixed at compile time (24, and the
-// reference's default 48): lane t owns the columns x = t (mod blockDim.x);
-// the slice groups go through P and the x filter one after another.
-template <int R, bool SPLIT>
+// reference's default 48), row y: lane t owns the columns x = t (mod
+// blockDim.x); the slice groups go through P and the x filter one after
+// another.  MFMA: the x filter on the matrix cores; with one column per lane
+// its values stay in registers from group to group.  Else (rows too wide for
+// the padding and the tap operand in LDS, from some 1500 columns of 24 slices
+// on) on the vector unit.  Bound by latency: the filter, the exponentials and
+// rotation filter, and the gather each take some 40% of a launch of 96
+// messages of 300x300x24 and overlap between the 4 blocks that fit a CU only
+// in part: 899 us with the filter on the vector unit, 765 now (467 without the
+// filter; 1.66 GB through memory).  48 slices: 118 -> 75 us per launch of an
+// image of 300x300.
+template <int R, bool SPLIT, bool MFMA>
+__device__ __forceinline__ void rowpass_body(const Bases &b, const MsgJob &J, const float *__restrict__ taps,
+                                             const int *__restrict__ shifts, float *P, int y) {
+  const int H = J.H, W = J.W;
+  const int kx = J.kx;
+  const RowGeom g = row_geom(W, kx);
+  constexpr int RG = MFMA ? row4_slices(R) : R / row_groups(R), NG = R / RG, Q = RG + 1;
+  float *t4 = P + row4_floats(RG, W, kx);
+  unsigned *bad = reinterpret_cast<unsigned *>(t4 + 4 * tap4_pitch(kx));  // a non-finite value among e
+  if (MFMA) {
+    // zeros before the row and as far behind it as a window reaches whose
+    // first output is inside
+    const int tail = (kx + W) * Q, end = (W + 4 * tap4_chunks(kx)) * Q;
+    for (int i = threadIdx.x; i < kx * Q; i += blockDim.x) P[i] = 0.0f;
+    for (int i = tail + (int)threadIdx.x; i < end; i += blockDim.x) P[i] = 0.0f;
+    tap4_fill(t4, taps + J.taps_x, kx);
+    if (threadIdx.x == 0) *bad = 0u;
+  } else {
+    zero_halo(P, RG, W, kx, g.Pw);
+  }
+
+  const float M = key2f(b.max_keys[J.src_key]);
+  const float negM = -M;
+  // exp(LOG_ZERO - M): the warp's fill value, on the path of every other value
+  const float e_fill = __builtin_amdgcn_exp2f((kLogZero + negM) * kLog2eF);
+  const float *src = cptr(b, J.src);
+  float *T = mptr(b, J.tmp);
+  const long long plane = (long long)H * J.tpitch;
+  const bool one = MFMA && W <= (int)blockDim.x;
+  float e[R];
+  unsigned bits = 0u;
+  auto values = [&](int x) {
+    float v[R];
+    rowpass_gather<R, SPLIT>(J, shifts, src, y, x, v);
+    rowpass_exp<R, SPLIT>(J, shifts, negM, e_fill, y, x, v, e);
+    // the rotation's taps are finite: its outputs are if its inputs are
+    if (MFMA) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) bits = max_bits(bits, e[r]);
+    }
+  };
+  auto group = [&](auto gc) {
+    constexpr int G = decltype(gc)::value;
+    if (G > 0) __syncthreads();  // every item of the group before is filtered
+    for (int x0 = 0; x0 < W; x0 += (int)blockDim.x) {
+      const int x = x0 + (int)threadIdx.x;
+      if (!one || G == 0) values(min(x, W - 1));  // past the row: its last column again
+      if (x < W) {
+        if (MFMA) rowpass_rotate<R, RG, G>(J, taps, e, P + (kx + x) * Q, std::integral_constant<int, 1>{});
+        else rowpass_rotate<R, RG, G>(J, taps, e, P + kx + x, g.Pw);
+      }
+    }
+    if (MFMA && G == 0) __syncthreads();  // the flag is clear
+    if (MFMA && bits >= kNonFinite) *bad = 1u;
+    __syncthreads();
+    float *Tg = T + G * RG * plane;
+    if (!MFMA) xfilter_rows(P, taps + J.taps_x, Tg, RG, J.tpitch, plane, y, g);
+    else if (__builtin_amdgcn_readfirstlane(*bad) == 0u) xfilter4<RG>(P, t4, kx, Tg, J.tpitch, plane, y, W);
+    else xfilter_plain(P, RG, taps + J.taps_x, kx, Tg, J.tpitch, plane, y, W);
+  };
+  group(std::integral_constant<int, 0>{});
+  if constexpr (NG > 1) group(std::integral_constant<int, 1>{});
+  if constexpr (NG > 2) {
+    group(std::integral_constant<int, 2>{});
+    group(std::integral_constant<int, 3>{});
+  }
+}
+
+template <int R, bool SPLIT, bool MFMA>
 __global__ __launch_bounds__(512) void k_rowpass_r(Bases b, const MsgJob *__restrict__ jobs,
                                                    const float *__restrict__ taps, const int *__restrict__ shifts) {
   extern __shared__ float4 lds4[];
@@ -401,37 +595,10 @@ __global__ __launch_bounds__(512) void k_rowpass_r(Bases b, const MsgJob *__rest
   const MsgJob &J = jobs[by];
   if (skip_inst(b, J.inst)) return;
   const int y = (int)bx;
-  const int H = J.H, W = J.W;
-  if (y >= H) return;
-  const int kx = J.kx;
-  const RowGeom g = row_geom(W, kx);
-  constexpr int RG = R / row_groups(R);
-  zero_halo(P, RG, W, kx, g);
-
-  const float M = key2f(b.max_keys[J.src_key]);
-  const float negM = -M;
-  // exp(LOG_ZERO - M): the warp's fill value, on the path of every other value
-  const float e_fill = __builtin_amdgcn_exp2f((kLogZero + negM) * kLog2eF);
-  const float *src = cptr(b, J.src);
-  float *T = mptr(b, J.tmp);
-  const long long plane = (long long)H * J.tpitch;
+  if (y >= J.H) return;
   // a warp whose offset changes along an axis takes the SPLIT variants
-  const bool split = SPLIT && J.split != 0;
-  for (int x = threadIdx.x; x < W; x += blockDim.x) {
-    if (split) rowpass_column<R, 0, true>(J, taps, shifts, src, negM, e_fill, P, y, g, x);
-    else rowpass_column<R, 0, false>(J, taps, shifts, src, negM, e_fill, P, y, g, x);
-  }
-  __syncthreads();
-  xfilter_rows(P, taps + J.taps_x, T, RG, J.tpitch, plane, y, g);
-  if constexpr (row_groups(R) > 1) {
-    __syncthreads();  // every item of the first group is filtered
-    for (int x = threadIdx.x; x < W; x += blockDim.x) {
-      if (split) rowpass_column<R, 1, true>(J, taps, shifts, src, negM, e_fill, P, y, g, x);
-      else rowpass_column<R, 1, false>(J, taps, shifts, src, negM, e_fill, P, y, g, x);
-    }
-    __syncthreads();
-    xfilter_rows(P, taps + J.taps_x, T + RG * plane, RG, J.tpitch, plane, y, g);
-  }
+  if (SPLIT && J.split != 0) rowpass_body<R, SPLIT, MFMA>(b, J, taps, shifts, P, y);
+  else rowpass_body<R, false, MFMA>(b, J, taps, shifts, P, y);
 }
 
 // Row pass for any rotation count: the exponentiated column goes through an
@@ -452,7 +619,7 @@ __global__ __launch_bounds__(512) void k_rowpass_any(Bases b, const MsgJob *__re
   const int Wa = (W + 3) & ~3;
   float *E = reinterpret_cast<float *>(lds4);
   float *P = E + R * Wa;
-  zero_halo(P, R, W, kx, g);
+  zero_halo(P, R, W, kx, g.Pw);
 
   const float M = key2f(b.max_keys[J.src_key]);
   const float negM = -M;
@@ -516,9 +683,16 @@ __global__ __launch_bounds__(512) void k_rowpass_any(Bases b, const MsgJob *__re
 // into the origin) in LDS; each of the four waves then computes ROWS rows,
 // one column per lane, with a ROWS-row register ring fed from LDS.  Taps run
 // in chunks of 8 (the tap pool is zero padded), so the ring indices are
-// static.  ROWS = 8 (the default: at most 79 VGPRs, 6 waves per SIMD) or 16
-// (twice the filter work per LDS read, at most 128 VGPRs and 4 waves); the
-// outputs are the same bit for bit.
+// static.  ROWS = 8 (the default) or 16; the outputs are the same bit for bit.
+//
+// MFMA: the filter on the matrix cores, the staged rows a ring in LDS (nothing
+// moves from tile to tile; with the move 1-4% slower).  Bound by memory at some
+// 4 TB/s of scattered grids, and by the barriers between filter and epilogue;
+// us per launch of 96 (32 for the root) messages of 300x300x24, by destination
+// kind, vector unit / MFMA 8 rows / 16 rows: downward middle 1340 / 1286 /
+// 1278, downward leaf 1055 / 948 / 1057, up root 978 / 870 / 935, up node 825
+// / 780 / 838.  The vector unit's filter is left for taps so many that the
+// operand does not fit LDS beside the rows.
 
 constexpr int kColTileX = 64;
 constexpr int kColWaves = 4;
@@ -544,6 +718,63 @@ __device__ __forceinline__ void col_chunk(float (&acc)[ROWS], float (&buf)[ROWS]
   }
 }
 
+// The y filter of a wave's ROWS rows x 64 columns on the MFMA: lane = column,
+// acc[g] = rows 4 g .. 4 g + 3, which take the taps f[k - i] against row k on
+// from the wave's first; a ring of ROWS / 4 row quads in registers, each read
+// once for all groups from the tile's ring of n rows (a multiple of 4; col:
+// this lane's column, row: the wave's first row).  The quads read behind the
+// tile's are the ring's oldest and multiplied by nothing.
+template <int ROWS>
+__device__ __forceinline__ void yfilter4(const float *col, int row, int n, const float *t4, int ky, float (&a)[ROWS]) {
+  constexpr int G = ROWS / 4;
+  const int NT = tap4_chunks(ky);
+  const float4 *tv = reinterpret_cast<const float4 *>(t4 + (threadIdx.x & 3) * tap4_pitch(ky));
+  f32x4_t acc[G];
+  float x[G][4];
+  auto quad = [&](float (&q)[4]) {
+    const float *p = col + row * kColTileX;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) q[i] = p[i * kColTileX];
+    row += 4;
+    if (row >= n) row -= n;
+  };
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    acc[g] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    quad(x[g]);
+  }
+  auto step = [&](auto uc) {
+    constexpr int u = decltype(uc)::value;
+    const float4 t = *tv++;
+#pragma unroll
+    for (int g = 0; g < G; ++g) acc[g] = mfma4(t.x, x[(u + g) % G][0], acc[g]);
+#pragma unroll
+    for (int g = 0; g < G; ++g) acc[g] = mfma4(t.y, x[(u + g) % G][1], acc[g]);
+#pragma unroll
+    for (int g = 0; g < G; ++g) acc[g] = mfma4(t.z, x[(u + g) % G][2], acc[g]);
+#pragma unroll
+    for (int g = 0; g < G; ++g) acc[g] = mfma4(t.w, x[(u + g) % G][3], acc[g]);
+    quad(x[u]);
+  };
+  using std::integral_constant;
+  int c = 0;
+  for (; c + G <= NT; c += G) {
+    step(integral_constant<int, 0>{});
+    step(integral_constant<int, 1>{});
+    if constexpr (G == 4) {
+      step(integral_constant<int, 2>{});
+      step(integral_constant<int, 3>{});
+    }
+  }
+  if (c < NT) step(integral_constant<int, 0>{});
+  if constexpr (G == 4) {
+    if (c + 1 < NT) step(integral_constant<int, 1>{});
+    if (c + 2 < NT) step(integral_constant<int, 2>{});
+  }
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i) a[i] = acc[i >> 2][i & 3];
+}
+
 // The caller's accumulation is a template (EPI, one variant per destination
 // kind), so every load of a tile is unconditional straight-line code: the
 // epilogue operands first, then the next tile's rows (always loaded, clamped
@@ -551,7 +782,7 @@ __device__ __forceinline__ void col_chunk(float (&acc)[ROWS], float (&buf)[ROWS]
 // operands only.
 // SPLIT: the launch may hold a split warp (J.split), whose inverse offsets
 // change once along x (per lane) or y (a second segment of rows)
-template <int EPI, int ROWS, bool SPLIT>
+template <int EPI, int ROWS, bool SPLIT, bool MFMA>
 __device__ __forceinline__ void colpass_strip(const Bases &b, const MsgJob &J, const float *__restrict__ taps,
                                               const int *__restrict__ shifts, int R, int r, int xt, float *tile) {
   constexpr int kColRows = ROWS;
@@ -580,6 +811,16 @@ __device__ __forceinline__ void colpass_strip(const Bases &b, const MsgJob &J, c
   const int Lp = col_padded_taps(ky);
   const int nrows = col_tile_rows(ky, ROWS);
   const float *fy = taps + J.taps_y;
+  // MFMA: the tap operand and a flag (a non-finite value was staged: the
+  // strip goes on a tap at a time) behind the tile
+  float *t4 = tile + nrows * kColTileX;
+  unsigned *bad = reinterpret_cast<unsigned *>(t4 + 4 * tap4_pitch(ky));
+  unsigned bits = 0u;
+  if (MFMA) {
+    tap4_fill(t4, fy, ky);
+    if (threadIdx.x == 0) *bad = 0u;
+    __syncthreads();
+  }
   const float M = key2f(b.max_keys[J.src_key]);
   // row pitches: pa of dst (and of the unary a marginal adds), pb of the
   // grids at the other pitch (EpiPitch)
@@ -614,11 +855,14 @@ __device__ __forceinline__ void colpass_strip(const Bases &b, const MsgJob &J, c
     if (ylo >= yhi) continue;
     const int oy = seg == 0 ? oy0 : oy0 + ystep;
     if (seg) __syncthreads();  // every wave is done with the first segment's tile
+    int base = 0;  // MFMA: ring row of the tile's first row
     for (int rr = wave; rr < nrows; rr += kColWaves) {
       const int row = ylo + oy - ky + rr;
-      const float v = src_raw(row);
-      tile[rr * kColTileX + lane] = src_ok(row) ? v : 0.0f;
+      const float raw = src_raw(row), v = src_ok(row) ? raw : 0.0f;
+      bits = max_bits(bits, v);
+      tile[rr * kColTileX + lane] = v;
     }
+    if (MFMA && bits >= kNonFinite) *bad = 1u;
     __syncthreads();
 
     for (int ty0 = ylo; ty0 < yhi; ty0 += kColTileY) {
@@ -656,28 +900,32 @@ __device__ __forceinline__ void colpass_strip(const Bases &b, const MsgJob &J, c
       for (int k = 0; k < kNew; ++k) pre[k] = src_raw(s1 + wave + kColWaves * k);
 
       const float *tw = tile + wave * kColRows * kColTileX + lane;
-      float a[kColRows], buf[kColRows];
+      float a[kColRows] = {};
+      int row0 = base + wave * kColRows;  // of the ring (MFMA)
+      if (row0 >= nrows) row0 -= nrows;
+      if (MFMA && __builtin_amdgcn_readfirstlane(*bad) == 0u) {
+        yfilter4<ROWS>(tile + lane, row0, nrows, t4, ky, a);
+      } else if (MFMA) {
+        for (int i = 0; i < kColRows; ++i) {
+          float v = 0.0f;
+          for (int t = 0; t < Lp; ++t) {
+            int rr = row0 + i + t;
+            if (rr >= nrows) rr -= nrows;
+            v = fmaf(tile[rr * kColTileX + lane], fy[t], v);
+          }
 #pragma unroll
-      for (int i = 0; i < kColRows; ++i) {
-        a[i] = 0.0f;
-        buf[i] = tw[i * kColTileX];
-      }
-      // taps in runs of the ring's period, then a tail (the tap count is
-      // padded to a multiple of 4 with zero taps)
-      int t0 = 0;
-      if constexpr (ROWS == 16) {
-        for (; t0 + 16 <= Lp; t0 += 16) {
-          col_chunk<0, 8, ROWS>(a, buf, fy, tw, t0);
-          col_chunk<8, 8, ROWS>(a, buf, fy, tw, t0 + 8);
-        }
-        const int rem = Lp - t0;
-        if (rem >= 8) {
-          col_chunk<0, 8, ROWS>(a, buf, fy, tw, t0);
-          if (rem == 12) col_chunk<8, 4, ROWS>(a, buf, fy, tw, t0 + 8);
-        } else if (rem == 4) {
-          col_chunk<0, 4, ROWS>(a, buf, fy, tw, t0);
+          for (int j = 0; j < kColRows; ++j) a[j] = j == i ? v : a[j];
         }
       } else {
+        float buf[kColRows];
+#pragma unroll
+        for (int i = 0; i < kColRows; ++i) {
+          a[i] = 0.0f;
+          buf[i] = tw[i * kColTileX];
+        }
+        // taps in runs of the ring's period, then a tail (the tap count is
+        // padded to a multiple of 4 with zero taps)
+        int t0 = 0;
         for (; t0 + 8 <= Lp; t0 += 8) col_chunk<0, 8, ROWS>(a, buf, fy, tw, t0);
         if (Lp - t0 == 4) col_chunk<0, 4, ROWS>(a, buf, fy, tw, t0);
       }
@@ -699,27 +947,38 @@ __device__ __forceinline__ void colpass_strip(const Bases &b, const MsgJob &J, c
                     kNeedB ? pbel[i] : 0.0f, xmask, leaf_u);
       }
       if (more) {
-        // move rows [64, nrows) to [0, Lp), then store the prefetched rows
-        for (int c0 = 0; c0 < Lp; c0 += kColMove * kColWaves) {
-          float mv[kColMove];
-          __syncthreads();  // every wave is done with this tile
+        if (MFMA) {
+          __syncthreads();  // every wave is done with the ring's oldest rows
+        } else {
+          // move rows [kColTileY, nrows) to [0, Lp), then store the prefetched rows
+          for (int c0 = 0; c0 < Lp; c0 += kColMove * kColWaves) {
+            float mv[kColMove];
+            __syncthreads();  // every wave is done with this tile
 #pragma unroll
-          for (int k = 0; k < kColMove; ++k) {
-            const int rr = c0 + wave + kColWaves * k;
-            if (rr < Lp) mv[k] = tile[(kColTileY + rr) * kColTileX + lane];
-          }
-          __syncthreads();
+            for (int k = 0; k < kColMove; ++k) {
+              const int rr = c0 + wave + kColWaves * k;
+              if (rr < Lp) mv[k] = tile[(kColTileY + rr) * kColTileX + lane];
+            }
+            __syncthreads();
 #pragma unroll
-          for (int k = 0; k < kColMove; ++k) {
-            const int rr = c0 + wave + kColWaves * k;
-            if (rr < Lp) tile[rr * kColTileX + lane] = mv[k];
+            for (int k = 0; k < kColMove; ++k) {
+              const int rr = c0 + wave + kColWaves * k;
+              if (rr < Lp) tile[rr * kColTileX + lane] = mv[k];
+            }
           }
         }
 #pragma unroll
         for (int k = 0; k < kNew; ++k) {
           const int row = s1 + wave + kColWaves * k;
-          tile[(Lp + wave + kColWaves * k) * kColTileX + lane] = src_ok(row) ? pre[k] : 0.0f;
+          const float v = src_ok(row) ? pre[k] : 0.0f;
+          bits = max_bits(bits, v);
+          int rr = (MFMA ? base : Lp) + wave + kColWaves * k;
+          if (MFMA && rr >= nrows) rr -= nrows;
+          tile[rr * kColTileX + lane] = v;
         }
+        if (MFMA && bits >= kNonFinite) *bad = 1u;
+        base += kColTileY;
+        if (base >= nrows) base -= nrows;
         __syncthreads();
       }
     }
@@ -733,7 +992,7 @@ __device__ __forceinline__ void colpass_strip(const Bases &b, const MsgJob &J, c
 // epilogue fits without spilling vector registers once its stored belief is
 // loaded after the filter (2.16 -> 1.33 ms per launch on 32 300x300x24
 // grids; unbounded, at 156 VGPRs and 3 waves per SIMD, it takes 1.65 ms).
-template <int HI, int ROWS, bool SPLIT>
+template <int HI, int ROWS, bool SPLIT, bool MFMA>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_colpass(
     Bases b, const MsgJob *__restrict__ jobs, const float *__restrict__ taps, const int *__restrict__ shifts, int R,
     int xtiles) {
@@ -748,15 +1007,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
   if (xt * kColTileX >= J.W) return;
   const int kind = epi_kind(J);
   if (HI == kEpiUpRoot || kind == kEpiUpRoot)
-    colpass_strip<kEpiUpRoot, ROWS, SPLIT>(b, J, taps, shifts, R, r, xt, tile);
+    colpass_strip<kEpiUpRoot, ROWS, SPLIT, MFMA>(b, J, taps, shifts, R, r, xt, tile);
   else if (HI == kEpiUpNode || kind == kEpiUpNode)
-    colpass_strip<kEpiUpNode, ROWS, SPLIT>(b, J, taps, shifts, R, r, xt, tile);
+    colpass_strip<kEpiUpNode, ROWS, SPLIT, MFMA>(b, J, taps, shifts, R, r, xt, tile);
   else if (HI == kEpiUpNodeU || kind == kEpiUpNodeU)
-    colpass_strip<kEpiUpNodeU, ROWS, SPLIT>(b, J, taps, shifts, R, r, xt, tile);
+    colpass_strip<kEpiUpNodeU, ROWS, SPLIT, MFMA>(b, J, taps, shifts, R, r, xt, tile);
   else if (HI == kEpiDownLeaf || kind == kEpiDownLeaf)
-    colpass_strip<kEpiDownLeaf, ROWS, SPLIT>(b, J, taps, shifts, R, r, xt, tile);
+    colpass_strip<kEpiDownLeaf, ROWS, SPLIT, MFMA>(b, J, taps, shifts, R, r, xt, tile);
   else
-    colpass_strip<kEpiDownMid, ROWS, SPLIT>(b, J, taps, shifts, R, r, xt, tile);
+    colpass_strip<kEpiDownMid, ROWS, SPLIT, MFMA>(b, J, taps, shifts, R, r, xt, tile);
 }
 
 // ----------------------------------------------------------------- k_root
@@ -981,6 +1240,10 @@ size_t rowpass_lds_bytes(int R, int W, int kx) {
   size_t p = rowpass_fixed(R) ? (size_t)(R / row_groups(R)) * g.Pw : (size_t)R * g.Pw + (size_t)R * ((W + 3) & ~3);
   return sizeof(float) * p;
 }
+// with the x filter on the matrix cores; 0 where there is no such kernel
+size_t rowpass4_lds_bytes(int R, int W, int kx) {
+  return rowpass_fixed(R) ? row4_lds_bytes(row4_slices(R), W, kx) : 0;
+}
 
 // The dynamic-LDS attribute of a kernel is one process-wide value per device
 // and function, while plans with different needs coexist: it is only ever
@@ -1001,93 +1264,124 @@ hipError_t raise_lds_limit(const void *f, size_t bytes) {
   return e;
 }
 
-hipError_t rowpass_set_lds_limit(size_t bytes) {
-  hipError_t e = raise_lds_limit(reinterpret_cast<const void *>(&k_rowpass_r<24, false>), bytes);
-  if (e == hipSuccess) e = raise_lds_limit(reinterpret_cast<const void *>(&k_rowpass_r<48, false>), bytes);
-  if (e == hipSuccess) e = raise_lds_limit(reinterpret_cast<const void *>(&k_rowpass_r<24, true>), bytes);
-  if (e == hipSuccess) e = raise_lds_limit(reinterpret_cast<const void *>(&k_rowpass_r<48, true>), bytes);
+// bytes, bytes4: the vector and the MFMA row pass's largest LDS
+hipError_t rowpass_set_lds_limit(size_t bytes, size_t bytes4) {
+  hipError_t e = raise_lds_limit(reinterpret_cast<const void *>(&k_rowpass_r<24, false, false>), bytes);
+  if (e == hipSuccess) e = raise_lds_limit(reinterpret_cast<const void *>(&k_rowpass_r<48, false, false>), bytes);
+  if (e == hipSuccess) e = raise_lds_limit(reinterpret_cast<const void *>(&k_rowpass_r<24, true, false>), bytes);
+  if (e == hipSuccess) e = raise_lds_limit(reinterpret_cast<const void *>(&k_rowpass_r<48, true, false>), bytes);
+  if (e == hipSuccess) e = raise_lds_limit(reinterpret_cast<const void *>(&k_rowpass_r<24, false, true>), bytes4);
+  if (e == hipSuccess) e = raise_lds_limit(reinterpret_cast<const void *>(&k_rowpass_r<48, false, true>), bytes4);
+  if (e == hipSuccess) e = raise_lds_limit(reinterpret_cast<const void *>(&k_rowpass_r<24, true, true>), bytes4);
+  if (e == hipSuccess) e = raise_lds_limit(reinterpret_cast<const void *>(&k_rowpass_r<48, true, true>), bytes4);
   if (e != hipSuccess) return e;
   return raise_lds_limit(reinterpret_cast<const void *>(&k_rowpass_any), bytes);
 }
 
-template <int ROWS, bool SPLIT>
+template <int ROWS, bool SPLIT, bool MFMA>
 static hipError_t colpass_rows_set_lds_limit(size_t bytes) {
-  hipError_t e = raise_lds_limit(reinterpret_cast<const void *>(&k_colpass<kEpiUpRoot, ROWS, SPLIT>), bytes);
-  if (e == hipSuccess) e = raise_lds_limit(reinterpret_cast<const void *>(&k_colpass<kEpiUpNode, ROWS, SPLIT>), bytes);
-  if (e == hipSuccess) e = raise_lds_limit(reinterpret_cast<const void *>(&k_colpass<kEpiUpNodeU, ROWS, SPLIT>), bytes);
-  if (e == hipSuccess) e = raise_lds_limit(reinterpret_cast<const void *>(&k_colpass<kEpiDownLeaf, ROWS, SPLIT>), bytes);
-  if (e == hipSuccess) e = raise_lds_limit(reinterpret_cast<const void *>(&k_colpass<kEpiDownMid, ROWS, SPLIT>), bytes);
+  hipError_t e = raise_lds_limit(reinterpret_cast<const void *>(&k_colpass<kEpiUpRoot, ROWS, SPLIT, MFMA>), bytes);
+  if (e == hipSuccess) e = raise_lds_limit(reinterpret_cast<const void *>(&k_colpass<kEpiUpNode, ROWS, SPLIT, MFMA>), bytes);
+  if (e == hipSuccess) e = raise_lds_limit(reinterpret_cast<const void *>(&k_colpass<kEpiUpNodeU, ROWS, SPLIT, MFMA>), bytes);
+  if (e == hipSuccess) e = raise_lds_limit(reinterpret_cast<const void *>(&k_colpass<kEpiDownLeaf, ROWS, SPLIT, MFMA>), bytes);
+  if (e == hipSuccess) e = raise_lds_limit(reinterpret_cast<const void *>(&k_colpass<kEpiDownMid, ROWS, SPLIT, MFMA>), bytes);
   return e;
 }
 
-// bytes: the LDS of the 16-row tile (the larger one)
-hipError_t colpass_set_lds_limit(size_t bytes) {
-  hipError_t e = colpass_rows_set_lds_limit<8, false>(bytes);
-  if (e == hipSuccess) e = colpass_rows_set_lds_limit<16, false>(bytes);
-  if (e == hipSuccess) e = colpass_rows_set_lds_limit<8, true>(bytes);
+// bytes: the LDS of the vector column pass; bytes4: of the MFMA one's 16-row
+// tile (the larger one)
+hipError_t colpass_set_lds_limit(size_t bytes, size_t bytes4) {
+  hipError_t e = colpass_rows_set_lds_limit<8, false, false>(bytes);
+  if (e == hipSuccess) e = colpass_rows_set_lds_limit<8, true, false>(bytes);
+  if (e == hipSuccess) e = colpass_rows_set_lds_limit<8, false, true>(bytes4);
+  if (e == hipSuccess) e = colpass_rows_set_lds_limit<16, false, true>(bytes4);
+  if (e == hipSuccess) e = colpass_rows_set_lds_limit<8, true, true>(bytes4);
   return e;
+}
+
+template <bool MFMA>
+static void launch_rowpass_r(int R, bool split, dim3 grid, dim3 blk, size_t lds_bytes, hipStream_t s, const Bases &b,
+                             const MsgJob *jobs, const float *taps, const int *shifts) {
+  if (R == 24 && !split)
+    hipLaunchKernelGGL((k_rowpass_r<24, false, MFMA>), grid, blk, lds_bytes, s, b, jobs, taps, shifts);
+  else if (R == 24)
+    hipLaunchKernelGGL((k_rowpass_r<24, true, MFMA>), grid, blk, lds_bytes, s, b, jobs, taps, shifts);
+  else if (!split)  // 48: the reference's default grid
+    hipLaunchKernelGGL((k_rowpass_r<48, false, MFMA>), grid, blk, lds_bytes, s, b, jobs, taps, shifts);
+  else
+    hipLaunchKernelGGL((k_rowpass_r<48, true, MFMA>), grid, blk, lds_bytes, s, b, jobs, taps, shifts);
 }
 
 // threads: block size (a multiple of 64; 0 = one thread per column, at most
 // 512); every loop of the row pass strides by the block size
 // split: some job's warp changes its offset along an axis (MsgJob::split)
+// lds4_bytes: LDS of the row pass with its x filter on the matrix cores, or 0
+// where the rows do not fit it
 hipError_t launch_rowpass(const Bases &b, const MsgJob *jobs, int n_jobs, const float *taps, const int *shifts,
-                          int R, int max_h, int max_w, size_t lds_bytes, hipStream_t s, int threads, bool split) {
+                          int R, int max_h, int max_w, size_t lds_bytes, size_t lds4_bytes, hipStream_t s, int threads,
+                          bool split) {
   if (n_jobs <= 0) return hipSuccess;
   dim3 grid(max_h, n_jobs);
   const int nt = threads > 0 ? std::min(threads, std::max(64, (max_w + 63) / 64 * 64))
                              : std::min(512, (max_w + 63) / 64 * 64);
-  if (R == 24 && !split)
-    hipLaunchKernelGGL((k_rowpass_r<24, false>), grid, dim3(nt), lds_bytes, s, b, jobs, taps, shifts);
-  else if (R == 24)
-    hipLaunchKernelGGL((k_rowpass_r<24, true>), grid, dim3(nt), lds_bytes, s, b, jobs, taps, shifts);
-  else if (R == 48 && !split)  // the reference's default grid
-    hipLaunchKernelGGL((k_rowpass_r<48, false>), grid, dim3(nt), lds_bytes, s, b, jobs, taps, shifts);
-  else if (R == 48)
-    hipLaunchKernelGGL((k_rowpass_r<48, true>), grid, dim3(nt), lds_bytes, s, b, jobs, taps, shifts);
-  else
+  if (!rowpass_fixed(R))
     hipLaunchKernelGGL(k_rowpass_any, grid, dim3(nt), lds_bytes, s, b, jobs, taps, shifts, R);
+  else if (lds4_bytes > 0)
+    launch_rowpass_r<true>(R, split, grid, dim3(nt), lds4_bytes, s, b, jobs, taps, shifts);
+  else
+    launch_rowpass_r<false>(R, split, grid, dim3(nt), lds_bytes, s, b, jobs, taps, shifts);
   return hipGetLastError();
 }
 
-// LDS of a column-pass tile: rows 0 = the larger (16-row) tile
+// LDS of the vector column pass's 16-row tile (the bound a filter is accepted
+// by; its 8-row tile, the one that runs, takes 32 rows of 256 bytes less)
 size_t colpass_lds_bytes(int ky, int rows) {
   return sizeof(float) * (size_t)col_tile_rows(ky, rows > 0 ? rows : 16) * kColTileX;
 }
+// LDS of the MFMA column pass's 16-row tile
+size_t colpass4_lds_bytes(int ky) {
+  return sizeof(float) * ((size_t)col_tile_rows(ky, 16) * kColTileX + 4 * tap4_pitch(ky) + 4);
+}
 
-template <int ROWS, bool SPLIT>
+template <int ROWS, bool SPLIT, bool MFMA>
 static void launch_colpass_rows(int epi_hi, dim3 grid, size_t lds_bytes, hipStream_t s, const Bases &b,
                                 const MsgJob *jobs, const float *taps, const int *shifts, int R, int xtiles) {
   const dim3 blk(kColWaves * 64);
   switch (epi_hi) {
-    case kEpiUpRoot: hipLaunchKernelGGL((k_colpass<kEpiUpRoot, ROWS, SPLIT>), grid, blk, lds_bytes, s, b, jobs, taps, shifts, R, xtiles); break;
-    case kEpiUpNode: hipLaunchKernelGGL((k_colpass<kEpiUpNode, ROWS, SPLIT>), grid, blk, lds_bytes, s, b, jobs, taps, shifts, R, xtiles); break;
-    case kEpiUpNodeU: hipLaunchKernelGGL((k_colpass<kEpiUpNodeU, ROWS, SPLIT>), grid, blk, lds_bytes, s, b, jobs, taps, shifts, R, xtiles); break;
-    case kEpiDownLeaf: hipLaunchKernelGGL((k_colpass<kEpiDownLeaf, ROWS, SPLIT>), grid, blk, lds_bytes, s, b, jobs, taps, shifts, R, xtiles); break;
-    default: hipLaunchKernelGGL((k_colpass<kEpiDownMid, ROWS, SPLIT>), grid, blk, lds_bytes, s, b, jobs, taps, shifts, R, xtiles); break;
+    case kEpiUpRoot: hipLaunchKernelGGL((k_colpass<kEpiUpRoot, ROWS, SPLIT, MFMA>), grid, blk, lds_bytes, s, b, jobs, taps, shifts, R, xtiles); break;
+    case kEpiUpNode: hipLaunchKernelGGL((k_colpass<kEpiUpNode, ROWS, SPLIT, MFMA>), grid, blk, lds_bytes, s, b, jobs, taps, shifts, R, xtiles); break;
+    case kEpiUpNodeU: hipLaunchKernelGGL((k_colpass<kEpiUpNodeU, ROWS, SPLIT, MFMA>), grid, blk, lds_bytes, s, b, jobs, taps, shifts, R, xtiles); break;
+    case kEpiDownLeaf: hipLaunchKernelGGL((k_colpass<kEpiDownLeaf, ROWS, SPLIT, MFMA>), grid, blk, lds_bytes, s, b, jobs, taps, shifts, R, xtiles); break;
+    default: hipLaunchKernelGGL((k_colpass<kEpiDownMid, ROWS, SPLIT, MFMA>), grid, blk, lds_bytes, s, b, jobs, taps, shifts, R, xtiles); break;
   }
 }
 
 // epi_hi: the highest destination kind (EpiKind) among the jobs; rows:
-// output rows per lane (8 or 16; 0 = the default); lds_bytes_16: the LDS of
-// the 16-row tile for the jobs' widest y filter (the 8-row tile takes 32
-// rows of 256 bytes less)
+// output rows per lane (8 or 16; 0 = the default); lds_bytes_16, lds4_bytes_16:
+// the LDS of the 16-row tile for the jobs' widest y filter, without and with
+// the MFMA's tap operand (0: it does not fit, the filter runs on the vector
+// unit, 8 rows per lane); an 8-row tile takes 32 rows of 256 bytes less
 // (split: some job's warp changes its offset along an axis; those launches
 // take 8 rows per lane)
 hipError_t launch_colpass(const Bases &b, const MsgJob *jobs, int n_jobs, const float *taps, const int *shifts,
-                          int R, int epi_hi, int max_w, size_t lds_bytes_16, hipStream_t s, int rows, bool split) {
+                          int R, int epi_hi, int max_w, size_t lds_bytes_16, size_t lds4_bytes_16, hipStream_t s,
+                          int rows, bool split) {
   if (n_jobs <= 0) return hipSuccess;
   if (rows == 0 || split) rows = kColRowsDefault;
   if (epi_hi < kEpiUpRoot || epi_hi > kEpiDownMid || (rows != 8 && rows != 16)) return hipErrorInvalidValue;
   const int xtiles = (max_w + kColTileX - 1) / kColTileX;
   dim3 grid(R * xtiles, n_jobs);
-  const size_t lds_8 = lds_bytes_16 - sizeof(float) * kColWaves * 8 * kColTileX;
-  if (split)
-    launch_colpass_rows<8, true>(epi_hi, grid, lds_8, s, b, jobs, taps, shifts, R, xtiles);
+  const size_t less = sizeof(float) * kColWaves * 8 * kColTileX;
+  if (lds4_bytes_16 == 0 && split)
+    launch_colpass_rows<8, true, false>(epi_hi, grid, lds_bytes_16 - less, s, b, jobs, taps, shifts, R, xtiles);
+  else if (lds4_bytes_16 == 0)
+    launch_colpass_rows<8, false, false>(epi_hi, grid, lds_bytes_16 - less, s, b, jobs, taps, shifts, R, xtiles);
+  else if (split)
+    launch_colpass_rows<8, true, true>(epi_hi, grid, lds4_bytes_16 - less, s, b, jobs, taps, shifts, R, xtiles);
   else if (rows == 16)
-    launch_colpass_rows<16, false>(epi_hi, grid, lds_bytes_16, s, b, jobs, taps, shifts, R, xtiles);
+    launch_colpass_rows<16, false, true>(epi_hi, grid, lds4_bytes_16, s, b, jobs, taps, shifts, R, xtiles);
   else
-    launch_colpass_rows<8, false>(epi_hi, grid, lds_8, s, b, jobs, taps, shifts, R, xtiles);
+    launch_colpass_rows<8, false, true>(epi_hi, grid, lds4_bytes_16 - less, s, b, jobs, taps, shifts, R, xtiles);
   return hipGetLastError();
 }
 

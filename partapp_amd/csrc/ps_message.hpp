@@ -20,7 +20,7 @@ struct MessageSetup {
   bool od = false;          // off-diagonal covariance: eigenbasis stages instead of the column pass
   bool split = false;       // a warp whose offset changes along an axis (MsgJob::split)
   OdExtent od_ext;          // launches of the eigenbasis stages
-  size_t lds = 0, col_lds = 0;
+  size_t lds = 0, lds4 = 0, col_lds = 0, col_lds4 = 0;
   // byte offsets in the block: job, max job, taps, shifts, max key, argmax key, grids
   size_t o_job = 0, o_max = 0, o_taps = 0, o_sh = 0, o_key = 0, o_mk = 0, o_T = 0;
   size_t total = 0;         // bytes of the block
