@@ -58,28 +58,68 @@ __device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v)
 // that run): every block of its jobs exits at once.
 __device__ __forceinline__ bool skip_inst(const Bases &b, int inst) { return b.active && b.active[inst] == 0u; }
 
-// Top-2 value keys of a wave's outputs (per lane k1 >= k2, every state seen
-// by one lane only), merged across the wave and then into a slot's
-// (best << 32) | second word with a compare-and-swap loop; the word only
-// grows, so the loop ends.  Every lane of the wave calls it.
-__device__ __forceinline__ void top2_flush(unsigned long long *slot, unsigned k1, unsigned k2, int lane) {
+// A block's result for the keys it feeds: the waves' parts, each merged over
+// its lanes, meet in LDS and one thread raises the keys.  Atomics on one cache
+// line queue up at 4 to 13 ns each, and all keys of an instance share a line: a
+// wave each, the leaf maxima of an image of 300x300x48 took 70 us for 17 us of
+// reading.  (Reading a key first and raising it only where it is lower queues up
+// just as much once thousands of waves are in flight, and each then waits for
+// its answer: 957 instead of 299 us for the leaf maxima of 32 images.)
+struct KeyPart {
+  unsigned key = 0u;                // of a source's maximum
+  unsigned long long amax = 0ull;   // (value key << 32) | flipped index of the best state
+  unsigned second = 0u;             // value key of the second best state, for the MAP certificate
+  __device__ __forceinline__ void merge(const KeyPart &o) {
+    key = max(key, o.key);
+    second = max(max(second, o.second), min((unsigned)(amax >> 32), (unsigned)(o.amax >> 32)));
+    amax = o.amax > amax ? o.amax : amax;
+  }
+};
+// the top-2 of a wave's lanes (k1 >= k2, every state seen by one lane only):
+// the second key, in every lane
+__device__ __forceinline__ unsigned wave_second(unsigned k1, unsigned k2) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
     const unsigned o1 = (unsigned)__shfl_xor((int)k1, o, 64), o2 = (unsigned)__shfl_xor((int)k2, o, 64);
     k2 = max(max(k2, o2), min(k1, o1));
     k1 = max(k1, o1);
   }
-  if (lane == 0 && k1) {
-    unsigned long long old = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    for (;;) {
-      const unsigned a1 = (unsigned)(old >> 32), a2 = (unsigned)old;
-      const unsigned long long nw = ((unsigned long long)max(a1, k1) << 32) | max(max(a2, k2), min(a1, k1));
-      if (nw == old) break;
-      const unsigned long long prev = atomicCAS(slot, old, nw);
-      if (prev == old) break;
-      old = prev;
-    }
+  return k2;
+}
+// A (best << 32) | second word raised by a compare-and-swap loop; the word
+// only grows, so the loop ends.
+__device__ __forceinline__ void top2_raise(unsigned long long *slot, unsigned k1, unsigned k2) {
+  unsigned long long old = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  for (;;) {
+    const unsigned a1 = (unsigned)(old >> 32), a2 = (unsigned)old;
+    const unsigned long long nw = ((unsigned long long)max(a1, k1) << 32) | max(max(a2, k2), min(a1, k1));
+    if (nw == old) break;
+    const unsigned long long prev = atomicCAS(slot, old, nw);
+    if (prev == old) break;
+    old = prev;
   }
+}
+// Every thread of the block calls it, with its wave's part; red holds one
+// entry per wave (LDS that no thread reads or writes any more).  Null keys are
+// not fed.
+__device__ __forceinline__ void block_raise(uint4 *red, KeyPart p, unsigned *max_key, unsigned long long *map_key,
+                                            unsigned long long *top2_key) {
+  const int waves = (int)(blockDim.x >> 6);
+  if ((threadIdx.x & 63) == 0)
+    red[threadIdx.x >> 6] = make_uint4(p.key, (unsigned)p.amax, (unsigned)(p.amax >> 32), p.second);
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  for (int w = 1; w < waves; ++w) {
+    const uint4 v = red[w];
+    KeyPart o;
+    o.key = v.x;
+    o.amax = (unsigned long long)v.z << 32 | v.y;
+    o.second = v.w;
+    p.merge(o);
+  }
+  if (max_key && p.key) atomicMax(max_key, p.key);
+  if (map_key && p.amax) atomicMax(map_key, p.amax);
+  if (top2_key && p.amax) top2_raise(top2_key, (unsigned)(p.amax >> 32), p.second);
 }
 // one more value key into a lane's top-2
 __device__ __forceinline__ void top2_add(unsigned &k1, unsigned &k2, unsigned k) {
@@ -235,19 +275,22 @@ struct Epi {
     if (pad_a) at(dst, eb) = kLogZero;
     if (kNeedB && pad_b) at(dst2, ebs) = kLogZero;
   }
-  // wave reductions and one atomic per wave; every lane of the wave calls it
-  __device__ __forceinline__ void flush(const Bases &b, const MsgJob &J, long long slice0, int lane) {
-    if (EPI == kEpiUpNode || EPI == kEpiUpNodeU || EPI == kEpiDownMid) {
-      const unsigned k = wave_max_u32(vmax > -INFINITY ? f2key(vmax) : 0u);
-      if (lane == 0 && k) atomicMax(b.max_keys + (kDown ? J.dst2_key : J.dst_key), k);
-    }
+  // the keys the outputs feed; every thread of the block calls it, and lds (16
+  // bytes per wave) is free once all have
+  __device__ __forceinline__ void flush(const Bases &b, const MsgJob &J, long long slice0, void *lds) {
+    constexpr bool kKey = EPI == kEpiUpNode || EPI == kEpiUpNodeU || EPI == kEpiDownMid;
+    if (!kKey && !kDown) return;
+    KeyPart p;
+    if (kKey) p.key = wave_max_u32(vmax > -INFINITY ? f2key(vmax) : 0u);
     if (kDown) {
       const unsigned flat = (unsigned)(slice0 + (best_eb >> 2));
-      const unsigned long long m =
-          wave_max_u64(best_key ? ((unsigned long long)best_key << 32) | (0xffffffffull - flat) : 0ull);
-      if (lane == 0 && m) atomicMax(b.map_keys + J.map_slot, m);
-      if (b.top2_keys) top2_flush(b.top2_keys + J.map_slot, best_key, second_key, lane);
+      p.amax = wave_max_u64(best_key ? ((unsigned long long)best_key << 32) | (0xffffffffull - flat) : 0ull);
+      if (b.top2_keys) p.second = wave_second(best_key, second_key);
     }
+    __syncthreads();
+    block_raise(static_cast<uint4 *>(lds), p, kKey ? b.max_keys + (kDown ? J.dst2_key : J.dst_key) : nullptr,
+                kDown ? b.map_keys + J.map_slot : nullptr,
+                kDown && b.top2_keys ? b.top2_keys + J.map_slot : nullptr);
   }
 };
 
@@ -302,29 +345,19 @@ __device__ __forceinline__ void dst_store(const MsgJob &J, float *dst, float *ds
   }
 }
 
-// Raise a key to v where it is lower: most waves only read it (same-address
-// atomics of a level's thousands of waves queue up at one cache line).
-__device__ __forceinline__ void raise_key(unsigned *k, unsigned v) {
-  if (__hip_atomic_load(k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < v) atomicMax(k, v);
-}
-__device__ __forceinline__ void raise_key(unsigned long long *k, unsigned long long v) {
-  if (__hip_atomic_load(k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < v) atomicMax(k, v);
-}
-
-// Wave reductions of DstAcc and one atomic per wave; every lane of the wave
-// calls it.
-__device__ __forceinline__ void dst_flush(const Bases &b, const MsgJob &J, bool has_dst2, DstAcc &a, int lane) {
+// The keys DstAcc feeds; every thread of the block calls it (red: LDS, an
+// entry per wave).
+__device__ __forceinline__ void dst_flush(const Bases &b, const MsgJob &J, bool has_dst2, const DstAcc &a, uint4 *red) {
+  KeyPart p;
   if (J.dst_kind == kDstUpNode) {
-    const unsigned v = wave_max_u32(a.kmax1);
-    if (lane == 0 && v) raise_key(b.max_keys + J.dst_key, v);
+    p.key = wave_max_u32(a.kmax1);
+    block_raise(red, p, b.max_keys + J.dst_key, nullptr, nullptr);
   } else if (J.dst_kind == kDstDown) {
-    const unsigned long long m = wave_max_u64(a.amax);
-    if (lane == 0 && m) raise_key(b.map_keys + J.map_slot, m);
-    if (b.top2_keys) top2_flush(b.top2_keys + J.map_slot, (unsigned)(a.amax >> 32), a.second, lane);
-    if (has_dst2) {
-      const unsigned v = wave_max_u32(a.kmax2);
-      if (lane == 0 && v) raise_key(b.max_keys + J.dst2_key, v);
-    }
+    p.amax = wave_max_u64(a.amax);
+    if (b.top2_keys) p.second = wave_second((unsigned)(a.amax >> 32), a.second);
+    if (has_dst2) p.key = wave_max_u32(a.kmax2);
+    block_raise(red, p, has_dst2 ? b.max_keys + J.dst2_key : nullptr, b.map_keys + J.map_slot,
+                b.top2_keys ? b.top2_keys + J.map_slot : nullptr);
   }
 }
 

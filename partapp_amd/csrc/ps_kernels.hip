@@ -117,59 +117,73 @@ __device__ __forceinline__ unsigned max_bits(unsigned m, float v) { return max(m
 
 // ------------------------------------------------------------------ k_max
 // Max of a leaf's source grid (getMinMax, multi_array_op.hpp:60-77).  Grids
-// without masks are scanned flat with 16-byte loads; masked ones by rows.
+// without masks are scanned flat with 16-byte loads, whatever their alignment;
+// masked ones by rows, a wave each, over the states the masks leave.
 
 __global__ __launch_bounds__(256) void k_max(Bases b, const MaxJob *__restrict__ jobs, int R, int chunk) {
+  __shared__ uint4 red[4];
   const MaxJob &J = jobs[blockIdx.y];
   if (skip_inst(b, J.inst)) return;
   const int H = J.H, W = J.W;
-  const long long n = (long long)R * H * W;
-  const long long e0 = (long long)blockIdx.x * chunk;
+  const int n = R * H * W;  // R H pitch < 2^31 is checked when the plan is built
+  const long long e0l = (long long)blockIdx.x * chunk;
+  if (e0l >= n) return;
+  const int e0 = (int)e0l, e1 = min(n - e0, chunk) + e0;
   unsigned km = 0u;
-  if (e0 < n) {
-    const long long e1 = min(e0 + (long long)chunk, n);
-    if (J.src_kind == kSrcZero) {
-      km = f2key(0.0f);
-    } else {
-      const float *src = cptr(b, J.src);
-      const bool plain = J.mask.rot_bits == 0ull && J.mask.strip == 0;
+  if (J.src_kind == kSrcZero) {
+    km = f2key(0.0f);
+  } else {
+    const float *src = cptr(b, J.src);
+    if (J.mask.rot_bits == 0ull && J.mask.strip == 0) {
+      // [a0, a1): whole 16-byte units; the elements before and behind them
+      const int head = (int)((0u - (unsigned)(reinterpret_cast<uintptr_t>(src + e0) >> 2)) & 3u);
+      const int a0 = min(e0 + head, e1), a1 = a0 + ((e1 - a0) & ~3);
+      const int t = (int)threadIdx.x;
+      if (t < a0 - e0) km = f2key(src[e0 + t]);
+      else if (t >= 4 && t - 4 < e1 - a1) km = f2key(src[a1 + t - 4]);
       // four independent loads per thread in flight (a lane past the end
       // reads its first element again, which leaves the max unchanged)
       constexpr int kU = 4;
-      if (plain && ((reinterpret_cast<uintptr_t>(src + e0) & 15) == 0) && ((e1 - e0) & 3) == 0) {
-        const float4 *s4 = reinterpret_cast<const float4 *>(src + e0);
-        const int n4 = (int)((e1 - e0) >> 2);
-        for (int i = threadIdx.x; i < n4; i += kU * blockDim.x) {
-          float4 v[kU];
+      const float4 *s4 = reinterpret_cast<const float4 *>(src + a0);
+      const int n4 = (a1 - a0) >> 2;
+      for (int i = t; i < n4; i += kU * blockDim.x) {
+        float4 v[kU];
 #pragma unroll
-          for (int u = 0; u < kU; ++u) {
-            const int j = i + u * (int)blockDim.x;
-            v[u] = s4[j < n4 ? j : i];
-          }
-#pragma unroll
-          for (int u = 0; u < kU; ++u)
-            km = max(km, max(max(f2key(v[u].x), f2key(v[u].y)), max(f2key(v[u].z), f2key(v[u].w))));
+        for (int u = 0; u < kU; ++u) {
+          const int j = i + u * (int)blockDim.x;
+          v[u] = s4[j < n4 ? j : i];
         }
-      } else {
-        const long long HW = (long long)H * W;
-        for (long long e = e0 + threadIdx.x; e < e1; e += kU * blockDim.x) {
+#pragma unroll
+        for (int u = 0; u < kU; ++u)
+          km = max(km, max(max(f2key(v[u].x), f2key(v[u].y)), max(f2key(v[u].z), f2key(v[u].w))));
+      }
+    } else {
+      // the chunk's rows: those that begin in it
+      const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+      const int row0 = (e0 + W - 1) / W, row1 = (e1 + W - 1) / W;
+      const int x0 = J.mask.strip, x1 = W - J.mask.strip;
+      bool any = J.mask.strip > 0;  // a masked state
+      for (int row = row0 + wave; row < row1; row += 4) {
+        if (masked(J.mask, row / H, x0, W)) {
+          any = true;
+          continue;
+        }
+        constexpr int kU = 4;
+        const float *p = src + row * W;
+        for (int x = x0 + lane; x < x1; x += kU * 64) {
           float v[kU];
 #pragma unroll
-          for (int u = 0; u < kU; ++u) {
-            const long long f = e + u * (long long)blockDim.x;
-            const long long g = f < e1 ? f : e;
-            const int r = (int)(g / HW);
-            const int x = (int)(g % W);
-            v[u] = masked(J.mask, r, x, W) ? kLogZero : src[g];
-          }
+          for (int u = 0; u < kU; ++u) v[u] = p[x + 64 * u < x1 ? x + 64 * u : x];
 #pragma unroll
           for (int u = 0; u < kU; ++u) km = max(km, f2key(v[u]));
         }
       }
+      if (any) km = max(km, f2key(kLogZero));
     }
   }
-  km = wave_max_u32(km);
-  if ((threadIdx.x & 63) == 0 && km != 0u) atomicMax(b.max_keys + J.key, km);
+  KeyPart p;
+  p.key = wave_max_u32(km);
+  block_raise(red, p, b.max_keys + J.key, nullptr, nullptr);
 }
 
 // -------------------------------------------------------------- k_rowpass
@@ -983,7 +997,7 @@ __device__ __forceinline__ void colpass_strip(const Bases &b, const MsgJob &J, c
       }
     }
   }
-  acc.flush(b, J, (long long)r * H * pa, lane);
+  acc.flush(b, J, (long long)r * H * pa, tile);
 }
 
 // HI: the highest destination kind among the launch's jobs (the kernel holds
@@ -1020,17 +1034,35 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 
 // ----------------------------------------------------------------- k_root
 
+// The root belief, its marginal and the children's log_from_root of a block of
+// 128 pixels, 8 waves: two tiles of 64, a quarter of the rotations each, so
+// that an image of 112x128 has 112 blocks of 6 steps in a row rather than 56 of
+// 24.  Bound by memory (11 grids, 3.04 GB in 716 us for 32 images of
+// 300x300x24), on one image by latency.  us before (a wave walks all rotations
+// and raises its own keys) / now: 26 / 11.7 (112x128x24), 99 / 48.6 (300x300x48),
+// 497 / 431 (6 uneven x48), 740 / 716 (32 300x300x24).  A block of 256 pixels:
+// 13.7, 56, 425, 708; half the rotations per wave 18, 55, 443, 719.  Stores
+// through the caches: odd grids' rows leave partial lines, which L2 merges;
+// nontemporal ones took 424 instead of 301 us on 23 uneven grids.
+//
 // KC: the number of root children when it is at most 8 (fully unrolled),
 // else kMaxRootChildren with the count read at run time.
 // LSE64: the root posterior's log-sum-exp over rotations accumulated in FP64
 // with a running maximum shift (the BF16 methods); otherwise in FP32 with
 // no shift, as the reference sums expf (:713-726: a belief above ~88.7
 // overflows to +inf there and here)
+constexpr int kRootWaves = 4;  // per 64 pixels, a quarter of the rotations each
+constexpr int kRootTiles = 2;  // 64-pixel tiles per block
+
 template <int KC, bool LSE64>
-__device__ __forceinline__ void root_pixels(const Bases &b, const RootJob &J, int R, int pix0) {
+__device__ __forceinline__ void root_pixels(const Bases &b, const RootJob &J, int R, int pix0, uint4 *red, float *bels) {
   const int H = J.H, W = J.W;
   const int HW = H * W;
-  const int pix = pix0 + threadIdx.x;
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = wv / kRootTiles, tile = wv % kRootTiles;
+  const int r0 = wave * R / kRootWaves, r1 = (wave + 1) * R / kRootWaves;  // this wave's rotations
+  const int pix = pix0 + tile * 64 + lane;
   const bool ok = pix < HW;
   const int pc = ok ? pix : HW - 1;  // loads of lanes past the end read the last pixel
   const int yc = pc / W;
@@ -1044,30 +1076,27 @@ __device__ __forceinline__ void root_pixels(const Bases &b, const RootJob &J, in
   const int K = KC <= 8 ? KC : J.K;
   const float *un = cptr(b, J.unary);
   float *marg = mptr(b, J.marginal);
+  const bool posts = J.root_post.buf >= 0 && b.root;
 
   unsigned kmax[KC];
 #pragma unroll
   for (int k = 0; k < KC; ++k) kmax[k] = 0u;
   unsigned long long amax = 0ull;
   unsigned second = 0u;  // second largest root belief (key), for the MAP certificate
-  float sum = 0.0f;
-  bool first = true;
-  double sum_d = 0.0;           // LSE64: sum of exp(belief - mref)
-  float mref = -INFINITY;       //        the largest belief so far
 
   // the loads of slice r + 1 are issued before slice r is processed (its
   // stores could alias them as far as the compiler knows)
-  float m[KC], u;
+  float m[KC], u = 0.0f;
   auto load = [&](int r, float (&mm)[KC], float &uu) {
     const int e = r * HW + pc, em = r * HPm + pcm;
 #pragma unroll
     for (int k = 0; k < KC; ++k) mm[k] = k < K ? cptr(b, J.msg[k])[em] : 0.0f;
     uu = un[e];
   };
-  load(0, m, u);
-  for (int r = 0; r < R; ++r) {
+  if (r0 < r1) load(r0, m, u);
+  for (int r = r0; r < r1; ++r) {
     float mn[KC], un_next;
-    load(r + 1 < R ? r + 1 : r, mn, un_next);
+    load(r + 1 < r1 ? r + 1 : r, mn, un_next);
     const int e = r * HW + pix;
     const float uu = masked(J.mask, r, x, W) ? kLogZero : u;
     // root belief: messages in joint order (:637), then the unary (:652-654)
@@ -1076,10 +1105,8 @@ __device__ __forceinline__ void root_pixels(const Bases &b, const RootJob &J, in
     for (int k = 0; k < KC; ++k)
       if (k < K) bel = bel + m[k];
     if (J.add_unary) bel = bel + uu;
-    // the root's rows are written whole by consecutive lanes: its stores
-    // stream past the caches (nontemporal), 10 % faster than cached stores
     if (ok) {
-      __builtin_nontemporal_store(bel, marg + e);
+      marg[e] = bel;
       const unsigned long long ak = amax_key(bel, (unsigned)e);
       const unsigned kv = (unsigned)(ak >> 32), kb = (unsigned)(amax >> 32);
       second = kv > kb ? kb : max(second, kv);
@@ -1096,57 +1123,75 @@ __device__ __forceinline__ void root_pixels(const Bases &b, const RootJob &J, in
           if (k < K && k != i) fr = fr + m[k];
         fr = fr + uu;
         if (ok) {
-          __builtin_nontemporal_store(fr, mptr(b, J.fr[i]) + e);
+          mptr(b, J.fr[i])[e] = fr;
           kmax[i] = max(kmax[i], f2key(fr));
         }
       }
     }
-    // root posterior over the valid rotations (:713-726)
-    if ((J.valid_rot >> r) & 1ull) {
-      if (LSE64) {
-        if (bel > mref) {
-          sum_d *= (double)__builtin_amdgcn_exp2f((mref - bel) * kLog2eF);
-          mref = bel;
-        }
-        sum_d += (double)__builtin_amdgcn_exp2f((bel - mref) * kLog2eF);
-      } else {
-        const float ev = expf(bel);
-        sum = first ? ev : sum + ev;
-        first = false;
-      }
-    }
+    if (posts) bels[r * (64 * kRootTiles) + tile * 64 + lane] = LSE64 ? bel : expf(bel);
 #pragma unroll
     for (int k = 0; k < KC; ++k) m[k] = mn[k];
     u = un_next;
   }
-  if (ok && J.root_post.buf >= 0 && b.root)
-    mptr(b, J.root_post)[pix] = LSE64 ? (sum_d > 0.0 ? log0((float)sum_d) + mref : kLogZero) : log0(sum);
 
-  const int lane = threadIdx.x & 63;
-  if (b.top2_keys) top2_flush(b.top2_keys + J.map_slot, (unsigned)(amax >> 32), second, lane);
-  amax = wave_max_u64(amax);
-  if (lane == 0 && amax) atomicMax(b.map_keys + J.map_slot, amax);
+  // the keys, as block_raise does it, the children's by as many lanes at once
+  unsigned *rk = reinterpret_cast<unsigned *>(red + kRootWaves * kRootTiles);  // [waves][KC]
+  KeyPart part;
+  if (b.top2_keys) part.second = wave_second((unsigned)(amax >> 32), second);
+  part.amax = wave_max_u64(amax);
 #pragma unroll
   for (int k = 0; k < KC; ++k) {
     if (k < K) {
-      unsigned v = wave_max_u32(kmax[k]);
-      if (lane == 0 && v) atomicMax(b.max_keys + J.fr_key[k], v);
+      const unsigned v = wave_max_u32(kmax[k]);
+      if (lane == 0) rk[wv * KC + k] = v;
     }
   }
+  block_raise(red, part, nullptr, b.map_keys + J.map_slot, b.top2_keys ? b.top2_keys + J.map_slot : nullptr);
+  if (wv == 1 && lane < K) {
+    unsigned v = 0u;
+    for (int w = 0; w < kRootWaves * kRootTiles; ++w) v = max(v, rk[w * KC + lane]);
+    if (v) atomicMax(b.max_keys + J.fr_key[lane], v);
+  }
+
+  // root posterior over the valid rotations in ascending order (:713-726)
+  if (!posts || wave != 0 || !ok) return;
+  float out;
+  if (LSE64) {
+    double sum = 0.0;  // of exp(belief - mref)
+    float mref = -INFINITY;  // the largest belief so far
+    for (int r = 0; r < R; ++r) {
+      if (!((J.valid_rot >> r) & 1ull)) continue;
+      const float bel = bels[r * (64 * kRootTiles) + tile * 64 + lane];
+      if (bel > mref) {
+        sum *= (double)__builtin_amdgcn_exp2f((mref - bel) * kLog2eF);
+        mref = bel;
+      }
+      sum += (double)__builtin_amdgcn_exp2f((bel - mref) * kLog2eF);
+    }
+    out = sum > 0.0 ? log0((float)sum) + mref : kLogZero;
+  } else {
+    float sum = 0.0f;
+    for (int r = 0; r < R; ++r)
+      if ((J.valid_rot >> r) & 1ull) sum += bels[r * (64 * kRootTiles) + tile * 64 + lane];
+    out = log0(sum);
+  }
+  mptr(b, J.root_post)[pix] = out;
 }
 
 // one instantiation per child count, chosen on the host: the variant for a
-// small tree then holds only its own K message registers (46 VGPRs for K = 5,
+// small tree then holds only its own K message registers (40 VGPRs for K = 5,
 // 8 waves per SIMD), not those of the widest tree
 template <int KC, bool LSE64>
-__global__ __launch_bounds__(256) void k_root(Bases b, const RootJob *__restrict__ jobs, int R) {
+__global__ __launch_bounds__(64 * kRootWaves * kRootTiles) void k_root(Bases b, const RootJob *__restrict__ jobs, int R) {
+  extern __shared__ float4 lds4[];  // [R][64]: beliefs (FP32 sum: their exponentials)
   unsigned bx, by;
   xcd_block(bx, by);
   const RootJob &J = jobs[by];
   if (skip_inst(b, J.inst)) return;
-  const int pix0 = (int)bx * blockDim.x;
+  const int pix0 = (int)bx * 64 * kRootTiles;
   if (pix0 >= J.H * J.W) return;
-  root_pixels<KC, LSE64>(b, J, R, pix0);
+  uint4 *red = reinterpret_cast<uint4 *>(lds4 + 16 * kRootTiles * R);
+  root_pixels<KC, LSE64>(b, J, R, pix0, red, reinterpret_cast<float *>(lds4));
 }
 
 // ------------------------------------------------------------ k_map_decode
@@ -1389,16 +1434,18 @@ hipError_t launch_colpass(const Bases &b, const MsgJob *jobs, int n_jobs, const 
 // root without children and counts above 8 take the variant that reads J.K
 template <bool LSE64>
 static void launch_root_k(const Bases &b, const RootJob *jobs, int k, int R, dim3 grid, dim3 blk, hipStream_t s) {
+  const int waves = kRootWaves * kRootTiles;
+  const size_t lds = sizeof(float) * 64 * kRootTiles * R + waves * (sizeof(uint4) + sizeof(unsigned) * kMaxRootChildren);
   switch (k) {
-    case 1: hipLaunchKernelGGL((k_root<1, LSE64>), grid, blk, 0, s, b, jobs, R); break;
-    case 2: hipLaunchKernelGGL((k_root<2, LSE64>), grid, blk, 0, s, b, jobs, R); break;
-    case 3: hipLaunchKernelGGL((k_root<3, LSE64>), grid, blk, 0, s, b, jobs, R); break;
-    case 4: hipLaunchKernelGGL((k_root<4, LSE64>), grid, blk, 0, s, b, jobs, R); break;
-    case 5: hipLaunchKernelGGL((k_root<5, LSE64>), grid, blk, 0, s, b, jobs, R); break;
-    case 6: hipLaunchKernelGGL((k_root<6, LSE64>), grid, blk, 0, s, b, jobs, R); break;
-    case 7: hipLaunchKernelGGL((k_root<7, LSE64>), grid, blk, 0, s, b, jobs, R); break;
-    case 8: hipLaunchKernelGGL((k_root<8, LSE64>), grid, blk, 0, s, b, jobs, R); break;
-    default: hipLaunchKernelGGL((k_root<kMaxRootChildren, LSE64>), grid, blk, 0, s, b, jobs, R); break;
+    case 1: hipLaunchKernelGGL((k_root<1, LSE64>), grid, blk, lds, s, b, jobs, R); break;
+    case 2: hipLaunchKernelGGL((k_root<2, LSE64>), grid, blk, lds, s, b, jobs, R); break;
+    case 3: hipLaunchKernelGGL((k_root<3, LSE64>), grid, blk, lds, s, b, jobs, R); break;
+    case 4: hipLaunchKernelGGL((k_root<4, LSE64>), grid, blk, lds, s, b, jobs, R); break;
+    case 5: hipLaunchKernelGGL((k_root<5, LSE64>), grid, blk, lds, s, b, jobs, R); break;
+    case 6: hipLaunchKernelGGL((k_root<6, LSE64>), grid, blk, lds, s, b, jobs, R); break;
+    case 7: hipLaunchKernelGGL((k_root<7, LSE64>), grid, blk, lds, s, b, jobs, R); break;
+    case 8: hipLaunchKernelGGL((k_root<8, LSE64>), grid, blk, lds, s, b, jobs, R); break;
+    default: hipLaunchKernelGGL((k_root<kMaxRootChildren, LSE64>), grid, blk, lds, s, b, jobs, R); break;
   }
 }
 
@@ -1406,8 +1453,8 @@ hipError_t launch_root(const Bases &b, const RootJob *jobs, int n_jobs, int k, i
                        hipStream_t s) {
   if (n_jobs <= 0) return hipSuccess;
   if (k < 0 || k > kMaxRootChildren) return hipErrorInvalidValue;
-  dim3 grid((max_hw + 255) / 256, n_jobs);
-  const dim3 blk(256);
+  dim3 grid((max_hw + 64 * kRootTiles - 1) / (64 * kRootTiles), n_jobs);
+  const dim3 blk(64 * kRootWaves * kRootTiles);
   if (lse64)
     launch_root_k<true>(b, jobs, k, R, grid, blk, s);
   else

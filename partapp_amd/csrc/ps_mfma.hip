@@ -822,7 +822,7 @@ __device__ __forceinline__ void colpass_mfma_strip(const Bases &b, const MsgJob 
       __syncthreads();
     }
   }
-  acc.flush(b, J, (long long)r * H * pa, lane);
+  acc.flush(b, J, (long long)r * H * pa, lds);
 }
 
 // ---------------------------------------- column pass on an fp16 row-pass output
@@ -1055,7 +1055,7 @@ __device__ __forceinline__ void colpass_f16_strip(const Bases &b, const MsgJob &
       __syncthreads();
     }
   }
-  acc.flush(b, J, (long long)r * H * pa, lane);
+  acc.flush(b, J, (long long)r * H * pa, lds);
 }
 
 // HI: the highest epilogue kind among the launch's jobs.  The kernel holds

@@ -360,7 +360,8 @@ __global__ __launch_bounds__(kOdThreads) void k_od_back(Bases b, const MsgJob *_
                 msg, pu[i], pb[i], da);
     }
   }
-  dst_flush(b, J, dst2 != nullptr, da, lane);
+  __shared__ uint4 red[4];
+  dst_flush(b, J, dst2 != nullptr, da, red);
 }
 
 // ------------------------------------------------------------ host launcher
