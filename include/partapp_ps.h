@@ -161,8 +161,9 @@ enum {
 };
 int ps_plan_set_method(ps_plan *plan, int method);
 /* Launch-shape knobs for an autotuner (results do not depend on them):
- *   PS_TUNE_MFMA_ROWS        output rows per block of the BF16 x pass (1..64,
- *                            default 4);
+ *   PS_TUNE_MFMA_ROWS        output rows per block of the BF16 x pass (1..64;
+ *                            by default 4, or fewer where that leaves CUs
+ *                            idle);
  *   PS_TUNE_FP32_ROW_THREADS threads per block of the FP32 row pass (a
  *                            multiple of 64 up to 512; 0 = one per column,
  *                            the default);

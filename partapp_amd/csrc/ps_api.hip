@@ -42,8 +42,8 @@ hipError_t launch_rowpass(const Bases &b, const MsgJob *jobs, int n_jobs, const 
 size_t colpass_lds_bytes(int ky, int rows);
 size_t colpass4_lds_bytes(int ky);
 hipError_t launch_colpass(const Bases &b, const MsgJob *jobs, int n_jobs, const float *taps, const int *shifts,
-                          int R, int epi_hi, int max_w, size_t lds_bytes_16, size_t lds4_bytes_16, hipStream_t s,
-                          int rows, bool split);
+                          int R, int epi_hi, int max_h, int max_w, size_t lds_bytes_16, size_t lds4_bytes_16,
+                          hipStream_t s, int rows, bool split);
 void od_extent(OdExtent &e, int R, const MsgJob &j);
 hipError_t od_set_lds_limit(const OdExtent &ext);
 hipError_t launch_offdiag(const Bases &b, const MsgJob *jobs, int n_jobs, const float *taps, const int *shifts, int R,
@@ -58,8 +58,8 @@ hipError_t launch_rowpass_mfma(const Bases &b, const MsgJob *jobs, int n_jobs, c
                                const uint4 *frags, int R, int terms, int rows, int max_h, int max_w,
                                size_t lds_bytes, bool leaf, hipStream_t s);
 hipError_t launch_colpass_mfma(const Bases &b, const MsgJob *jobs, int n_jobs, const uint4 *frags, const int *shifts,
-                               int R, int terms, bool t16, int epi_hi, int max_w, size_t lds_bytes, bool leaf,
-                               hipStream_t s);
+                               int R, int terms, bool t16, int epi_hi, int max_h, int max_w, size_t lds_bytes,
+                               bool leaf, hipStream_t s);
 hipError_t launch_map_decode(const Bases &b, const MapJob *jobs, int n, ps_map *out, hipStream_t s);
 }  // namespace ps
 
@@ -178,7 +178,7 @@ struct ps_plan {
   size_t frag_units = 0;
   int terms = 0;      // x pass: 0 FP32, else the BF16 Toeplitz terms (1, 2, 3)
   int col_terms = 0;  // y pass
-  int mfma_rows = 4;  // output rows per block of the BF16 x pass (tunable)
+  int mfma_rows = 0;  // output rows per block of the BF16 x pass (tunable; 0: by the launch's size)
   float *scratch = nullptr;
   size_t scratch_elems = 0;
   unsigned *keys = nullptr;
@@ -818,9 +818,9 @@ extern "C" int ps_plan_create(const ps_model *model, const ps_instance *instance
   size_t o_taps = align(o_maps + B.maps.size() * sizeof(MapJob));
   size_t o_shifts = align(o_taps + B.taps.size() * sizeof(float));
   size_t o_keys = align(o_shifts + B.shifts.size() * sizeof(int));
-  size_t o_mkeys = align(o_keys + (size_t)pl->n_keys * sizeof(unsigned));
-  size_t o_top2 = align(o_mkeys + (size_t)pl->n_map * sizeof(unsigned long long));
-  size_t o_flags = align(o_top2 + (size_t)pl->n_map * sizeof(unsigned long long));
+  size_t o_mkeys = align(o_keys + (size_t)pl->n_keys * kMaxKeyStride * sizeof(unsigned));
+  size_t o_top2 = align(o_mkeys + (size_t)pl->n_map * kMapKeyStride * sizeof(unsigned long long));
+  size_t o_flags = align(o_top2 + (size_t)pl->n_map * kMapKeyStride * sizeof(unsigned long long));
   size_t o_nfb = align(o_flags + (size_t)n_instances * sizeof(unsigned));
   size_t total = align(o_nfb + (size_t)n_instances * sizeof(unsigned));
   hipError_t e = pool_get(&pl->tables, total);
@@ -1205,10 +1205,11 @@ static hipError_t sweep(ps_plan *pl, const Bases &b, int terms, int col_terms, p
       const long ev2 = profile_begin(pp, 3, s);
       if (mf)
         e = launch_colpass_mfma(b, jobs + c.start, c.count, pl->frags, pl->shifts, pl->R, col_terms, terms != 3,
-                                c.epi_hi, c.max_w, terms != 3 ? L.mfma_col16_lds : L.mfma_col_lds[tc], c.leaf, s);
+                                c.epi_hi, c.max_h, c.max_w, terms != 3 ? L.mfma_col16_lds : L.mfma_col_lds[tc], c.leaf,
+                                s);
       else
-        e = launch_colpass(b, jobs + c.start, c.count, pl->taps, pl->shifts, pl->R, c.epi_hi, c.max_w, L.col_lds,
-                           L.col_lds4, s, c.col_rows, c.split);
+        e = launch_colpass(b, jobs + c.start, c.count, pl->taps, pl->shifts, pl->R, c.epi_hi, c.max_h, c.max_w,
+                           L.col_lds, L.col_lds4, s, c.col_rows, c.split);
       profile_end(pp, ev2, s);
     }
     // the column pass class also times the eigenbasis stages
@@ -1324,7 +1325,7 @@ static hipError_t sweep_subset(ps_plan *pl, const Bases &b, ps_map *map_dev, hip
     for (size_t k = 0; k < L.col_classes.size() && e == hipSuccess; ++k) {
       const WidthClass &c = L.col_classes[k];
       const long ev2 = profile_begin(pp, 3, s);
-      e = launch_colpass(b, jobs + ls.col[k].start, ls.col[k].count, pl->taps, pl->shifts, pl->R, c.epi_hi, c.max_w,
+      e = launch_colpass(b, jobs + ls.col[k].start, ls.col[k].count, pl->taps, pl->shifts, pl->R, c.epi_hi, c.max_h, c.max_w,
                          L.col_lds, L.col_lds4, s, c.col_rows, c.split);
       profile_end(pp, ev2, s);
     }
@@ -1628,7 +1629,7 @@ int message_enqueue(const MessageSetup &ms, char *mem, const float *child_dev, f
     if (ms.od)
       e = launch_offdiag(b, jd, 1, td, sd, ms.R, ms.od_ext, s);
     else
-      e = launch_colpass(b, jd, 1, td, sd, ms.R, ms.epi, ms.W, ms.col_lds, ms.col_lds4, s, 0, ms.split);
+      e = launch_colpass(b, jd, 1, td, sd, ms.R, ms.epi, ms.H, ms.W, ms.col_lds, ms.col_lds4, s, 0, ms.split);
   }
   // the block may be reused right after: the call is synchronous
   if (e == hipSuccess) e = hipStreamSynchronize(s);

@@ -40,6 +40,14 @@ __device__ __forceinline__ void xcd_block(unsigned &bx, unsigned &by) {
   bx = l - by * gridDim.x;
 }
 
+// A column pass's rows [ya, yb), a part (gridDim.z of them) of a strip that
+// walks tiles of th rows.
+__device__ __forceinline__ void col_part(int H, int th, int &ya, int &yb) {
+  const int rows = ((H + th - 1) / th + (int)gridDim.z - 1) / (int)gridDim.z * th;
+  ya = (int)blockIdx.z * rows;
+  yb = min(H, ya + rows);
+}
+
 __device__ __forceinline__ unsigned wave_max_u32(unsigned v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v = max(v, (unsigned)__shfl_xor((int)v, o, 64));
@@ -58,11 +66,21 @@ __device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v)
 // that run): every block of its jobs exits at once.
 __device__ __forceinline__ bool skip_inst(const Bases &b, int inst) { return b.active && b.active[inst] == 0u; }
 
+__device__ __forceinline__ unsigned *max_key(const Bases &b, int k) { return b.max_keys + (size_t)k * kMaxKeyStride; }
+__device__ __forceinline__ unsigned long long *map_key(const Bases &b, int k) {
+  return b.map_keys + (size_t)k * kMapKeyStride;
+}
+// the MAP certificate's, or null where there is none
+__device__ __forceinline__ unsigned long long *top2_key(const Bases &b, int k) {
+  return b.top2_keys ? b.top2_keys + (size_t)k * kMapKeyStride : nullptr;
+}
+
 // A block's result for the keys it feeds: the waves' parts, each merged over
 // its lanes, meet in LDS and one thread raises the keys.  Atomics on one cache
-// line queue up at 4 to 13 ns each, and all keys of an instance share a line: a
-// wave each, the leaf maxima of an image of 300x300x48 took 70 us for 17 us of
-// reading.  (Reading a key first and raising it only where it is lower queues up
+// line queue up at 4 to 13 ns each: by a wave each, all keys of an instance in one
+// line, the leaf maxima of an image of 300x300x48 took 70 us for 17 us of
+// reading (27 so, and 17 with a line per key).  (Reading a key first and
+// raising it only where it is lower queues up
 // just as much once thousands of waves are in flight, and each then waits for
 // its answer: 957 instead of 299 us for the leaf maxima of 32 images.)
 struct KeyPart {
@@ -288,9 +306,8 @@ struct Epi {
       if (b.top2_keys) p.second = wave_second(best_key, second_key);
     }
     __syncthreads();
-    block_raise(static_cast<uint4 *>(lds), p, kKey ? b.max_keys + (kDown ? J.dst2_key : J.dst_key) : nullptr,
-                kDown ? b.map_keys + J.map_slot : nullptr,
-                kDown && b.top2_keys ? b.top2_keys + J.map_slot : nullptr);
+    block_raise(static_cast<uint4 *>(lds), p, kKey ? max_key(b, kDown ? J.dst2_key : J.dst_key) : nullptr,
+                kDown ? map_key(b, J.map_slot) : nullptr, kDown ? top2_key(b, J.map_slot) : nullptr);
   }
 };
 
@@ -351,13 +368,13 @@ __device__ __forceinline__ void dst_flush(const Bases &b, const MsgJob &J, bool 
   KeyPart p;
   if (J.dst_kind == kDstUpNode) {
     p.key = wave_max_u32(a.kmax1);
-    block_raise(red, p, b.max_keys + J.dst_key, nullptr, nullptr);
+    block_raise(red, p, max_key(b, J.dst_key), nullptr, nullptr);
   } else if (J.dst_kind == kDstDown) {
     p.amax = wave_max_u64(a.amax);
     if (b.top2_keys) p.second = wave_second((unsigned)(a.amax >> 32), a.second);
     if (has_dst2) p.key = wave_max_u32(a.kmax2);
-    block_raise(red, p, has_dst2 ? b.max_keys + J.dst2_key : nullptr, b.map_keys + J.map_slot,
-                b.top2_keys ? b.top2_keys + J.map_slot : nullptr);
+    block_raise(red, p, has_dst2 ? max_key(b, J.dst2_key) : nullptr, map_key(b, J.map_slot),
+                top2_key(b, J.map_slot));
   }
 }
 

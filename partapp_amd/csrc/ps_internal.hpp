@@ -15,6 +15,11 @@ constexpr int kMaxTaps = 1000;     // multi_array_filter.hpp:243-244
 constexpr int kNoSourceRow = -(1 << 30);  // row offset of an output slice with no source slice
 constexpr int kMfmaMaxKK = 8;      // BF16 Toeplitz passes: half widths up to 47 (2k + 32 <= 8 * 16)
 
+// Keys lie a 128-byte line apart: the blocks of a launch raise them by atomics,
+// which queue up line by line.
+constexpr int kMaxKeyStride = 32;  // in unsigned
+constexpr int kMapKeyStride = 16;  // in unsigned long long
+
 // Which base pointer an offset is relative to.
 enum BufId : int { kBufUnary = 0, kBufMarginal = 1, kBufScratch = 2, kBufRoot = 3 };
 
@@ -208,5 +213,9 @@ struct MapJob {
   int inst;
   int pad0_;
 };
+
+// (ps_kernels.hip) the parts that a column pass of `blocks` strips of `tiles`
+// tiles cuts each strip into
+int col_parts(int blocks, int tiles);
 
 }  // namespace ps

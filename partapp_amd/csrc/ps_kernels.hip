@@ -45,10 +45,10 @@ namespace ps {
 __global__ void k_reset(Bases b, int n_keys, int n_map, int keys_per_inst, int map_per_inst, unsigned *flags,
                         int n_flags) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n_keys && !skip_inst(b, i / keys_per_inst)) b.max_keys[i] = 0u;
+  if (i < n_keys && !skip_inst(b, i / keys_per_inst)) *max_key(b, i) = 0u;
   if (i < n_map && !skip_inst(b, i / map_per_inst)) {
-    b.map_keys[i] = 0ull;
-    if (b.top2_keys) b.top2_keys[i] = 0ull;
+    *map_key(b, i) = 0ull;
+    if (b.top2_keys) *top2_key(b, i) = 0ull;
   }
   if (flags && i < n_flags) flags[i] = 0u;
 }
@@ -183,7 +183,7 @@ __global__ __launch_bounds__(256) void k_max(Bases b, const MaxJob *__restrict__
   }
   KeyPart p;
   p.key = wave_max_u32(km);
-  block_raise(red, p, b.max_keys + J.key, nullptr, nullptr);
+  block_raise(red, p, max_key(b, J.key), nullptr, nullptr);
 }
 
 // -------------------------------------------------------------- k_rowpass
@@ -552,7 +552,7 @@ __device__ __forceinline__ void rowpass_body(const Bases &b, const MsgJob &J, co
     zero_halo(P, RG, W, kx, g.Pw);
   }
 
-  const float M = key2f(b.max_keys[J.src_key]);
+  const float M = key2f(*max_key(b, J.src_key));
   const float negM = -M;
   // exp(LOG_ZERO - M): the warp's fill value, on the path of every other value
   const float e_fill = __builtin_amdgcn_exp2f((kLogZero + negM) * kLog2eF);
@@ -635,7 +635,7 @@ __global__ __launch_bounds__(512) void k_rowpass_any(Bases b, const MsgJob *__re
   float *P = E + R * Wa;
   zero_halo(P, R, W, kx, g.Pw);
 
-  const float M = key2f(b.max_keys[J.src_key]);
+  const float M = key2f(*max_key(b, J.src_key));
   const float negM = -M;
   const float e_fill = expf(kLogZero + negM);
   const float *src = cptr(b, J.src);
@@ -798,7 +798,8 @@ __device__ __forceinline__ void yfilter4(const float *col, int row, int n, const
 // change once along x (per lane) or y (a second segment of rows)
 template <int EPI, int ROWS, bool SPLIT, bool MFMA>
 __device__ __forceinline__ void colpass_strip(const Bases &b, const MsgJob &J, const float *__restrict__ taps,
-                                              const int *__restrict__ shifts, int R, int r, int xt, float *tile) {
+                                              const int *__restrict__ shifts, int R, int r, int xt, int ya, int yb,
+                                              float *tile) {
   constexpr int kColRows = ROWS;
   constexpr int kColTileY = kColRows * kColWaves;
   constexpr bool kNeedU = Epi<EPI>::kNeedU;
@@ -835,7 +836,7 @@ __device__ __forceinline__ void colpass_strip(const Bases &b, const MsgJob &J, c
     if (threadIdx.x == 0) *bad = 0u;
     __syncthreads();
   }
-  const float M = key2f(b.max_keys[J.src_key]);
+  const float M = key2f(*max_key(b, J.src_key));
   // row pitches: pa of dst (and of the unary a marginal adds), pb of the
   // grids at the other pitch (EpiPitch)
   const int pa = J.dst.pitch, pb = epi_pitch_b<EPI>(J);
@@ -853,8 +854,8 @@ __device__ __forceinline__ void colpass_strip(const Bases &b, const MsgJob &J, c
   auto src_raw = [&](int row) -> float { return Tc[(long long)min(max(row, 0), H - 1) * tp]; };
   auto src_ok = [&](int row) -> bool { return lcol_ok && row >= 0 && row < H; };
 
-  // The output rows run in segments of one inverse row offset oy: [0, ybrk)
-  // and, for a split warp, [ybrk, H).  Within a segment, tile t holds source
+  // The output rows [ya, yb) run in segments of one inverse row offset oy: up
+  // to ybrk and, for a split warp, from it on.  Within a segment, tile t holds source
   // rows s_t + [0, nrows), s_t = ylo + 64 t + oy - ky.  Tile t+1 shares rows
   // [64, nrows) of tile t (moved to [0, Lp) in LDS) and needs 64 new rows,
   // fetched into registers while tile t is filtered.
@@ -865,7 +866,7 @@ __device__ __forceinline__ void colpass_strip(const Bases &b, const MsgJob &J, c
   // lines save)
   unsigned Wb = (unsigned)pa * 4u, Wb2 = (unsigned)pb * 4u;
   for (int seg = 0; seg < (SPLIT ? 2 : 1); ++seg) {
-    const int ylo = seg == 0 ? 0 : ybrk, yhi = seg == 0 ? ybrk : H;
+    const int ylo = seg == 0 ? ya : max(ya, ybrk), yhi = seg == 0 ? min(yb, ybrk) : yb;
     if (ylo >= yhi) continue;
     const int oy = seg == 0 ? oy0 : oy0 + ystep;
     if (seg) __syncthreads();  // every wave is done with the first segment's tile
@@ -1019,17 +1020,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
   const int r = (int)bx / xtiles;
   const int xt = (int)bx - r * xtiles;
   if (xt * kColTileX >= J.W) return;
+  int ya, yb;
+  col_part(J.H, kColWaves * ROWS, ya, yb);
+  if (ya >= yb) return;
   const int kind = epi_kind(J);
   if (HI == kEpiUpRoot || kind == kEpiUpRoot)
-    colpass_strip<kEpiUpRoot, ROWS, SPLIT, MFMA>(b, J, taps, shifts, R, r, xt, tile);
+    colpass_strip<kEpiUpRoot, ROWS, SPLIT, MFMA>(b, J, taps, shifts, R, r, xt, ya, yb, tile);
   else if (HI == kEpiUpNode || kind == kEpiUpNode)
-    colpass_strip<kEpiUpNode, ROWS, SPLIT, MFMA>(b, J, taps, shifts, R, r, xt, tile);
+    colpass_strip<kEpiUpNode, ROWS, SPLIT, MFMA>(b, J, taps, shifts, R, r, xt, ya, yb, tile);
   else if (HI == kEpiUpNodeU || kind == kEpiUpNodeU)
-    colpass_strip<kEpiUpNodeU, ROWS, SPLIT, MFMA>(b, J, taps, shifts, R, r, xt, tile);
+    colpass_strip<kEpiUpNodeU, ROWS, SPLIT, MFMA>(b, J, taps, shifts, R, r, xt, ya, yb, tile);
   else if (HI == kEpiDownLeaf || kind == kEpiDownLeaf)
-    colpass_strip<kEpiDownLeaf, ROWS, SPLIT, MFMA>(b, J, taps, shifts, R, r, xt, tile);
+    colpass_strip<kEpiDownLeaf, ROWS, SPLIT, MFMA>(b, J, taps, shifts, R, r, xt, ya, yb, tile);
   else
-    colpass_strip<kEpiDownMid, ROWS, SPLIT, MFMA>(b, J, taps, shifts, R, r, xt, tile);
+    colpass_strip<kEpiDownMid, ROWS, SPLIT, MFMA>(b, J, taps, shifts, R, r, xt, ya, yb, tile);
 }
 
 // ----------------------------------------------------------------- k_root
@@ -1146,11 +1150,11 @@ __device__ __forceinline__ void root_pixels(const Bases &b, const RootJob &J, in
       if (lane == 0) rk[wv * KC + k] = v;
     }
   }
-  block_raise(red, part, nullptr, b.map_keys + J.map_slot, b.top2_keys ? b.top2_keys + J.map_slot : nullptr);
+  block_raise(red, part, nullptr, map_key(b, J.map_slot), top2_key(b, J.map_slot));
   if (wv == 1 && lane < K) {
     unsigned v = 0u;
     for (int w = 0; w < kRootWaves * kRootTiles; ++w) v = max(v, rk[w * KC + lane]);
-    if (v) atomicMax(b.max_keys + J.fr_key[lane], v);
+    if (v) atomicMax(max_key(b, J.fr_key[lane]), v);
   }
 
   // root posterior over the valid rotations in ascending order (:713-726)
@@ -1201,7 +1205,7 @@ __global__ void k_map_decode(Bases b, const MapJob *__restrict__ jobs, int n, ps
   if (i >= n) return;
   const MapJob J = jobs[i];
   if (skip_inst(b, J.inst)) return;
-  const unsigned long long k = b.map_keys[J.slot];
+  const unsigned long long k = *map_key(b, J.slot);
   ps_map m;
   if (k == 0ull) {
     m.rotidx = -1;
@@ -1230,7 +1234,7 @@ __global__ void k_certify(const unsigned long long *__restrict__ top2, int n_map
                           unsigned *flags) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n_map) return;
-  const unsigned long long t = top2[i];
+  const unsigned long long t = top2[(size_t)i * kMapKeyStride];
   const unsigned k1 = (unsigned)(t >> 32), k2 = (unsigned)t;
   const float v1 = k1 ? key2f(k1) : -INFINITY;
   const float v2 = k2 ? key2f(k2) : -INFINITY;
@@ -1401,6 +1405,16 @@ static void launch_colpass_rows(int epi_hi, dim3 grid, size_t lds_bytes, hipStre
   }
 }
 
+// A strip walks its tiles one after another, a few us each, most of it waiting.
+// A launch of few strips cuts them into parts, each its own block, as long as
+// all blocks fit the chip at once, 4 per CU; a part fills its own ring, whose
+// extra rows cost more than the waits once the chip is full (300x300x48, 960
+// strips: 94 instead of 86 us in two parts).  us per launch, one part / by this
+// rule: 22.0 / 17.3, 21.4 / 17.8, 19.7 / 16.0 and 18.1 / 14.9 (FP32, 112x128x24,
+// 192 or 240 strips), 21.1 / 17.4, 19.5 / 16.2, 18.2 / 16.0 and 15.7 / 13.1
+// (fp16, 160x160x24, 288 or 360 strips), 10.8 / 8.6 (one message of 41x57x24).
+int col_parts(int blocks, int tiles) { return std::max(1, std::min(tiles, 1024 / blocks)); }
+
 // epi_hi: the highest destination kind (EpiKind) among the jobs; rows:
 // output rows per lane (8 or 16; 0 = the default); lds_bytes_16, lds4_bytes_16:
 // the LDS of the 16-row tile for the jobs' widest y filter, without and with
@@ -1409,13 +1423,14 @@ static void launch_colpass_rows(int epi_hi, dim3 grid, size_t lds_bytes, hipStre
 // (split: some job's warp changes its offset along an axis; those launches
 // take 8 rows per lane)
 hipError_t launch_colpass(const Bases &b, const MsgJob *jobs, int n_jobs, const float *taps, const int *shifts,
-                          int R, int epi_hi, int max_w, size_t lds_bytes_16, size_t lds4_bytes_16, hipStream_t s,
-                          int rows, bool split) {
+                          int R, int epi_hi, int max_h, int max_w, size_t lds_bytes_16, size_t lds4_bytes_16,
+                          hipStream_t s, int rows, bool split) {
   if (n_jobs <= 0) return hipSuccess;
   if (rows == 0 || split) rows = kColRowsDefault;
   if (epi_hi < kEpiUpRoot || epi_hi > kEpiDownMid || (rows != 8 && rows != 16)) return hipErrorInvalidValue;
   const int xtiles = (max_w + kColTileX - 1) / kColTileX;
-  dim3 grid(R * xtiles, n_jobs);
+  const int tile_y = kColWaves * rows;
+  dim3 grid(R * xtiles, n_jobs, col_parts(R * xtiles * n_jobs, (max_h + tile_y - 1) / tile_y));
   const size_t less = sizeof(float) * kColWaves * 8 * kColTileX;
   if (lds4_bytes_16 == 0 && split)
     launch_colpass_rows<8, true, false>(epi_hi, grid, lds_bytes_16 - less, s, b, jobs, taps, shifts, R, xtiles);

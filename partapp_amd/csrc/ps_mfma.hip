@@ -277,7 +277,7 @@ __device__ __forceinline__ void rowpass_mfma_body(Bases b, const MsgJob *__restr
 
   // exp(b - M) = 2^(b log2 e - M log2 e)
   constexpr float kLog2e = 1.4426950408889634f;
-  const float M = J.src_kind == kSrcGrid || !T16 ? key2f(b.max_keys[J.src_key]) : 0.0f;
+  const float M = J.src_kind == kSrcGrid || !T16 ? key2f(*max_key(b, J.src_key)) : 0.0f;
   const float *src = cptr(b, J.src);
   const bool zero_src = J.src_kind == kSrcZero;
   const UnaryMask mk = J.src_mask;
@@ -630,7 +630,7 @@ __device__ __forceinline__ void colpass_mfma_strip(const Bases &b, const MsgJob 
   if (threadIdx.x < 64) cmax[threadIdx.x] = 0u;
   const int ox = shifts[J.shifts + 2 * R + r];
   const int oy = shifts[J.shifts + 3 * R + r];
-  const float M = key2f(b.max_keys[J.src_key]);
+  const float M = key2f(*max_key(b, J.src_key));
   // row pitches: pa of dst (and of the unary a marginal adds), pitch_b of
   // the grids at the other pitch (Epi::kSide)
   const int pa = J.dst.pitch, pitch_b = epi_pitch_b<EPI>(J);
@@ -841,7 +841,8 @@ __device__ __forceinline__ void colpass_mfma_strip(const Bases &b, const MsgJob 
 // The ring keeps staging every tile, so the next kept tile finds its rows.
 template <int EPI, bool PRUNE, bool RS>
 __device__ __forceinline__ void colpass_f16_strip(const Bases &b, const MsgJob &J, const uint4 *__restrict__ frags,
-                                                  const int *__restrict__ shifts, int R, int r, int xt, uint4 *lds) {
+                                                  const int *__restrict__ shifts, int R, int r, int xt, int ya, int yb,
+                                                  uint4 *lds) {
   constexpr bool kNeedU = Epi<EPI>::kNeedU;
   constexpr bool kNeedB = Epi<EPI>::kNeedB;
   const int H = J.H, W = J.W;
@@ -942,12 +943,12 @@ __device__ __forceinline__ void colpass_f16_strip(const Bases &b, const MsgJob &
 #pragma unroll
   for (int q = 0; q < kFill; ++q) {
     const int c = wave + 4 * q;
-    if (c < nrows / 16) load16(oy - ky + 16 * c, fill[q]);
+    if (c < nrows / 16) load16(ya + oy - ky + 16 * c, fill[q]);
   }
 #pragma unroll
   for (int q = 0; q < kFill; ++q) {
     const int c = wave + 4 * q;
-    if (c < nrows / 16) put16(oy - ky + 16 * c, 16 * c, fill[q]);
+    if (c < nrows / 16) put16(ya + oy - ky + 16 * c, 16 * c, fill[q]);
   }
   __syncthreads();
 
@@ -980,7 +981,7 @@ __device__ __forceinline__ void colpass_f16_strip(const Bases &b, const MsgJob &
   Epi<EPI> acc;
   int base = 0;
   const unsigned char *kp = PRUNE ? b.keep + J.keep_off + (long long)r * J.keep_ty * J.keep_tx + xt : nullptr;
-  for (int ty0 = 0; ty0 < H; ty0 += 64) {
+  for (int ty0 = ya; ty0 < yb; ty0 += 64) {
     asm volatile("" : "+s"(Wb), "+s"(Wb2), "+s"(tp));  // per-row offsets recomputed per tile, not hoisted
     const int yl = ty0 + ry + 4 * h;
     const unsigned eb0 = (unsigned)(yl * pa + xa) * 4u;
@@ -1006,7 +1007,7 @@ __device__ __forceinline__ void colpass_f16_strip(const Bases &b, const MsgJob &
         }
       }
     }
-    const bool more = ty0 + 64 < H;
+    const bool more = ty0 + 64 < yb;
     const int pre_row = ty0 + oy - ky + nrows + 16 * wave;
     h2_t pre[8];
     load16(pre_row, pre);
@@ -1074,17 +1075,20 @@ __global__ __launch_bounds__(256) void k_colpass_f16(Bases b, const MsgJob *__re
   const int r = (int)bx / xtiles;
   const int xt = (int)bx - r * xtiles;
   if (xt * 64 >= J.W) return;
+  int ya, yb;
+  col_part(J.H, 64, ya, yb);
+  if (ya >= yb) return;
   const int kind = epi_kind(J);
   if (HI == kEpiUpRoot || kind == kEpiUpRoot)
-    colpass_f16_strip<kEpiUpRoot, PRUNE, RS>(b, J, frags, shifts, R, r, xt, lds);
+    colpass_f16_strip<kEpiUpRoot, PRUNE, RS>(b, J, frags, shifts, R, r, xt, ya, yb, lds);
   else if (HI == kEpiUpNode || kind == kEpiUpNode)
-    colpass_f16_strip<kEpiUpNode, PRUNE, RS>(b, J, frags, shifts, R, r, xt, lds);
+    colpass_f16_strip<kEpiUpNode, PRUNE, RS>(b, J, frags, shifts, R, r, xt, ya, yb, lds);
   else if (HI == kEpiUpNodeU || kind == kEpiUpNodeU)
-    colpass_f16_strip<kEpiUpNodeU, PRUNE, RS>(b, J, frags, shifts, R, r, xt, lds);
+    colpass_f16_strip<kEpiUpNodeU, PRUNE, RS>(b, J, frags, shifts, R, r, xt, ya, yb, lds);
   else if (HI == kEpiDownLeaf || kind == kEpiDownLeaf)
-    colpass_f16_strip<kEpiDownLeaf, PRUNE, RS>(b, J, frags, shifts, R, r, xt, lds);
+    colpass_f16_strip<kEpiDownLeaf, PRUNE, RS>(b, J, frags, shifts, R, r, xt, ya, yb, lds);
   else
-    colpass_f16_strip<kEpiDownMid, PRUNE, RS>(b, J, frags, shifts, R, r, xt, lds);
+    colpass_f16_strip<kEpiDownMid, PRUNE, RS>(b, J, frags, shifts, R, r, xt, ya, yb, lds);
 }
 
 template <int TERMS>
@@ -1183,7 +1187,13 @@ hipError_t launch_rowpass_mfma(const Bases &b, const MsgJob *jobs, int n_jobs, c
                                size_t lds_bytes, bool leaf, hipStream_t s) {
   if (n_jobs <= 0) return hipSuccess;
   // one lane per column: the plan only routes grids of width <= 512 here
-  if ((R != 24 && R != 48) || terms < 1 || terms > 3 || max_w > 512 || rows < 1) return hipErrorInvalidValue;
+  if ((R != 24 && R != 48) || terms < 1 || terms > 3 || max_w > 512 || rows < 0) return hipErrorInvalidValue;
+  // several rows per block share the taps and prefetch the next row; fewer of
+  // them where that leaves CUs without a block (160x160x24, 160 or 200 blocks of
+  // 4 rows: 22.2 and 19.7 us per launch of leaf and inner messages; two rows
+  // 16.5 and 14.6, one row 14.4 and 13.3)
+  if (rows == 0)
+    for (rows = 4; rows > 1 && (max_h + rows - 1) / rows * n_jobs < 512;) rows >>= 1;
   dim3 grid((max_h + rows - 1) / rows, n_jobs);
   const int nt = std::min(512, std::max(64, (max_w + 63) / 64 * 64));
   if (terms == 3) {
@@ -1222,13 +1232,13 @@ static void launch_colpass_f16(int epi_hi, dim3 grid, size_t lds_bytes, hipStrea
 // epi_hi: the highest epilogue kind (EpiKind) among the jobs; leaf: the jobs
 // include a leaf's message (fp16 rows with their own exponents)
 hipError_t launch_colpass_mfma(const Bases &b, const MsgJob *jobs, int n_jobs, const uint4 *frags, const int *shifts,
-                               int R, int terms, bool t16, int epi_hi, int max_w, size_t lds_bytes, bool leaf,
-                               hipStream_t s) {
+                               int R, int terms, bool t16, int epi_hi, int max_h, int max_w, size_t lds_bytes,
+                               bool leaf, hipStream_t s) {
   if (n_jobs <= 0) return hipSuccess;
   if (terms < 1 || terms > 3 || (!t16 && terms != 3) || epi_hi < kEpiUpRoot || epi_hi > kEpiDownMid)
     return hipErrorInvalidValue;
   const int xtiles = (max_w + 63) / 64;
-  dim3 grid(R * xtiles, n_jobs);
+  dim3 grid(R * xtiles, n_jobs, t16 ? col_parts(R * xtiles * n_jobs, (max_h + 63) / 64) : 1);
   if (t16) {  // fp16 operands: exact data, split taps, whatever the method's terms
     if (b.keep) {  // a pruned execution
       if (leaf)

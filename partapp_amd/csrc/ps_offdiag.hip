@@ -318,7 +318,7 @@ __global__ __launch_bounds__(kOdThreads) void k_od_back(Bases b, const MsgJob *_
   if (J.split && x >= sh[12 * R + r]) ox += sh[13 * R + r];
   const int ybrk = J.split ? sh[14 * R + r] : H, ystep = J.split ? sh[15 * R + r] : 0;
   const int xs = x + ox;
-  const float M = key2f(b.max_keys[J.src_key]);
+  const float M = key2f(*max_key(b, J.src_key));
   float *dst = mptr(b, J.dst);
   const float *dun = J.dst_unary.buf >= 0 ? cptr(b, J.dst_unary) : nullptr;
   float *dst2 = J.dst2.buf >= 0 ? mptr(b, J.dst2) : nullptr;
