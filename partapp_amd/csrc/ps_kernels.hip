@@ -197,33 +197,40 @@ __global__ __launch_bounds__(256) void k_max(Bases b, const MaxJob *__restrict__
 // two halves 9.7 instead of 8.8 ms per 32 x 300x300x24 sweep)
 __host__ __device__ constexpr int row_groups(int R) { return R >= 48 ? 2 : 1; }
 
-// LDS of the row pass with the x filter on the MFMA: P[position][RG + 1], the
-// RG slices of a column next to each other (written and read at immediate
-// offsets; an odd pitch, so 16 positions 4 apart are 16 different banks), kx
-// zeros before the row and the last tile's window behind it; the tap operand and
-// the flag follow.  24 slices go through at once (12 at a time halve the LDS
-// and cost a second pass over the rotation filter's inputs: 855 against 765 us
-// per launch of 96 messages of 300x300x24), 48 in four groups of 12 (24 beside
-// the 48 values held from group to group spill).
+// LDS of the row pass with the x filter on the MFMA: P[position][pitch], the RG
+// slices of a column next to each other (written and read at immediate
+// offsets), kx zeros before the row and the last column's window behind it; the
+// tap operand and the flag follow.  24 slices go through at once (12 at a time
+// halve the LDS and cost a second pass over the rotation filter's inputs: 855
+// against 765 us per launch of 96 messages of 300x300x24) and are read in pairs
+// (half the LDS instructions: 759 -> 733 us there, 153 -> 140 on uneven grids);
+// 48 go in four groups of 12 (24 beside the 48 values held from group to group
+// spill; three groups of 16, read four at a time, 77.6 against 74.5 us per launch
+// of one 300x300 image).  The pitches spread the 16 positions x 4 slices of a
+// read over all banks.
 __host__ __device__ constexpr int row4_slices(int R) { return R == 24 ? 24 : 12; }
-__host__ __device__ __forceinline__ int row4_len(int W, int k) { return ((W + 63) & ~63) + 4 * tap4_chunks(k); }
+__host__ __device__ constexpr bool row4_pairs(int rg) { return rg % 8 == 0; }
+__host__ __device__ constexpr int row4_pitch(int rg) { return row4_pairs(rg) ? rg + 2 : rg + 1; }
+__host__ __device__ __forceinline__ int row4_len(int W, int k) { return ((W + 3) & ~3) + 4 * tap4_chunks(k); }
 __host__ __device__ __forceinline__ size_t row4_floats(int rg, int W, int k) {
-  return ((size_t)row4_len(W, k) * (rg + 1) + 3) & ~(size_t)3;
+  return ((size_t)row4_len(W, k) * row4_pitch(rg) + 3) & ~(size_t)3;
 }
 __host__ __device__ __forceinline__ size_t row4_lds_bytes(int rg, int W, int k) {
   return sizeof(float) * (row4_floats(rg, W, k) + 4 * tap4_pitch(k) + 4);
 }
 
 // x filter of the RG rows of P (RG a multiple of 4), row y of T: wave w takes
-// the 64-column tiles w, w + waves, ...; lane 4 b + m reads slice 4 s + m from
-// position 4 b of the tile on, and holds after the last step, in acc[s][i],
-// slice 4 s + i at column `lane`: stores of whole lines.  One LDS read of four
-// steps' taps serves RG / 4 groups of slices.
+// the 64-column tiles w, w + waves, ...; lane 4 b + m reads slices 4 s + m (in
+// pairs: S m + s), s < S = RG / 4, from position 4 b of the tile on (past the row,
+// its last positions again), and holds after the last step, in acc[s][i], slice
+// 4 s + i (S i + s) at column `lane`: stores of whole lines.  One LDS read of
+// four steps' taps serves the S groups of slices.
 template <int RG>
 __device__ __forceinline__ void xfilter4(const float *P, const float *t4, int kx, float *T, int tp, long long plane,
                                          int y, int W) {
   static_assert(RG % 4 == 0, "rows in groups of four");
-  constexpr int S = RG / 4, Q = RG + 1;
+  constexpr int S = RG / 4, Q = row4_pitch(RG);
+  constexpr bool kPairs = row4_pairs(RG);
   const int lane = threadIdx.x & 63, m = lane & 3;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int NT = tap4_chunks(kx), tiles = (W + 63) >> 6;
@@ -231,7 +238,7 @@ __device__ __forceinline__ void xfilter4(const float *P, const float *t4, int kx
   const long long plane_b = plane * 4;
   for (int j = wave; j < tiles; j += (int)(blockDim.x >> 6)) {
     const float4 *tv = reinterpret_cast<const float4 *>(t4 + m * tap4_pitch(kx));
-    const float *d = P + (64 * j + (lane & ~3)) * Q + m;
+    const float *d = P + min(64 * j + (lane & ~3), ((W + 3) & ~3) - 4) * Q + (kPairs ? m * S : m);
     f32x4_t acc[S];
 #pragma unroll
     for (int s = 0; s < S; ++s) acc[s] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
@@ -241,7 +248,15 @@ __device__ __forceinline__ void xfilter4(const float *P, const float *t4, int kx
 #pragma unroll
       for (int k = 0; k < 4; ++k)
 #pragma unroll
-        for (int s = 0; s < S; ++s) x[k][s] = d[k * Q + 4 * s];
+        for (int s = 0; s < S; ++s) {
+          if (!kPairs) {
+            x[k][s] = d[k * Q + 4 * s];
+          } else if (s % 2 == 0) {
+            const float2 v = *reinterpret_cast<const float2 *>(d + k * Q + s);
+            x[k][s] = v.x;
+            x[k][s + 1] = v.y;
+          }
+        }
       d += 4 * Q;
 #pragma unroll
       for (int s = 0; s < S; ++s) acc[s] = mfma4(x[0][s], t.x, acc[s]);
@@ -256,12 +271,10 @@ __device__ __forceinline__ void xfilter4(const float *P, const float *t4, int kx
     if ((int)xo < tp) {
       char *o = trow;
 #pragma unroll
-      for (int s = 0; s < S; ++s)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          *reinterpret_cast<float *>(o + xo * 4u) = acc[s][i];
-          o += plane_b;
-        }
+      for (int n = 0; n < RG; ++n) {
+        *reinterpret_cast<float *>(o + xo * 4u) = kPairs ? acc[n % S][n / S] : acc[n / 4][n % 4];
+        o += plane_b;
+      }
     }
   }
 }
@@ -274,7 +287,7 @@ __device__ __forceinline__ void xfilter_plain(const float *P, int rg, const floa
   for (int i = threadIdx.x; i < rg * W; i += blockDim.x) {
     const int r = i / W, x = i - r * W;
     float a = 0.0f;
-    for (int t = 0; t < Lp; ++t) a = fmaf(P[(x + t) * (rg + 1) + r], f[t], a);
+    for (int t = 0; t < Lp; ++t) a = fmaf(P[(x + t) * row4_pitch(rg) + r], f[t], a);
     T[r * plane + (long long)y * tp + x] = a;
   }
 }
@@ -528,7 +541,7 @@ __device__ __forceinline__ void rowpass_rotate(const MsgJob &J, const float *__r
 // on) on the vector unit.  Bound by latency: the filter, the exponentials and
 // rotation filter, and the gather each take some 40% of a launch of 96
 // messages of 300x300x24 and overlap between the 4 blocks that fit a CU only
-// in part: 899 us with the filter on the vector unit, 765 now (467 without the
+// in part: 899 us with the filter on the vector unit, 733 now (467 without the
 // filter; 1.66 GB through memory).  48 slices: 118 -> 75 us per launch of an
 // image of 300x300.
 template <int R, bool SPLIT, bool MFMA>
@@ -537,7 +550,7 @@ __device__ __forceinline__ void rowpass_body(const Bases &b, const MsgJob &J, co
   const int H = J.H, W = J.W;
   const int kx = J.kx;
   const RowGeom g = row_geom(W, kx);
-  constexpr int RG = MFMA ? row4_slices(R) : R / row_groups(R), NG = R / RG, Q = RG + 1;
+  constexpr int RG = MFMA ? row4_slices(R) : R / row_groups(R), NG = R / RG, Q = row4_pitch(RG);
   float *t4 = P + row4_floats(RG, W, kx);
   unsigned *bad = reinterpret_cast<unsigned *>(t4 + 4 * tap4_pitch(kx));  // a non-finite value among e
   if (MFMA) {
