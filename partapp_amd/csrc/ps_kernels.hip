@@ -1060,7 +1060,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 // 497 / 431 (6 uneven x48), 740 / 716 (32 300x300x24).  A block of 256 pixels:
 // 13.7, 56, 425, 708; half the rotations per wave 18, 55, 443, 719.  Stores
 // through the caches: odd grids' rows leave partial lines, which L2 merges;
-// nontemporal ones took 424 instead of 301 us on 23 uneven grids.
+// nontemporal ones took 394 instead of 302 us on an uneven batch, and 724 instead
+// of 708 on the even one (blocks of 256 pixels).
 //
 // KC: the number of root children when it is at most 8 (fully unrolled),
 // else kMaxRootChildren with the count read at run time.
