@@ -77,12 +77,12 @@ __device__ __forceinline__ unsigned long long *top2_key(const Bases &b, int k) {
 
 // A block's result for the keys it feeds: the waves' parts, each merged over
 // its lanes, meet in LDS and one thread raises the keys.  Atomics on one cache
-// line queue up at 4 to 13 ns each: by a wave each, all keys of an instance in one
-// line, the leaf maxima of an image of 300x300x48 took 70 us for 17 us of
-// reading (27 so, and 17 with a line per key).  (Reading a key first and
-// raising it only where it is lower queues up
-// just as much once thousands of waves are in flight, and each then waits for
-// its answer: 957 instead of 299 us for the leaf maxima of 32 images.)
+// line queue up at 4 to 13 ns each: by a wave each, all keys of an instance in
+// one line, the leaf maxima of an image of 300x300x48 took 70 us for 17 us of
+// reading (27 so, and 17 with a line per key).  (Reading a key first and raising
+// it only where it is lower queues up just as much once thousands of waves are
+// in flight, and each then waits for its answer: 957 instead of 299 us for the
+// leaf maxima of 32 images.)
 struct KeyPart {
   unsigned key = 0u;                // of a source's maximum
   unsigned long long amax = 0ull;   // (value key << 32) | flipped index of the best state
