@@ -102,11 +102,18 @@ __device__ __forceinline__ f32x4_t mfma4(float a, float b, f32x4_t c) {
 // copies' 16-byte units start in different LDS banks (an odd pitch).
 __host__ __device__ __forceinline__ int tap4_chunks(int k) { return (2 * k + 1 + 3 + 3) >> 2; }
 __host__ __device__ __forceinline__ int tap4_pitch(int k) { return 4 * (tap4_chunks(k) | 1); }
-__device__ __forceinline__ void tap4_fill(float *t4, const float *__restrict__ f, int k) {
+// A thread's first element is loaded ahead, to wait beside the row pass's
+// gather (a launch of 112x128x24: 13.6 -> 12.9 us, of 32 300x300x24: 757 -> 743).
+__device__ __forceinline__ float tap4_load(const float *__restrict__ f, int k) {
+  const int i = (int)threadIdx.x, t = (i >> 2) - (i & 3);
+  return f[min(max(t, 0), 2 * k)];
+}
+__device__ __forceinline__ void tap4_store(float *t4, float first, const float *__restrict__ f, int k) {
   const int L = 2 * k + 1, n4 = 4 * tap4_chunks(k), pitch = tap4_pitch(k);
   for (int i = threadIdx.x; i < 4 * n4; i += blockDim.x) {
     const int n = i & 3, e = i >> 2, t = e - n;
-    t4[n * pitch + e] = t >= 0 && t < L ? f[t] : 0.0f;
+    const float v = i == (int)threadIdx.x ? first : f[min(max(t, 0), 2 * k)];
+    t4[n * pitch + e] = t >= 0 && t < L ? v : 0.0f;
   }
 }
 
@@ -541,7 +548,7 @@ __device__ __forceinline__ void rowpass_rotate(const MsgJob &J, const float *__r
 // on) on the vector unit.  Bound by latency: the filter, the exponentials and
 // rotation filter, and the gather each take some 40% of a launch of 96
 // messages of 300x300x24 and overlap between the 4 blocks that fit a CU only
-// in part: 899 us with the filter on the vector unit, 733 now (467 without the
+// in part: 899 us with the filter on the vector unit, some 730 now (467 without the
 // filter; 1.66 GB through memory).  48 slices: 118 -> 75 us per launch of an
 // image of 300x300.
 template <int R, bool SPLIT, bool MFMA>
@@ -559,7 +566,6 @@ __device__ __forceinline__ void rowpass_body(const Bases &b, const MsgJob &J, co
     const int tail = (kx + W) * Q, end = (W + 4 * tap4_chunks(kx)) * Q;
     for (int i = threadIdx.x; i < kx * Q; i += blockDim.x) P[i] = 0.0f;
     for (int i = tail + (int)threadIdx.x; i < end; i += blockDim.x) P[i] = 0.0f;
-    tap4_fill(t4, taps + J.taps_x, kx);
     if (threadIdx.x == 0) *bad = 0u;
   } else {
     zero_halo(P, RG, W, kx, g.Pw);
@@ -573,6 +579,7 @@ __device__ __forceinline__ void rowpass_body(const Bases &b, const MsgJob &J, co
   float *T = mptr(b, J.tmp);
   const long long plane = (long long)H * J.tpitch;
   const bool one = MFMA && W <= (int)blockDim.x;
+  const float tap0 = MFMA ? tap4_load(taps + J.taps_x, kx) : 0.0f;
   float e[R];
   unsigned bits = 0u;
   auto values = [&](int x) {
@@ -596,7 +603,10 @@ __device__ __forceinline__ void rowpass_body(const Bases &b, const MsgJob &J, co
         else rowpass_rotate<R, RG, G>(J, taps, e, P + kx + x, g.Pw);
       }
     }
-    if (MFMA && G == 0) __syncthreads();  // the flag is clear
+    if (MFMA && G == 0) {
+      tap4_store(t4, tap0, taps + J.taps_x, kx);
+      __syncthreads();  // the flag is clear
+    }
     if (MFMA && bits >= kNonFinite) *bad = 1u;
     __syncthreads();
     float *Tg = T + G * RG * plane;
@@ -845,7 +855,7 @@ __device__ __forceinline__ void colpass_strip(const Bases &b, const MsgJob &J, c
   unsigned *bad = reinterpret_cast<unsigned *>(t4 + 4 * tap4_pitch(ky));
   unsigned bits = 0u;
   if (MFMA) {
-    tap4_fill(t4, fy, ky);
+    tap4_store(t4, tap4_load(fy, ky), fy, ky);
     if (threadIdx.x == 0) *bad = 0u;
     __syncthreads();
   }
