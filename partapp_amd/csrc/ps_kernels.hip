@@ -209,7 +209,7 @@ __host__ __device__ constexpr int row_groups(int R) { return R >= 48 ? 2 : 1; }
 // offsets), kx zeros before the row and the last column's window behind it; the
 // tap operand and the flag follow.  24 slices go through at once (12 at a time
 // halve the LDS and cost a second pass over the rotation filter's inputs: 855
-// against 765 us per launch of 96 messages of 300x300x24) and are read in pairs
+// against 765 us per launch of 32 images of 300x300x24) and are read in pairs
 // (half the LDS instructions: 759 -> 733 us there, 153 -> 140 on uneven grids);
 // 48 go in four groups of 12 (24 beside the 48 values held from group to group
 // spill; three groups of 16, read four at a time, 77.6 against 74.5 us per launch
@@ -546,10 +546,10 @@ __device__ __forceinline__ void rowpass_rotate(const MsgJob &J, const float *__r
 // its values stay in registers from group to group.  Else (rows too wide for
 // the padding and the tap operand in LDS, from some 1500 columns of 24 slices
 // on) on the vector unit.  Bound by latency: the filter, the exponentials and
-// rotation filter, and the gather each take some 40% of a launch of 96
-// messages of 300x300x24 and overlap between the 4 blocks that fit a CU only
-// in part: 899 us with the filter on the vector unit, some 730 now (467 without the
-// filter; 1.66 GB through memory).  48 slices: 118 -> 75 us per launch of an
+// rotation filter, and the gather with the stores overlap between the 4 blocks
+// that fit a CU only in part: 899 us per launch of 32 images of 300x300x24 with the filter on the
+// vector unit, some 730 now (467 without the filter, which is what its 2.49 GB
+// take at the rate of a copy).  48 slices: 118 -> 75 us per launch of an
 // image of 300x300.
 template <int R, bool SPLIT, bool MFMA>
 __device__ __forceinline__ void rowpass_body(const Bases &b, const MsgJob &J, const float *__restrict__ taps,
@@ -725,7 +725,7 @@ __global__ __launch_bounds__(512) void k_rowpass_any(Bases b, const MsgJob *__re
 // MFMA: the filter on the matrix cores, the staged rows a ring in LDS (nothing
 // moves from tile to tile; with the move 1-4% slower).  Bound by memory at some
 // 4 TB/s of scattered grids, and by the barriers between filter and epilogue;
-// us per launch of 96 (32 for the root) messages of 300x300x24, by destination
+// us per launch of 32 images of 300x300x24, by destination
 // kind, vector unit / MFMA 8 rows / 16 rows: downward middle 1340 / 1286 /
 // 1278, downward leaf 1055 / 948 / 1057, up root 978 / 870 / 935, up node 825
 // / 780 / 838.  The vector unit's filter is left for taps so many that the
@@ -1064,7 +1064,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 // The root belief, its marginal and the children's log_from_root of a block of
 // 128 pixels, 8 waves: two tiles of 64, a quarter of the rotations each, so
 // that an image of 112x128 has 112 blocks of 6 steps in a row rather than 56 of
-// 24.  Bound by memory (11 grids, 3.04 GB in 716 us for 32 images of
+// 24.  Bound by memory (12 grids, 3.32 GB in 716 us for 32 images of
 // 300x300x24), on one image by latency.  us before (a wave walks all rotations
 // and raises its own keys) / now: 26 / 11.7 (112x128x24), 99 / 48.6 (300x300x48),
 // 497 / 431 (6 uneven x48), 740 / 716 (32 300x300x24).  A block of 256 pixels:
