@@ -120,6 +120,10 @@ __device__ __forceinline__ void tap4_store(float *t4, float first, const float *
 // bit patterns from here on (infinities, NaNs, and anything negative, which
 // no filter operand is) are not for the MFMA
 constexpr unsigned kNonFinite = 0x7f800000u;
+// The row pass looks at the values before the rotation filter, whose finite
+// sums can overflow: below 2^122 they cannot, with at most 48 taps of at most
+// 1 (a fill value exp(LOG_ZERO - M) lies above it where M < LOG_ZERO - 84.5).
+constexpr unsigned kRowNonFinite = 0x7c800000u;
 __device__ __forceinline__ unsigned max_bits(unsigned m, float v) { return max(m, __float_as_uint(v)); }
 
 // ------------------------------------------------------------------ k_max
@@ -559,7 +563,7 @@ __device__ __forceinline__ void rowpass_body(const Bases &b, const MsgJob &J, co
   const RowGeom g = row_geom(W, kx);
   constexpr int RG = MFMA ? row4_slices(R) : R / row_groups(R), NG = R / RG, Q = row4_pitch(RG);
   float *t4 = P + row4_floats(RG, W, kx);
-  unsigned *bad = reinterpret_cast<unsigned *>(t4 + 4 * tap4_pitch(kx));  // a non-finite value among e
+  unsigned *bad = reinterpret_cast<unsigned *>(t4 + 4 * tap4_pitch(kx));  // P may hold a non-finite value
   if (MFMA) {
     // zeros before the row and as far behind it as a window reaches whose
     // first output is inside
@@ -586,7 +590,6 @@ __device__ __forceinline__ void rowpass_body(const Bases &b, const MsgJob &J, co
     float v[R];
     rowpass_gather<R, SPLIT>(J, shifts, src, y, x, v);
     rowpass_exp<R, SPLIT>(J, shifts, negM, e_fill, y, x, v, e);
-    // the rotation's taps are finite: its outputs are if its inputs are
     if (MFMA) {
 #pragma unroll
       for (int r = 0; r < R; ++r) bits = max_bits(bits, e[r]);
@@ -607,7 +610,7 @@ __device__ __forceinline__ void rowpass_body(const Bases &b, const MsgJob &J, co
       tap4_store(t4, tap0, taps + J.taps_x, kx);
       __syncthreads();  // the flag is clear
     }
-    if (MFMA && bits >= kNonFinite) *bad = 1u;
+    if (MFMA && bits >= kRowNonFinite) *bad = 1u;
     __syncthreads();
     float *Tg = T + G * RG * plane;
     if (!MFMA) xfilter_rows(P, taps + J.taps_x, Tg, RG, J.tpitch, plane, y, g);
