@@ -136,10 +136,11 @@ __global__ __launch_bounds__(256) void k_max(Bases b, const MaxJob *__restrict__
   const MaxJob &J = jobs[blockIdx.y];
   if (skip_inst(b, J.inst)) return;
   const int H = J.H, W = J.W;
-  const int n = R * H * W;  // R H pitch < 2^31 is checked when the plan is built
-  const long long e0l = (long long)blockIdx.x * chunk;
-  if (e0l >= n) return;
-  const int e0 = (int)e0l, e1 = min(n - e0, chunk) + e0;
+  // 64 bits: a message's grid (any rotation count, full covariance) may hold
+  // 2^31 states and more; in the chunk [e0, e0 + n) 32 do
+  const long long total = (long long)R * H * W, e0 = (long long)blockIdx.x * chunk;
+  if (e0 >= total) return;
+  const int n = (int)min(total - e0, (long long)chunk);
   unsigned km = 0u;
   if (J.src_kind == kSrcZero) {
     km = f2key(0.0f);
@@ -147,11 +148,12 @@ __global__ __launch_bounds__(256) void k_max(Bases b, const MaxJob *__restrict__
     const float *src = cptr(b, J.src);
     if (J.mask.rot_bits == 0ull && J.mask.strip == 0) {
       // [a0, a1): whole 16-byte units; the elements before and behind them
-      const int head = (int)((0u - (unsigned)(reinterpret_cast<uintptr_t>(src + e0) >> 2)) & 3u);
-      const int a0 = min(e0 + head, e1), a1 = a0 + ((e1 - a0) & ~3);
+      src += e0;
+      const int head = (int)((0u - (unsigned)(reinterpret_cast<uintptr_t>(src) >> 2)) & 3u);
+      const int a0 = min(head, n), a1 = a0 + ((n - a0) & ~3);
       const int t = (int)threadIdx.x;
-      if (t < a0 - e0) km = f2key(src[e0 + t]);
-      else if (t >= 4 && t - 4 < e1 - a1) km = f2key(src[a1 + t - 4]);
+      if (t < a0) km = f2key(src[t]);
+      else if (t >= 4 && t - 4 < n - a1) km = f2key(src[a1 + t - 4]);
       // four independent loads per thread in flight (a lane past the end
       // reads its first element again, which leaves the max unchanged)
       constexpr int kU = 4;
@@ -171,7 +173,7 @@ __global__ __launch_bounds__(256) void k_max(Bases b, const MaxJob *__restrict__
     } else {
       // the chunk's rows: those that begin in it
       const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-      const int row0 = (e0 + W - 1) / W, row1 = (e1 + W - 1) / W;
+      const int row0 = (int)((e0 + W - 1) / W), row1 = (int)((e0 + n + W - 1) / W);
       const int x0 = J.mask.strip, x1 = W - J.mask.strip;
       bool any = J.mask.strip > 0;  // a masked state
       for (int row = row0 + wave; row < row1; row += 4) {
@@ -180,7 +182,7 @@ __global__ __launch_bounds__(256) void k_max(Bases b, const MaxJob *__restrict__
           continue;
         }
         constexpr int kU = 4;
-        const float *p = src + row * W;
+        const float *p = src + (long long)row * W;
         for (int x = x0 + lane; x < x1; x += kU * 64) {
           float v[kU];
 #pragma unroll
