@@ -1546,6 +1546,10 @@ int message_prepare(const ps_model *model, int height, int width, const double o
   MessagePlan mp;
   st = build_message_plan(m.ep, height, width, offset_c, offset_p, C, rot_mean, rot_sigma, scale, is_sparse != 0, mp);
   if (st != PS_OK) return st;
+  // as in a plan: the column pass and the row passes of 24 and 48 rotations
+  // index a grid in 32 bits (the others, in 64, take any size)
+  if ((!mp.od || R == 24 || R == 48) && (long long)R * height * width >= (1ll << 31))
+    return set_error(PS_ERR_UNSUPPORTED, "R*H*W must be below 2^31");
   Builder B(m);
   MsgJob mj;
   std::memset(&mj, 0, sizeof(mj));

@@ -1,10 +1,12 @@
 """Messages of very large grids: 2^31 states and more where the kernels index
-in 64 bits (any rotation count but 24 and 48, full covariance)."""
+in 64 bits (any rotation count but 24 and 48, full covariance), refused where
+they do not."""
 import math
 
 import numpy as np
 import pytest
 
+from partapp_amd._lib import PsError
 from partapp_amd.api import ExpParam, Joint, PartModel, compute_rot_joint_marginal
 
 pytestmark = pytest.mark.gpu
@@ -36,3 +38,18 @@ def test_more_than_2_31_states(gpu):
         assert (got - want).abs().max().item() < 1e-4
     del child, out
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("R,C", [(24, (4.0, 1.0, 1.0, 9.0)), (48, (4.0, 0.0, 0.0, 9.0)), (2, (4.0, 0.0, 0.0, 9.0))])
+def test_refused(gpu, R, C):
+    # (one address stands for the grids: the call is refused before it reads them)
+    import torch
+    import ctypes
+    from partapp_amd._lib import check, lib
+    m, t = model(R), torch.zeros(64, device=gpu)
+    two, four = ctypes.c_double * 2, ctypes.c_double * 4
+    H = (1 << 31) // (R * 256) + 1
+    with pytest.raises(PsError) as e:
+        check(lib().ps_message(m.handle, t.data_ptr(), t.data_ptr(), H, 256, two(0, 0), two(0, 0), four(*C), 0.0, 0.0, 1.0,
+                               0, None), "ps_message")
+    assert e.value.status == -5
