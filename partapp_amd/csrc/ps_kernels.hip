@@ -494,7 +494,7 @@ __device__ __forceinline__ void rowpass_gather(const MsgJob &J, const int *__res
 #pragma unroll
   for (int ro = 0; ro < R; ++ro) {
     const int yy = min(max(ys + fwd_oy<R, SPLIT>(shifts, so, ro, ys), 0), H - 1);
-    const char *srow = reinterpret_cast<const char *>(src) + (unsigned)(shifts[so + 3 * R + ro] * HW + yy * Ps) * 4u;
+    const char *srow = reinterpret_cast<const char *>(src + (unsigned)(shifts[so + 3 * R + ro] * HW + yy * Ps));
     const int xx4 = min(max(x4 + fwd_ox<R, SPLIT>(shifts, so, ro, x) * 4, 0), xmax4);
     v[ro] = *reinterpret_cast<const float *>(srow + (unsigned)xx4);
   }

@@ -1,6 +1,6 @@
 """Messages of very large grids: 2^31 states and more where the kernels index
 in 64 bits (any rotation count but 24 and 48, full covariance), refused where
-they do not."""
+they do not; grids of more than 4 GB."""
 import math
 
 import numpy as np
@@ -36,6 +36,24 @@ def test_more_than_2_31_states(gpu):
         got = out[:, rows, 40:-40]
         # float weights and sums of 13 x 19 taps, exp and log of the hardware (1 ulp each)
         assert (got - want).abs().max().item() < 1e-4
+    del child, out
+    torch.cuda.empty_cache()
+
+
+def test_source_beyond_4_gb(gpu):
+    # 24 rotations: the last rows of the last slice lie beyond the grid's first 4 GB; each output is the same sum as in
+    # a grid of the last rows alone
+    import torch
+    R, H, W, tail = 24, 32000, 1400, 200
+    assert 1 << 30 < R * H * W - 100 * W and R * H * W < 1 << 31
+    if torch.cuda.mem_get_info()[0] < 30 << 30:
+        pytest.skip("needs 30 GB of device memory")
+    args = ((3.3, -2.7), (-1.4, 4.9), (4.0, 0.0, 0.0, 5.5), 0.2, 0.3, 1.0)
+    child = torch.full((R, H, W), -3.0, device=gpu)
+    child[:, -tail:] = torch.randn((R, tail, W), device=gpu, generator=torch.Generator("cuda").manual_seed(0)) - 3.0
+    want = compute_rot_joint_marginal(model(R), child[:, -tail:].contiguous(), *args)
+    out = compute_rot_joint_marginal(model(R), child, *args)
+    assert torch.equal(out[:, -100:], want[:, -100:])
     del child, out
     torch.cuda.empty_cache()
 
