@@ -290,7 +290,9 @@ int ps_find_local_max(const float *grids_dev, const long long *offsets, const in
  * lands; then scores < 0 become 1e-4 and the log is taken (0 -> LOG_ZERO).
  * Writes log_unary_dev [n][height][width].  Synchronous.  Allocates device
  * memory only for more than 1440 slices (their warps) and for nearest warps
- * that cannot be inverted or shrink extremely (8 bytes per output cell). */
+ * that cannot be inverted or shrink extremely (8 bytes per output cell).
+ * A nearest warp may write onto its own input (that too takes 8 bytes per
+ * output cell); the buffers of a bilinear one must not overlap. */
 int ps_ingest_scores(const float *score_grid_dev, int n, int grid_height, int grid_width, const double *Tig,
                      int interpolate, int height, int width, float *log_unary_dev, void *stream);
 

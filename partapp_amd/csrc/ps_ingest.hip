@@ -14,6 +14,7 @@
 #include <algorithm>
 #include <cfloat>
 #include <cmath>
+#include <functional>
 #include <string>
 #include <vector>
 
@@ -247,7 +248,13 @@ extern "C" int ps_ingest_scores(const float *score_grid_dev, int n, int grid_hei
   hipStream_t st = static_cast<hipStream_t>(stream);
   std::vector<IngestWarp> warps(n);
   for (int s = 0; s < n; ++s) std::copy(&mats[6 * (size_t)s], &mats[6 * (size_t)s] + 6, warps[s].m);
-  bool gather = true, four = true;
+  // a nearest warp onto its own input (log_unary_dev overlapping the grid) is
+  // the scatter's, whose keys hold every value before the first is written
+  const float *grid_end = score_grid_dev + (long long)n * grid_height * grid_width;
+  const float *out_end = log_unary_dev + (long long)n * height * width;
+  const bool overlap = std::less<const float *>()(score_grid_dev, out_end) &&
+                       std::less<const float *>()(log_unary_dev, grid_end);
+  bool gather = interpolate || !overlap, four = true;
   for (int s = 0; s < n && !interpolate && gather; ++s) {
     bool f = false;
     gather = ingest_gather(warps[s].m, grid_height, grid_width, height, width, f);
@@ -288,8 +295,8 @@ extern "C" int ps_ingest_scores(const float *score_grid_dev, int n, int grid_hei
     if (eg != hipSuccess) return set_error(PS_ERR_HIP, std::string("ingest: ") + hipGetErrorString(eg));
     return PS_OK;
   }
-  // some slice's warp is singular, too ill-conditioned or shrinks too much
-  // for the gather: scatter with last-writer keys
+  // the buffers overlap, or some slice's warp is singular, too ill-conditioned
+  // or shrinks too much for the gather: scatter with last-writer keys
   const long long out_n = (long long)n * height * width;
   const size_t mat_bytes = (mats.size() * sizeof(double) + 255) & ~(size_t)255;
   void *ws = nullptr;
