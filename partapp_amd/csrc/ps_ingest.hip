@@ -440,8 +440,20 @@ extern "C" int ps_add_dpm_score(float *part_unary_dev, int S, int R, int height,
     if (n_dpm > 1 && n_dpm < R) return set_error(PS_ERR_INVALID_ARG, "a rotation-dependent DPM prior needs R grids");
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
-  hipLaunchKernelGGL(k_dpm_add, pixel_blocks((long long)height * width, (long long)S * R), dim3(kIngThreads), 0, st,
-                     part_unary_dev, S, R, height, width, dpm_dev, n_dpm, weight, mode, std::log(1e-4));
+  const long long hw = (long long)height * width, n = (long long)S * R;
+  const bool per_r = mode == PS_DPM_RAW ? n_dpm == R : n_dpm > 1;
+  auto add = [&](float *g, int s, int r, const float *dpm, int nd) {
+    hipLaunchKernelGGL(k_dpm_add, pixel_blocks(hw, (long long)s * r), dim3(kIngThreads), 0, st, g, s, r, height, width,
+                       dpm, nd, weight, mode, std::log(1e-4));
+  };
+  // scores that are slices of the part itself: a slice already added to is read
+  // as it then is, so the slices go one after another
+  const std::less<const float *> before;
+  if (before(dpm_dev, part_unary_dev + n * hw) && before(part_unary_dev, dpm_dev + (per_r ? R : 1) * hw)) {
+    for (long long k = 0; k < n; ++k) add(part_unary_dev + k * hw, 1, 1, dpm_dev + (per_r ? k % R : 0) * hw, 1);
+  } else {
+    add(part_unary_dev, S, R, dpm_dev, n_dpm);
+  }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return set_error(PS_ERR_HIP, std::string("dpm score: ") + hipGetErrorString(e));
   return PS_OK;
