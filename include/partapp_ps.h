@@ -150,8 +150,10 @@ int ps_plan_execute_graph(ps_plan *plan, const float *log_unary, float *log_marg
  * on 300x300x24 grids: about 1.5e-4 for BF16 / BF16_MIXED, 1e-4 for BF16X2,
  * 2e-6 for BF16X3 and FP32.  Available for 24 rotations and half widths up to
  * 47 (sigma * scale up to 15.5 px); a level of messages outside that runs FP32
- * (ps_plan_method_levels counts the levels that use the method).  No
- * reference counterpart: a precision option of this library. */
+ * (ps_plan_method_levels counts the levels that use the method).  A plan's
+ * first BF16 method forms its operand tables on the device (an allocation and
+ * a short wait, neither of which joins a capture under way).  No reference
+ * counterpart: a precision option of this library. */
 enum {
   PS_METHOD_FP32 = 0,
   PS_METHOD_BF16 = 1,
@@ -192,7 +194,8 @@ int ps_plan_method_levels(const ps_plan *plan, int *levels, int *mfma_levels);
  * call then waits for the stream) and only the flagged instances' jobs are
  * launched again; under ps_plan_execute_graph the flags stay on the device
  * and the FP32 launches cover the batch, their other blocks exiting at once.
- * tau = 0 turns the guard off (the default).  ps_plan_read_map_guard
+ * tau = 0 turns the guard off (the default).  A plan's first tau > 0
+ * allocates the re-sweep's tables (in no capture).  ps_plan_read_map_guard
  * reports how many instances the last execution re-evaluated (and, if
  * flags_host is given, which: [n_instances]); it waits for `stream`. */
 /* Pruned execution (no counterpart in the reference).  keep_dev holds one

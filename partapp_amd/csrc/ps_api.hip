@@ -13,6 +13,7 @@
 #include <cmath>
 #include <cstdint>
 #include <cstring>
+#include <map>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -908,16 +909,47 @@ struct OnDevice {
   }
 };
 
+// Lets the calling thread allocate and wait while one of its streams, or any
+// stream in the default mode, is being captured: for what a plan gets on the
+// first call that needs it, none of which belongs in the captured graph.
+struct OutsideCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  OutsideCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~OutsideCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
+// A stream of the library's own on the current device, made on first use and
+// kept (making one for a plan's tables took 45 us, forming them 25): a launch
+// on the default stream would join the capture of a stream that waits for it.
+hipError_t own_stream(int device, hipStream_t *s) {
+  static std::mutex mu;
+  static std::map<int, hipStream_t> streams;
+  std::lock_guard<std::mutex> lock(mu);
+  hipStream_t &st = streams[device];
+  if (!st) {
+    const hipError_t e = hipStreamCreateWithFlags(&st, hipStreamNonBlocking);
+    if (e != hipSuccess) {
+      st = nullptr;
+      return e;
+    }
+  }
+  *s = st;
+  return hipSuccess;
+}
+
 // the operand tables of the BF16 passes, complete on return (the plan may be
 // executed on any stream)
 int ensure_fragments(ps_plan *pl) {
   if (pl->frags || pl->frag_units == 0) return PS_OK;
   OnDevice on(pl->device);
+  OutsideCapture outside;
   uint4 *f = nullptr;
   if (pool_get(&f, pl->frag_units * 16) != hipSuccess)
     return set_error(PS_ERR_OUT_OF_MEMORY, "fragment tables (" + std::to_string(pl->frag_units * 16) + " bytes)");
-  hipError_t e = launch_fragments(pl->jobs, (int)pl->h_jobs.size(), pl->taps, pl->R, f, nullptr);
-  if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+  hipStream_t s = nullptr;
+  hipError_t e = own_stream(pl->device, &s);
+  if (e == hipSuccess) e = launch_fragments(pl->jobs, (int)pl->h_jobs.size(), pl->taps, pl->R, f, s);
+  if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) {
     pool_put(f, false);
     return hip_error(e, "fragment tables");
@@ -933,6 +965,7 @@ int ensure_fragments(ps_plan *pl) {
 int ensure_guard(ps_plan *pl) {
   if (pl->ctables) return PS_OK;
   OnDevice on(pl->device);
+  OutsideCapture outside;
   auto align = [](size_t v) { return (v + 255) & ~(size_t)255; };
   pl->cbytes = align(2 * pl->h_jobs.size() * sizeof(MsgJob)) + align(pl->h_roots.size() * sizeof(RootJob)) +
                align(pl->h_maxes.size() * sizeof(MaxJob)) + align(pl->h_maps.size() * sizeof(MapJob));
