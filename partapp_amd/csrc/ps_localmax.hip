@@ -14,6 +14,14 @@
 //   k_lmax_collect  the keys at or above that 22-bit threshold (all of them
 //                   when there are at most max_n)
 //   k_lmax_select   one workgroup per grid sorts those few in LDS
+// Where some grid has more of those keys than LDS takes (k_lmax_select tells
+// the host), all of it runs again with a third histogram (the last 10 bits);
+// where too many values equal that threshold, k_lmax_collect takes the keys
+// above it and k_lmax_select the first of the equal ones in the scan.
+// Grids near LOG_ZERO do it (the bin spans 64 units of value there) and plateaus.
+// Selected by one workgroup from every mark, byte by byte, such a grid of
+// 24 x 300 x 300 took 7.6 ms, now 0.67 (0.18 without the second run), a
+// plateau of 1000 x 1000 6.2 and now 3.0 ms.
 // key = (order key of value) << 32 | (2^32-1 - scan index): distinct, so the
 // result does not depend on the order in which the keys were collected.
 //
@@ -57,11 +65,14 @@ constexpr int kBins = 2048;     // 11 bits
 constexpr int kCap = 8192;      // keys collected per grid (64 KB, sorted in LDS)
 constexpr int kMarkRows = 16;   // rows of a wave's 64-column tile
 
-// per grid: both histograms, then the marked points and the collected keys
+// per grid: the histograms, the marked points and the collected keys; the second
+// run's: whether the third histogram is needed, the 32-bit threshold where only
+// values above it are collected (tie)
 struct LmState {
-  unsigned hist[2][kBins];
+  unsigned hist[3][kBins];
   unsigned marked, collected;
-  unsigned pad_[62];
+  unsigned third, tie, tie_key;
+  unsigned pad_[59];
 };
 
 __device__ __forceinline__ unsigned okey(float f) {
@@ -86,8 +97,7 @@ __device__ __forceinline__ unsigned long long lm_key(const LmGrid &G, float v, i
 // One wave per 64 columns x 16 rows of a slice, a lane per column, the 3 x 3
 // neighbourhood sliding down: five loads per point, four of them lines that
 // the wave or its neighbours have just read.
-__global__ __launch_bounds__(256) void k_lmax_mark(const float *__restrict__ grids, LmBatch gd,
-                                                   unsigned long long *__restrict__ mask, LmState *__restrict__ st) {
+__global__ __launch_bounds__(256) void k_lmax_mark(const float *__restrict__ grids, LmBatch gd, unsigned long long *__restrict__ mask, LmState *__restrict__ st) {
   __shared__ unsigned hist[kBins];
   unsigned bx, by;
   xcd_block(bx, by);
@@ -232,6 +242,8 @@ __device__ __forceinline__ void lm_marked(const float *__restrict__ grids, const
   }
 }
 
+// DIGIT 1: the next 11 bits, 2: the last 10.
+template <int DIGIT>
 __global__ __launch_bounds__(256) void k_lmax_refine(const float *__restrict__ grids, LmBatch gd,
                                                      const unsigned long long *__restrict__ mask,
                                                      LmState *__restrict__ st, int max_n) {
@@ -239,18 +251,27 @@ __global__ __launch_bounds__(256) void k_lmax_refine(const float *__restrict__ g
   LmState &S = st[blockIdx.y];
   if (S.marked <= (unsigned)max_n) return;
   unsigned need = (unsigned)max_n;
-  const unsigned b1 = (unsigned)lm_bin(S.hist[0], need, part);
+  unsigned top = (unsigned)lm_bin(S.hist[0], need, part);  // the leading bits of the values counted
+  if (DIGIT == 2) {
+    const unsigned b = (unsigned)lm_bin(S.hist[1], need, part);
+    top = top << 11 | b;
+    // the keys at or above the 22-bit threshold
+    const bool third = (unsigned)max_n - need + S.hist[1][b] > (unsigned)kCap;
+    if (blockIdx.x == 0 && threadIdx.x == 0) S.third = third;
+    if (!third) return;
+  }
+  constexpr int kShift = DIGIT == 1 ? 10 : 0, kTop = DIGIT == 1 ? 21 : 10;
   for (int i = threadIdx.x; i < kBins; i += 256) hist[i] = 0u;
   __syncthreads();
+  const LmGrid &G = gd.g[blockIdx.y];
   const unsigned wave = (unsigned)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  lm_marked(grids, gd.g[blockIdx.y], mask, blockIdx.x * 4 + wave, gridDim.x * 4,
-            [&](bool on, float v, int, int, int) {
-              const unsigned k = okey(v);
-              if (on && (k >> 21) == b1) atomicAdd(&hist[(k >> 10) & (kBins - 1)], 1u);
-            });
+  lm_marked(grids, G, mask, blockIdx.x * 4 + wave, gridDim.x * 4, [&](bool on, float v, int, int, int) {
+    const unsigned k = okey(v);
+    if (on && (k >> kTop) == top) atomicAdd(&hist[(k >> kShift) & ((1u << (kTop - kShift)) - 1u)], 1u);
+  });
   __syncthreads();
   for (int i = threadIdx.x; i < kBins; i += 256)
-    if (hist[i]) atomicAdd(&S.hist[1][i], hist[i]);
+    if (hist[i]) atomicAdd(&S.hist[DIGIT][i], hist[i]);
 }
 
 __global__ __launch_bounds__(256) void k_lmax_collect(const float *__restrict__ grids, LmBatch gd,
@@ -261,11 +282,23 @@ __global__ __launch_bounds__(256) void k_lmax_collect(const float *__restrict__ 
   LmState &S = st[blockIdx.y];
   const LmGrid &G = gd.g[blockIdx.y];
   unsigned thr = 0u;  // least value key that is collected
-  if (S.marked > (unsigned)max_n) {
+  const unsigned marked = S.marked, third = S.third;
+  if (marked > (unsigned)max_n) {
     unsigned need = (unsigned)max_n;
     const unsigned b1 = (unsigned)lm_bin(S.hist[0], need, part);
     const unsigned b2 = (unsigned)lm_bin(S.hist[1], need, part);
     thr = b1 << 21 | b2 << 10;
+    if (third) {
+      const unsigned b3 = (unsigned)lm_bin(S.hist[2], need, part);
+      thr |= b3;
+      if ((unsigned)max_n - need + S.hist[2][b3] > (unsigned)kCap) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+          S.tie = 1u;
+          S.tie_key = thr;
+        }
+        if (++thr == 0u) return;  // only what lies above: nothing does
+      }
+    }
   }
   unsigned long long *out = keys + (long long)blockIdx.y * kCap;
   const int lane = threadIdx.x & 63;
@@ -277,7 +310,7 @@ __global__ __launch_bounds__(256) void k_lmax_collect(const float *__restrict__ 
     unsigned at = 0u;
     if (lane == 0) at = atomicAdd(&S.collected, (unsigned)__popcll(w));
     at = (unsigned)__shfl((int)at, 0, 64) + (unsigned)__popcll(w & ((1ull << lane) - 1ull));
-    // more than fit (a run of equal values at the threshold): counted only
+    // more than fit: counted only
     if (take && at < (unsigned)kCap) out[at] = lm_key(G, v, d, y, x);
   });
 }
@@ -305,44 +338,46 @@ __global__ __launch_bounds__(kSelThreads) void k_lmax_select(const float *__rest
                                                              const unsigned long long *__restrict__ mask,
                                                              const LmState *__restrict__ st,
                                                              const unsigned long long *__restrict__ keys, int max_n,
-                                                             ps_local_max *__restrict__ out, int *__restrict__ out_n) {
+                                                             ps_local_max *__restrict__ out, int *__restrict__ out_n,
+                                                             unsigned *more_host) {
   __shared__ unsigned long long s[kCap];
   __shared__ unsigned hist[256];
-  __shared__ unsigned long long prefix_s;
-  __shared__ unsigned need_s, fill_s;
+  __shared__ unsigned prefix_s, need_s, fill_s;
   const LmGrid &G = gd.g[blockIdx.x];
+  const LmState &S = st[blockIdx.x];
   const unsigned long long *c = keys + (long long)blockIdx.x * kCap;
-  const unsigned marked = st[blockIdx.x].marked, n = st[blockIdx.x].collected;
+  const unsigned marked = S.marked, n = S.collected;
   const int keep = (int)min(marked, (unsigned)max_n);
+  if (n > (unsigned)kCap) {  // the first run only
+    if (threadIdx.x == 0) __hip_atomic_store(more_host, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    return;
+  }
+  const bool tie = S.tie != 0u;
+  // all of them in scan order (by 2^32-1 - scan descending), or the largest
+  const bool all = marked <= (unsigned)max_n;
+  const int size = tie ? keep : (int)n;
   int n2 = 1;
-  if (n <= (unsigned)kCap) {
-    // all of them in scan order (by 2^32-1 - scan descending), or the largest
-    const bool all = marked <= (unsigned)max_n;
-    while (n2 < (int)n) n2 <<= 1;
-    for (int i = threadIdx.x; i < n2; i += blockDim.x)
-      s[i] = i < (int)n ? (all ? swap_halves(c[i]) : c[i]) : 0ull;
-    bitonic_desc(s, n2);
-    if (all) {
-      for (int i = threadIdx.x; i < keep; i += blockDim.x) s[i] = swap_halves(s[i]);
-      __syncthreads();
-    }
-  } else {
-    // more keys share the threshold's 22 bits than LDS holds: radix select of
-    // the max_n largest over the marks, most significant byte first
+  while (n2 < size) n2 <<= 1;
+  for (int i = threadIdx.x; i < n2; i += blockDim.x) s[i] = i < (int)n ? (all ? swap_halves(c[i]) : c[i]) : 0ull;
+  if (tie) {
+    // fewer than max_n values above the threshold, more than LDS holds equal
+    // to it: radix select of the first in the scan, the most significant byte
+    // of 2^32-1 - scan first
+    const unsigned v0 = S.tie_key;
     if (threadIdx.x == 0) {
-      prefix_s = 0ull;
-      need_s = (unsigned)max_n;
-      fill_s = 0u;
+      prefix_s = 0u;
+      need_s = (unsigned)max_n - n;
+      fill_s = n;
     }
     const unsigned wave = (unsigned)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    unsigned long long m = 0ull;
-    for (int shift = 56; shift >= 0; shift -= 8) {
+    unsigned m = 0u;
+    for (int shift = 24; shift >= 0; shift -= 8) {
       if (threadIdx.x < 256) hist[threadIdx.x] = 0u;
       __syncthreads();
-      const unsigned long long prefix = prefix_s;
+      const unsigned prefix = prefix_s;
       lm_marked(grids, G, mask, wave, kSelThreads / 64, [&](bool on, float v, int d, int y, int x) {
-        const unsigned long long k = lm_key(G, v, d, y, x);
-        if (on && (k & m) == prefix) atomicAdd(&hist[(unsigned)(k >> shift) & 255u], 1u);
+        const unsigned k = (unsigned)lm_key(G, v, d, y, x);
+        if (on && okey(v) == v0 && (k & m) == prefix) atomicAdd(&hist[(k >> shift) & 255u], 1u);
       });
       __syncthreads();
       if (threadIdx.x == 0) {
@@ -353,20 +388,22 @@ __global__ __launch_bounds__(kSelThreads) void k_lmax_select(const float *__rest
           acc += hist[bin];
         }
         need_s = need - acc;
-        prefix_s = prefix | ((unsigned long long)bin << shift);
+        prefix_s = prefix | ((unsigned)bin << shift);
       }
-      m |= 0xffull << shift;
+      m |= 0xffu << shift;
       __syncthreads();
     }
-    // keys are distinct: exactly max_n of them are >= the selected key
-    const unsigned long long thr = prefix_s;
+    // scan indices are distinct: exactly max_n - n of them are >= the selected one
+    const unsigned thr = prefix_s;
     lm_marked(grids, G, mask, wave, kSelThreads / 64, [&](bool on, float v, int d, int y, int x) {
       const unsigned long long k = lm_key(G, v, d, y, x);
-      if (on && k >= thr) s[atomicAdd(&fill_s, 1u)] = k;
+      if (on && okey(v) == v0 && (unsigned)k >= thr) s[atomicAdd(&fill_s, 1u)] = k;
     });
-    while (n2 < keep) n2 <<= 1;
-    for (int i = keep + threadIdx.x; i < n2; i += blockDim.x) s[i] = 0ull;
-    bitonic_desc(s, n2);
+  }
+  bitonic_desc(s, n2);
+  if (all) {
+    for (int i = threadIdx.x; i < keep; i += blockDim.x) s[i] = swap_halves(s[i]);
+    __syncthreads();
   }
   ps_local_max *o = out + (long long)blockIdx.x * max_n;
   for (int i = threadIdx.x; i < keep; i += blockDim.x) {
@@ -420,34 +457,44 @@ extern "C" int ps_find_local_max(const float *grids_dev, const long long *offset
   LmState *st = reinterpret_cast<LmState *>(base);
   unsigned long long *keys = reinterpret_cast<unsigned long long *>(base + o_keys);
   unsigned long long *mask = reinterpret_cast<unsigned long long *>(base + o_mask);
+  unsigned *more = nullptr;  // in host memory
+  hipError_t e = pool_get_host(&more);
+  if (e == hipSuccess) *more = 0u;
   // counters cleared by a small kernel (this entry point synchronizes and is
   // not capturable)
   const long long n_state = (long long)(o_keys / sizeof(unsigned));
-  hipLaunchKernelGGL(k_lmax_clear, dim3((unsigned)((n_state + 255) / 256)), dim3(256), 0, s,
-                     reinterpret_cast<unsigned *>(st), n_state);
-  hipError_t e = hipGetLastError();
-  for (int g0 = 0; g0 < n_grids && e == hipSuccess; g0 += LmBatch::kMax) {
-    const int n = std::min(n_grids - g0, LmBatch::kMax);
-    LmBatch b;
-    std::copy(gd.begin() + g0, gd.begin() + g0 + n, b.g);
-    long long tiles = 0, most = 0;
-    for (int i = 0; i < n; ++i) {
-      tiles = std::max(tiles, (long long)b.g[i].D * ((b.g[i].H + kMarkRows - 1) / kMarkRows) * b.g[i].wq);
-      most = std::max(most, (long long)b.g[i].D * b.g[i].H * b.g[i].wq);
+  for (const bool third : {false, true}) {
+    if (e == hipSuccess) {
+      hipLaunchKernelGGL(k_lmax_clear, dim3((unsigned)((n_state + 255) / 256)), dim3(256), 0, s,
+                         reinterpret_cast<unsigned *>(st), n_state);
+      e = hipGetLastError();
     }
-    const dim3 blk(256);
-    // the marked points again: 8 words per wave and turn, at most 128 blocks a grid
-    const dim3 again((unsigned)std::min<long long>(128, (most + 31) / 32), (unsigned)n);
-    const dim3 mark((unsigned)std::min<long long>(1 << 22, (tiles + 3) / 4), (unsigned)n);
-    hipLaunchKernelGGL(k_lmax_mark, mark, blk, 0, s, grids_dev, b, mask, st + g0);
-    hipLaunchKernelGGL(k_lmax_refine, again, blk, 0, s, grids_dev, b, mask, st + g0, max_n);
-    hipLaunchKernelGGL(k_lmax_collect, again, blk, 0, s, grids_dev, b, mask, st + g0, max_n,
-                       keys + (long long)g0 * kCap);
-    hipLaunchKernelGGL(k_lmax_select, dim3((unsigned)n), dim3(kSelThreads), 0, s, grids_dev, b, mask, st + g0,
-                       keys + (long long)g0 * kCap, max_n, out_dev + (long long)g0 * max_n, count_dev + g0);
-    e = hipGetLastError();
+    for (int g0 = 0; g0 < n_grids && e == hipSuccess; g0 += LmBatch::kMax) {
+      const int n = std::min(n_grids - g0, LmBatch::kMax);
+      LmBatch b;
+      std::copy(gd.begin() + g0, gd.begin() + g0 + n, b.g);
+      long long tiles = 0, most = 0;
+      for (int i = 0; i < n; ++i) {
+        tiles = std::max(tiles, (long long)b.g[i].D * ((b.g[i].H + kMarkRows - 1) / kMarkRows) * b.g[i].wq);
+        most = std::max(most, (long long)b.g[i].D * b.g[i].H * b.g[i].wq);
+      }
+      const dim3 blk(256);
+      // the marked points again: 8 words per wave and turn, at most 128 blocks a grid
+      const dim3 again((unsigned)std::min<long long>(128, (most + 31) / 32), (unsigned)n);
+      const dim3 mark((unsigned)std::min<long long>(1 << 22, (tiles + 3) / 4), (unsigned)n);
+      hipLaunchKernelGGL(k_lmax_mark, mark, blk, 0, s, grids_dev, b, mask, st + g0);
+      hipLaunchKernelGGL(k_lmax_refine<1>, again, blk, 0, s, grids_dev, b, mask, st + g0, max_n);
+      if (third) hipLaunchKernelGGL(k_lmax_refine<2>, again, blk, 0, s, grids_dev, b, mask, st + g0, max_n);
+      hipLaunchKernelGGL(k_lmax_collect, again, blk, 0, s, grids_dev, b, mask, st + g0, max_n,
+                         keys + (long long)g0 * kCap);
+      hipLaunchKernelGGL(k_lmax_select, dim3((unsigned)n), dim3(kSelThreads), 0, s, grids_dev, b, mask, st + g0,
+                         keys + (long long)g0 * kCap, max_n, out_dev + (long long)g0 * max_n, count_dev + g0, more);
+      e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (e != hipSuccess || *more == 0u) break;
   }
-  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  pool_put_host(more, e == hipSuccess);
   pool_put(ws, e == hipSuccess);
   if (e != hipSuccess) return set_error(PS_ERR_HIP, std::string("local max: ") + hipGetErrorString(e));
   return PS_OK;

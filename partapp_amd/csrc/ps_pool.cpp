@@ -22,6 +22,7 @@ struct Pool {
   std::mutex mu;
   std::vector<Block> idle;          // oldest first
   std::map<void *, Block> lent;
+  std::vector<unsigned *> words;    // idle
 };
 Pool &pool() {
   static Pool *p = new Pool;
@@ -113,18 +114,52 @@ void pool_put(void *p, bool idle) {
   for (const Block &b : freed) (void)hipFree(b.p);
 }
 
+hipError_t pool_get_host(unsigned **p) {
+  *p = nullptr;
+  Pool &q = pool();
+  {
+    std::lock_guard<std::mutex> lock(q.mu);
+    if (!q.words.empty()) {
+      *p = q.words.back();
+      q.words.pop_back();
+      return hipSuccess;
+    }
+  }
+  // portable: any device's kernels write it
+  return hipHostMalloc(reinterpret_cast<void **>(p), sizeof(unsigned), hipHostMallocPortable);
+}
+
+void pool_put_host(unsigned *p, bool idle) {
+  if (!p) return;
+  Pool &q = pool();
+  if (idle) {
+    std::lock_guard<std::mutex> lock(q.mu);
+    if (q.words.size() < kPoolWords) {
+      q.words.push_back(p);
+      return;
+    }
+  }
+  (void)hipHostFree(p);
+}
+
 hipError_t pool_trim() {
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
   Pool &q = pool();
   std::vector<Block> freed;
+  std::vector<unsigned *> words;
   {
     std::lock_guard<std::mutex> lock(q.mu);
     freed = take_idle(q, dev);
+    words.swap(q.words);
   }
   for (const Block &b : freed) {
     const hipError_t f = hipFree(b.p);
+    if (e == hipSuccess) e = f;
+  }
+  for (unsigned *w : words) {
+    const hipError_t f = hipHostFree(w);
     if (e == hipSuccess) e = f;
   }
   return e;

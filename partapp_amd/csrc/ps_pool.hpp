@@ -30,7 +30,13 @@ hipError_t pool_get(T **p, size_t bytes) {
 // give a block back (null: nothing); idle: no work on it is pending, else it
 // is freed, which waits for the device
 void pool_put(void *p, bool idle);
-// free the cached blocks of the current device
+// A word of pinned host memory that kernels write and the caller reads once its
+// stream has ended (a word copied back costs a call some 10 us, one allocated for
+// it far more); at most kPoolWords are kept.
+constexpr size_t kPoolWords = 16;
+hipError_t pool_get_host(unsigned **p);
+void pool_put_host(unsigned *p, bool idle);
+// free the cached blocks of the current device, and the words
 hipError_t pool_trim();
 
 }  // namespace ps

@@ -1,0 +1,52 @@
+"""Local maxima of grids whose values share more leading bits than the first
+threshold looks at: values near LOG_ZERO, few distinct values, plateaus, of any
+sign; against the oracle's scan (ties by scan order)."""
+import numpy as np
+import pytest
+
+import oracle
+from partapp_amd.api import find_local_max
+
+pytestmark = pytest.mark.gpu
+
+
+def got(g, max_n, gpu):
+    import torch
+    r = find_local_max(torch.from_numpy(g).to(gpu), max_n)
+    return [(int(a["d"]), int(a["x"]), int(a["y"]), float(a["score"])) for a in r]
+
+
+def ref(g, max_n):
+    return [(int(d), int(x), int(y), float(np.float32(v))) for d, x, y, v in oracle.find_local_max(g, max_n)]
+
+
+def grid(kind):
+    rng = np.random.default_rng(sum(map(ord, kind)))
+    shape = (4, 250, 300)  # some 25000 maxima of noise
+    if kind == "near_log_zero":    # spacing 1/16: all in one 22-bit bin, tens to a value
+        return rng.normal(-1e6, 4, shape)
+    if kind == "some_live":        # a few hundred above, the rest as before
+        g = rng.normal(-1e6, 4, shape)
+        g[1, ::16, ::20] = rng.normal(-3, 1, g[1, ::16, ::20].shape)
+        return g
+    if kind == "six_values":       # thousands to a value
+        return -1e6 + rng.integers(0, 6, shape)
+    if kind == "two_planes":       # a plateau in every other slice, none of whose neighbours reach it
+        g = np.zeros(shape)
+        g[::2] = 1.0
+        g[0, 100:110, 50:60] = rng.random((10, 10)) + 1.0
+        return g
+    if kind == "negative_plane":
+        g = np.full((1,) + shape[1:], -2.5)
+        g[0, 7, 5:300:7] = -2.25
+        return g
+    g = np.full((1,) + shape[1:], np.inf)  # infinite_plane
+    return g
+
+
+@pytest.mark.parametrize("kind", ["near_log_zero", "some_live", "six_values", "two_planes", "negative_plane",
+                                  "infinite_plane"])
+@pytest.mark.parametrize("max_n", [1, 30, 1000, 4096])
+def test_shared_bits(gpu, kind, max_n):
+    g = grid(kind).astype(np.float32)
+    assert got(g, max_n, gpu) == ref(g, max_n)
