@@ -36,6 +36,7 @@
 #include <algorithm>
 #include <cstring>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/partapp_ps.h"
@@ -64,6 +65,7 @@ constexpr int kMaxLocalMax = 4096;
 constexpr int kBins = 2048;     // 11 bits
 constexpr int kCap = 8192;      // keys collected per grid (64 KB, sorted in LDS)
 constexpr int kMarkRows = 16;   // rows of a wave's 64-column tile
+constexpr int kTabGrids = 1024; // grids of one set of launches that reads a table
 
 // per grid: the histograms, the marked points and the collected keys; the second
 // run's: whether the third histogram is needed, the 32-bit threshold where only
@@ -89,6 +91,15 @@ __global__ __launch_bounds__(256) void k_lmax_clear(unsigned *__restrict__ p, lo
   if (i < n) p[i] = 0u;
 }
 
+// grid i of a launch: from the arguments, or (TAB) from the table.  Two
+// variants of each kernel: chosen at run time, its sizes end up in vector
+// registers and every address with them, and marking takes 1.5 times as long.
+template <bool TAB>
+__device__ __forceinline__ const LmGrid &lm_grid(const LmBatch &b, const LmGrid *__restrict__ tab, unsigned i) {
+  if constexpr (TAB) return tab[i];
+  else return b.g[i];
+}
+
 __device__ __forceinline__ unsigned long long lm_key(const LmGrid &G, float v, int d, int y, int x) {
   const unsigned scan = (unsigned)(((long long)d * G.W + x) * G.H + y);  // d, then x, then y
   return ((unsigned long long)okey(v) << 32) | (unsigned long long)(0xffffffffu - scan);
@@ -97,11 +108,13 @@ __device__ __forceinline__ unsigned long long lm_key(const LmGrid &G, float v, i
 // One wave per 64 columns x 16 rows of a slice, a lane per column, the 3 x 3
 // neighbourhood sliding down: five loads per point, four of them lines that
 // the wave or its neighbours have just read.
-__global__ __launch_bounds__(256) void k_lmax_mark(const float *__restrict__ grids, LmBatch gd, unsigned long long *__restrict__ mask, LmState *__restrict__ st) {
+template <bool TAB>
+__global__ __launch_bounds__(256) void k_lmax_mark(const float *__restrict__ grids, LmBatch gd,
+                                                   const LmGrid *__restrict__ tab, unsigned long long *__restrict__ mask, LmState *__restrict__ st) {
   __shared__ unsigned hist[kBins];
   unsigned bx, by;
   xcd_block(bx, by);
-  const LmGrid &G = gd.g[by];
+  const LmGrid &G = lm_grid<TAB>(gd, tab, by);
   const int D = G.D, H = G.H, W = G.W;
   const unsigned yt = (unsigned)(H + kMarkRows - 1) / kMarkRows, wq = (unsigned)G.wq;
   const unsigned tiles = (unsigned)D * yt * wq;  // at most D H W < 2^31
@@ -243,8 +256,9 @@ __device__ __forceinline__ void lm_marked(const float *__restrict__ grids, const
 }
 
 // DIGIT 1: the next 11 bits, 2: the last 10.
-template <int DIGIT>
+template <int DIGIT, bool TAB>
 __global__ __launch_bounds__(256) void k_lmax_refine(const float *__restrict__ grids, LmBatch gd,
+                                                     const LmGrid *__restrict__ tab,
                                                      const unsigned long long *__restrict__ mask,
                                                      LmState *__restrict__ st, int max_n) {
   __shared__ unsigned hist[kBins], part[4];
@@ -263,7 +277,7 @@ __global__ __launch_bounds__(256) void k_lmax_refine(const float *__restrict__ g
   constexpr int kShift = DIGIT == 1 ? 10 : 0, kTop = DIGIT == 1 ? 21 : 10;
   for (int i = threadIdx.x; i < kBins; i += 256) hist[i] = 0u;
   __syncthreads();
-  const LmGrid &G = gd.g[blockIdx.y];
+  const LmGrid &G = lm_grid<TAB>(gd, tab, blockIdx.y);
   const unsigned wave = (unsigned)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   lm_marked(grids, G, mask, blockIdx.x * 4 + wave, gridDim.x * 4, [&](bool on, float v, int, int, int) {
     const unsigned k = okey(v);
@@ -274,13 +288,15 @@ __global__ __launch_bounds__(256) void k_lmax_refine(const float *__restrict__ g
     if (hist[i]) atomicAdd(&S.hist[DIGIT][i], hist[i]);
 }
 
+template <bool TAB>
 __global__ __launch_bounds__(256) void k_lmax_collect(const float *__restrict__ grids, LmBatch gd,
+                                                      const LmGrid *__restrict__ tab,
                                                       const unsigned long long *__restrict__ mask,
                                                       LmState *__restrict__ st, int max_n,
                                                       unsigned long long *__restrict__ keys) {
   __shared__ unsigned part[4];
   LmState &S = st[blockIdx.y];
-  const LmGrid &G = gd.g[blockIdx.y];
+  const LmGrid &G = lm_grid<TAB>(gd, tab, blockIdx.y);
   unsigned thr = 0u;  // least value key that is collected
   const unsigned marked = S.marked, third = S.third;
   if (marked > (unsigned)max_n) {
@@ -334,7 +350,9 @@ __device__ void bitonic_desc(unsigned long long *s, int n) {
 
 __device__ __forceinline__ unsigned long long swap_halves(unsigned long long k) { return (k << 32) | (k >> 32); }
 
+template <bool TAB>
 __global__ __launch_bounds__(kSelThreads) void k_lmax_select(const float *__restrict__ grids, LmBatch gd,
+                                                             const LmGrid *__restrict__ tab,
                                                              const unsigned long long *__restrict__ mask,
                                                              const LmState *__restrict__ st,
                                                              const unsigned long long *__restrict__ keys, int max_n,
@@ -343,7 +361,7 @@ __global__ __launch_bounds__(kSelThreads) void k_lmax_select(const float *__rest
   __shared__ unsigned long long s[kCap];
   __shared__ unsigned hist[256];
   __shared__ unsigned prefix_s, need_s, fill_s;
-  const LmGrid &G = gd.g[blockIdx.x];
+  const LmGrid &G = lm_grid<TAB>(gd, tab, blockIdx.x);
   const LmState &S = st[blockIdx.x];
   const unsigned long long *c = keys + (long long)blockIdx.x * kCap;
   const unsigned marked = S.marked, n = S.collected;
@@ -432,12 +450,16 @@ extern "C" int ps_find_local_max(const float *grids_dev, const long long *offset
   if (!grids_dev || !offsets || !dims || n_grids < 1 || !out_dev || !count_dev)
     return set_error(PS_ERR_INVALID_ARG, "null argument or n_grids < 1");
   if (max_n < 1 || max_n > kMaxLocalMax) return set_error(PS_ERR_UNSUPPORTED, "max_n must be in [1, 4096]");
+  // grids of one set of launches: in the kernels' arguments, or in a table
+  // where a call has very many
+  const int step = n_grids <= LmBatch::kMax ? LmBatch::kMax : kTabGrids;
   std::vector<LmGrid> gd(n_grids);
-  long long words = 0;
+  long long words = 0, most_words = 0;  // of one set
   for (int g = 0; g < n_grids; ++g) {
     const int D = dims[3 * g], H = dims[3 * g + 1], W = dims[3 * g + 2];
     if (D < 1 || H < 1 || W < 1 || offsets[g] < 0) return set_error(PS_ERR_INVALID_ARG, "bad grid dims or offset");
     if ((long long)D * H * W >= (1ll << 31)) return set_error(PS_ERR_UNSUPPORTED, "grid too large");
+    if (g % step == 0) words = 0;
     gd[g].off = offsets[g];
     gd[g].mask_off = words;
     gd[g].D = D;
@@ -445,50 +467,60 @@ extern "C" int ps_find_local_max(const float *grids_dev, const long long *offset
     gd[g].W = W;
     gd[g].wq = (W + 63) / 64;
     words += (long long)D * H * gd[g].wq;
+    most_words = std::max(most_words, words);
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
-  // workspace: histograms and counters, collected keys, marks
-  const size_t o_keys = sizeof(LmState) * (size_t)n_grids;
-  const size_t o_mask = o_keys + sizeof(unsigned long long) * kCap * (size_t)n_grids;
+  // workspace, used by one set after another: histograms and counters,
+  // collected keys, marks; the table
+  const size_t n_set = (size_t)std::min(n_grids, step);
+  const size_t o_keys = sizeof(LmState) * n_set;
+  const size_t o_mask = o_keys + sizeof(unsigned long long) * kCap * n_set;
+  const size_t o_tab = o_mask + sizeof(unsigned long long) * (size_t)most_words;
+  const bool table = n_grids > LmBatch::kMax;
   void *ws = nullptr;
-  if (pool_get(&ws, o_mask + sizeof(unsigned long long) * (size_t)words) != hipSuccess)
+  if (pool_get(&ws, o_tab + (table ? sizeof(LmGrid) * (size_t)n_grids : 0)) != hipSuccess)
     return set_error(PS_ERR_OUT_OF_MEMORY, "local max workspace");
   char *base = static_cast<char *>(ws);
   LmState *st = reinterpret_cast<LmState *>(base);
   unsigned long long *keys = reinterpret_cast<unsigned long long *>(base + o_keys);
   unsigned long long *mask = reinterpret_cast<unsigned long long *>(base + o_mask);
+  LmGrid *tab = table ? reinterpret_cast<LmGrid *>(base + o_tab) : nullptr;
   unsigned *more = nullptr;  // in host memory
   hipError_t e = pool_get_host(&more);
   if (e == hipSuccess) *more = 0u;
-  // counters cleared by a small kernel (this entry point synchronizes and is
-  // not capturable)
-  const long long n_state = (long long)(o_keys / sizeof(unsigned));
+  if (table && e == hipSuccess)
+    e = hipMemcpyAsync(tab, gd.data(), sizeof(LmGrid) * (size_t)n_grids, hipMemcpyHostToDevice, s);
   for (const bool third : {false, true}) {
-    if (e == hipSuccess) {
-      hipLaunchKernelGGL(k_lmax_clear, dim3((unsigned)((n_state + 255) / 256)), dim3(256), 0, s,
-                         reinterpret_cast<unsigned *>(st), n_state);
-      e = hipGetLastError();
-    }
-    for (int g0 = 0; g0 < n_grids && e == hipSuccess; g0 += LmBatch::kMax) {
-      const int n = std::min(n_grids - g0, LmBatch::kMax);
+    for (int g0 = 0; g0 < n_grids && e == hipSuccess; g0 += step) {
+      const int n = std::min(n_grids - g0, step);
+      const LmGrid *one = gd.data() + g0, *t = table ? tab + g0 : nullptr;
       LmBatch b;
-      std::copy(gd.begin() + g0, gd.begin() + g0 + n, b.g);
+      if (!table) std::copy(one, one + n, b.g);
       long long tiles = 0, most = 0;
       for (int i = 0; i < n; ++i) {
-        tiles = std::max(tiles, (long long)b.g[i].D * ((b.g[i].H + kMarkRows - 1) / kMarkRows) * b.g[i].wq);
-        most = std::max(most, (long long)b.g[i].D * b.g[i].H * b.g[i].wq);
+        tiles = std::max(tiles, (long long)one[i].D * ((one[i].H + kMarkRows - 1) / kMarkRows) * one[i].wq);
+        most = std::max(most, (long long)one[i].D * one[i].H * one[i].wq);
       }
+      // counters cleared by a small kernel (this entry point synchronizes and is
+      // not capturable)
+      const long long n_state = (long long)(sizeof(LmState) / sizeof(unsigned)) * n;
+      hipLaunchKernelGGL(k_lmax_clear, dim3((unsigned)((n_state + 255) / 256)), dim3(256), 0, s,
+                         reinterpret_cast<unsigned *>(st), n_state);
       const dim3 blk(256);
       // the marked points again: 8 words per wave and turn, at most 128 blocks a grid
       const dim3 again((unsigned)std::min<long long>(128, (most + 31) / 32), (unsigned)n);
-      const dim3 mark((unsigned)std::min<long long>(1 << 22, (tiles + 3) / 4), (unsigned)n);
-      hipLaunchKernelGGL(k_lmax_mark, mark, blk, 0, s, grids_dev, b, mask, st + g0);
-      hipLaunchKernelGGL(k_lmax_refine<1>, again, blk, 0, s, grids_dev, b, mask, st + g0, max_n);
-      if (third) hipLaunchKernelGGL(k_lmax_refine<2>, again, blk, 0, s, grids_dev, b, mask, st + g0, max_n);
-      hipLaunchKernelGGL(k_lmax_collect, again, blk, 0, s, grids_dev, b, mask, st + g0, max_n,
-                         keys + (long long)g0 * kCap);
-      hipLaunchKernelGGL(k_lmax_select, dim3((unsigned)n), dim3(kSelThreads), 0, s, grids_dev, b, mask, st + g0,
-                         keys + (long long)g0 * kCap, max_n, out_dev + (long long)g0 * max_n, count_dev + g0, more);
+      const dim3 mark((unsigned)std::min<long long>(1 << 20, (tiles + 3) / 4), (unsigned)n);
+      auto launch = [&](auto tabc) {
+        constexpr bool T = decltype(tabc)::value;
+        hipLaunchKernelGGL((k_lmax_mark<T>), mark, blk, 0, s, grids_dev, b, t, mask, st);
+        hipLaunchKernelGGL((k_lmax_refine<1, T>), again, blk, 0, s, grids_dev, b, t, mask, st, max_n);
+        if (third) hipLaunchKernelGGL((k_lmax_refine<2, T>), again, blk, 0, s, grids_dev, b, t, mask, st, max_n);
+        hipLaunchKernelGGL((k_lmax_collect<T>), again, blk, 0, s, grids_dev, b, t, mask, st, max_n, keys);
+        hipLaunchKernelGGL((k_lmax_select<T>), dim3((unsigned)n), dim3(kSelThreads), 0, s, grids_dev, b, t, mask, st, keys,
+                           max_n, out_dev + (long long)g0 * max_n, count_dev + g0, more);
+      };
+      if (table) launch(std::true_type());
+      else launch(std::false_type());
       e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipStreamSynchronize(s);

@@ -1,6 +1,7 @@
 """Local maxima of grids whose values share more leading bits than the first
-threshold looks at: values near LOG_ZERO, few distinct values, plateaus, of any
-sign; against the oracle's scan (ties by scan order)."""
+threshold looks at: values near LOG_ZERO, few distinct values, plateaus, in
+grids of any sign, and more grids than one set of launches takes; against the
+oracle's scan (ties by scan order)."""
 import numpy as np
 import pytest
 
@@ -50,3 +51,14 @@ def grid(kind):
 def test_shared_bits(gpu, kind, max_n):
     g = grid(kind).astype(np.float32)
     assert got(g, max_n, gpu) == ref(g, max_n)
+
+
+@pytest.mark.parametrize("n", [96, 97, 1025])
+def test_many_grids(gpu, n):
+    import torch
+    rng = np.random.default_rng(n)
+    gs = [rng.normal(0, 1, (1 + i % 3, 3 + i % 7, 5 + i % 80)).astype(np.float32) for i in range(n)]
+    gs[n - 1] = np.full((1, 100, 100), 2.0, np.float32)
+    res = find_local_max([torch.from_numpy(g).to(gpu) for g in gs], 12)
+    for g, r in zip(gs, res):
+        assert [(int(a["d"]), int(a["x"]), int(a["y"]), float(a["score"])) for a in r] == ref(g, 12)
