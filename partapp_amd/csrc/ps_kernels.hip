@@ -549,20 +549,26 @@ __device__ __forceinline__ void rowpass_rotate(const MsgJob &J, const float *__r
 // reference's default 48), row y: lane t owns the columns x = t (mod
 // blockDim.x); the slice groups go through P and the x filter one after
 // another.  MFMA: the x filter on the matrix cores; with one column per lane
-// its values stay in registers from group to group.  Else (rows too wide for
-// the padding and the tap operand in LDS, from some 1500 columns of 24 slices
-// on) on the vector unit.  Bound by latency: the filter, the exponentials and
+// its values stay in registers from group to group.  Else (row_on_mfma) on the
+// vector unit.  Bound by latency: the filter, the exponentials and
 // rotation filter, and the gather with the stores overlap between the 4 blocks
 // that fit a CU only in part: 899 us per launch of 32 images of 300x300x24 with the filter on the
 // vector unit, some 730 now (467 without the filter, which is what its 2.49 GB
 // take at the rate of a copy).  48 slices: 118 -> 75 us per launch of an
 // image of 300x300.
-template <int R, bool SPLIT, bool MFMA>
+// KIND: the filter on the vector unit, on the matrix cores, or there with rows
+// of more columns than threads, where waves past the row do nothing (a test that
+// the narrower rows do without: with it 382 becomes 402 us per sweep of 8 images
+// of 200x300x24; without it 834 instead of 736 at 200x520).
+enum RowKind : int { kRowVector = 0, kRowMfma = 1, kRowMfmaWide = 2 };
+
+template <int R, bool SPLIT, int KIND>
 __device__ __forceinline__ void rowpass_body(const Bases &b, const MsgJob &J, const float *__restrict__ taps,
                                              const int *__restrict__ shifts, float *P, int y) {
   const int H = J.H, W = J.W;
   const int kx = J.kx;
   const RowGeom g = row_geom(W, kx);
+  constexpr bool MFMA = KIND != kRowVector;
   constexpr int RG = MFMA ? row4_slices(R) : R / row_groups(R), NG = R / RG, Q = row4_pitch(RG);
   float *t4 = P + row4_floats(RG, W, kx);
   unsigned *bad = reinterpret_cast<unsigned *>(t4 + 4 * tap4_pitch(kx));  // P may hold a non-finite value
@@ -602,6 +608,7 @@ __device__ __forceinline__ void rowpass_body(const Bases &b, const MsgJob &J, co
     if (G > 0) __syncthreads();  // every item of the group before is filtered
     for (int x0 = 0; x0 < W; x0 += (int)blockDim.x) {
       const int x = x0 + (int)threadIdx.x;
+      if (KIND != kRowMfma && __builtin_amdgcn_readfirstlane(x) >= W) break;
       if (!one || G == 0) values(min(x, W - 1));  // past the row: its last column again
       if (x < W) {
         if (MFMA) rowpass_rotate<R, RG, G>(J, taps, e, P + (kx + x) * Q, std::integral_constant<int, 1>{});
@@ -627,7 +634,7 @@ __device__ __forceinline__ void rowpass_body(const Bases &b, const MsgJob &J, co
   }
 }
 
-template <int R, bool SPLIT, bool MFMA>
+template <int R, bool SPLIT, int KIND>
 __global__ __launch_bounds__(512) void k_rowpass_r(Bases b, const MsgJob *__restrict__ jobs,
                                                    const float *__restrict__ taps, const int *__restrict__ shifts) {
   extern __shared__ float4 lds4[];
@@ -639,8 +646,8 @@ __global__ __launch_bounds__(512) void k_rowpass_r(Bases b, const MsgJob *__rest
   const int y = (int)bx;
   if (y >= J.H) return;
   // a warp whose offset changes along an axis takes the SPLIT variants
-  if (SPLIT && J.split != 0) rowpass_body<R, SPLIT, MFMA>(b, J, taps, shifts, P, y);
-  else rowpass_body<R, false, MFMA>(b, J, taps, shifts, P, y);
+  if (SPLIT && J.split != 0) rowpass_body<R, SPLIT, KIND>(b, J, taps, shifts, P, y);
+  else rowpass_body<R, false, KIND>(b, J, taps, shifts, P, y);
 }
 
 // Row pass for any rotation count: the exponentiated column goes through an
@@ -1342,16 +1349,20 @@ hipError_t raise_lds_limit(const void *f, size_t bytes) {
   return e;
 }
 
+template <int KIND>
+static hipError_t rowpass_kind_set_lds_limit(size_t bytes) {
+  hipError_t e = raise_lds_limit(reinterpret_cast<const void *>(&k_rowpass_r<24, false, KIND>), bytes);
+  if (e == hipSuccess) e = raise_lds_limit(reinterpret_cast<const void *>(&k_rowpass_r<48, false, KIND>), bytes);
+  if (e == hipSuccess) e = raise_lds_limit(reinterpret_cast<const void *>(&k_rowpass_r<24, true, KIND>), bytes);
+  if (e == hipSuccess) e = raise_lds_limit(reinterpret_cast<const void *>(&k_rowpass_r<48, true, KIND>), bytes);
+  return e;
+}
+
 // bytes, bytes4: the vector and the MFMA row pass's largest LDS
 hipError_t rowpass_set_lds_limit(size_t bytes, size_t bytes4) {
-  hipError_t e = raise_lds_limit(reinterpret_cast<const void *>(&k_rowpass_r<24, false, false>), bytes);
-  if (e == hipSuccess) e = raise_lds_limit(reinterpret_cast<const void *>(&k_rowpass_r<48, false, false>), bytes);
-  if (e == hipSuccess) e = raise_lds_limit(reinterpret_cast<const void *>(&k_rowpass_r<24, true, false>), bytes);
-  if (e == hipSuccess) e = raise_lds_limit(reinterpret_cast<const void *>(&k_rowpass_r<48, true, false>), bytes);
-  if (e == hipSuccess) e = raise_lds_limit(reinterpret_cast<const void *>(&k_rowpass_r<24, false, true>), bytes4);
-  if (e == hipSuccess) e = raise_lds_limit(reinterpret_cast<const void *>(&k_rowpass_r<48, false, true>), bytes4);
-  if (e == hipSuccess) e = raise_lds_limit(reinterpret_cast<const void *>(&k_rowpass_r<24, true, true>), bytes4);
-  if (e == hipSuccess) e = raise_lds_limit(reinterpret_cast<const void *>(&k_rowpass_r<48, true, true>), bytes4);
+  hipError_t e = rowpass_kind_set_lds_limit<kRowVector>(bytes);
+  if (e == hipSuccess) e = rowpass_kind_set_lds_limit<kRowMfma>(bytes4);
+  if (e == hipSuccess) e = rowpass_kind_set_lds_limit<kRowMfmaWide>(bytes4);
   if (e != hipSuccess) return e;
   return raise_lds_limit(reinterpret_cast<const void *>(&k_rowpass_any), bytes);
 }
@@ -1377,17 +1388,41 @@ hipError_t colpass_set_lds_limit(size_t bytes, size_t bytes4) {
   return e;
 }
 
-template <bool MFMA>
+template <int KIND>
 static void launch_rowpass_r(int R, bool split, dim3 grid, dim3 blk, size_t lds_bytes, hipStream_t s, const Bases &b,
                              const MsgJob *jobs, const float *taps, const int *shifts) {
   if (R == 24 && !split)
-    hipLaunchKernelGGL((k_rowpass_r<24, false, MFMA>), grid, blk, lds_bytes, s, b, jobs, taps, shifts);
+    hipLaunchKernelGGL((k_rowpass_r<24, false, KIND>), grid, blk, lds_bytes, s, b, jobs, taps, shifts);
   else if (R == 24)
-    hipLaunchKernelGGL((k_rowpass_r<24, true, MFMA>), grid, blk, lds_bytes, s, b, jobs, taps, shifts);
+    hipLaunchKernelGGL((k_rowpass_r<24, true, KIND>), grid, blk, lds_bytes, s, b, jobs, taps, shifts);
   else if (!split)  // 48: the reference's default grid
-    hipLaunchKernelGGL((k_rowpass_r<48, false, MFMA>), grid, blk, lds_bytes, s, b, jobs, taps, shifts);
+    hipLaunchKernelGGL((k_rowpass_r<48, false, KIND>), grid, blk, lds_bytes, s, b, jobs, taps, shifts);
   else
-    hipLaunchKernelGGL((k_rowpass_r<48, true, MFMA>), grid, blk, lds_bytes, s, b, jobs, taps, shifts);
+    hipLaunchKernelGGL((k_rowpass_r<48, true, KIND>), grid, blk, lds_bytes, s, b, jobs, taps, shifts);
+}
+
+// Whether a launch of `blocks` rows of up to W columns takes its x filter to the
+// matrix cores.  It does where the rows fit, but where that costs blocks per CU
+// (its layout takes 26 floats a column of 24 slices, 24 on the vector unit) or,
+// with more columns than threads, work: 48 slices go through in four groups
+// rather than two, and a column's values are then gathered and exponentiated
+// again for each.  us of all row passes of a sweep of 200-row images (half width
+// 36), vector unit / matrix cores:
+//   24 slices, 8 images: 877 / 757 (W 460, 3 / 2 blocks per CU), 1325 / 1593
+//     (W 760, 2 / 1), 2103 / 1812 (W 800, 1 / 1)
+//   48 slices, 4 images: 1343 / 838 (W 500, a column a thread), 1502 / 1821
+//     (W 600, 2 / 3 blocks per CU), 2873 / 2197 (W 800, 1 / 2), 4268 / 5302
+//     (W 1480, 1 / 1); three columns a thread 4049 / 4154 (W 1400, 1 / 2)
+static bool row_on_mfma(int R, int W, size_t lds, size_t lds4, long long blocks) {
+  if (lds4 == 0) return false;
+  const int waves = std::min(512, (W + 63) / 64 * 64) / 64;
+  // blocks per CU by LDS and by registers (waves of the kernel per CU), and no
+  // more than there are
+  auto per_cu = [&](size_t bytes, int max_waves) {
+    return std::min({(long long)(160 * 1024 / bytes), (long long)(max_waves / waves), (blocks + 255) / 256});
+  };
+  const long long v = per_cu(lds, R == 24 ? 32 : 16), m = per_cu(lds4, R == 24 ? 32 : 24);
+  return R == 24 || W <= 512 ? 2 * m > v : W <= 1024 && m >= 2 * v;
 }
 
 // threads: block size (a multiple of 64; 0 = one thread per column, at most
@@ -1404,10 +1439,12 @@ hipError_t launch_rowpass(const Bases &b, const MsgJob *jobs, int n_jobs, const 
                              : std::min(512, (max_w + 63) / 64 * 64);
   if (!rowpass_fixed(R))
     hipLaunchKernelGGL(k_rowpass_any, grid, dim3(nt), lds_bytes, s, b, jobs, taps, shifts, R);
-  else if (lds4_bytes > 0)
-    launch_rowpass_r<true>(R, split, grid, dim3(nt), lds4_bytes, s, b, jobs, taps, shifts);
+  else if (!row_on_mfma(R, max_w, lds_bytes, lds4_bytes, (long long)max_h * n_jobs))
+    launch_rowpass_r<kRowVector>(R, split, grid, dim3(nt), lds_bytes, s, b, jobs, taps, shifts);
+  else if (max_w > 512)
+    launch_rowpass_r<kRowMfmaWide>(R, split, grid, dim3(nt), lds4_bytes, s, b, jobs, taps, shifts);
   else
-    launch_rowpass_r<false>(R, split, grid, dim3(nt), lds_bytes, s, b, jobs, taps, shifts);
+    launch_rowpass_r<kRowMfma>(R, split, grid, dim3(nt), lds4_bytes, s, b, jobs, taps, shifts);
   return hipGetLastError();
 }
 
