@@ -117,6 +117,7 @@ SIGNATURES = {
                                               ctypes.c_void_p]),
     "ps_plan_tune": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int, ctypes.c_int]),
     "ps_plan_tune_class": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_int]),
+    "ps_plan_tune_default": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int, ctypes.c_int]),
     "ps_plan_classes": (ctypes.c_int, [ctypes.c_void_p, c_int_p, c_int_p, ctypes.c_int]),
     "ps_plan_set_profiling": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int]),
     "ps_plan_set_profiling_classes": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_uint]),

@@ -265,8 +265,12 @@ class Plan:
     TUNE_FP32_COL_ROWS = 3
 
     def tune(self, knob, value, cls=None):
-        """Set a launch-shape knob for every launch class, or for one."""
-        if cls is None:
+        """Set a launch-shape knob for every launch class, or for one (value
+        None: its default, for TUNE_MFMA_ROWS by the launch's size)."""
+        if value is None:
+            check(lib().ps_plan_tune_default(self.handle, knob, -1 if cls is None else int(cls)),
+                  "ps_plan_tune_default")
+        elif cls is None:
             check(lib().ps_plan_tune(self.handle, knob, int(value)), "ps_plan_tune")
         else:
             check(lib().ps_plan_tune_class(self.handle, knob, int(cls), int(value)), "ps_plan_tune_class")
@@ -296,7 +300,8 @@ class Plan:
     def autotune(self, unary, marg, root, maps, method_is_fp32=False, reps=2, stream=None, max_classes=8):
         """Choose the launch shapes of the current method by timing whole
         sweeps on the caller's buffers (HIP events on the execution stream):
-        the BF16 methods' rows per x-pass block (candidates 2, 4, 8, 16); for
+        the BF16 methods' rows per x-pass block (candidates: the default,
+        by the launch's size, and 1, 2, 4, 8, 16); for
         the FP32 method the row pass's threads per block (one per column,
         128, 192, 256), then the column pass's output rows per lane (8, 16).
         Per knob: first one value for every launch class, then class by class
@@ -304,17 +309,22 @@ class Plan:
         sweep with the others fixed; skipped above max_classes classes, where
         it would take more sweeps than it can save).  Sets the choices and
         returns {"knobs": [{"knob": name, "all": {candidate: ms},
-        "per_class": [(class, value, ms)]}], "ms": final ms per sweep}."""
+        "per_class": [(class, value, ms)]}], "ms": final ms per sweep}; the
+        default is named "default"."""
         import torch
         s = stream if stream is not None else torch.cuda.current_stream()
         if method_is_fp32:
             knobs = [(self.TUNE_FP32_ROW_THREADS, "fp32_row_threads", (0, 128, 192, 256)),
                      (self.TUNE_FP32_COL_ROWS, "fp32_col_rows_per_lane", (8, 16))]
         else:
-            knobs = [(self.TUNE_MFMA_ROWS, "mfma_rows_per_block", (2, 4, 8, 16))]
+            knobs = [(self.TUNE_MFMA_ROWS, "mfma_rows_per_block", (None, 1, 2, 4, 8, 16))]
         classes = self.classes()
         out = []
         cur = None
+
+        def label(value):
+            return "default" if value is None else value
+
         for knob, name, cands in knobs:
             times = {}
             for c in cands:
@@ -335,8 +345,8 @@ class Plan:
                         if t < cur:
                             cur, pick = t, c
                     self.tune(knob, pick, cls=k)
-                    per_class.append((k, pick, round(cur, 3)))
-            out.append({"knob": name, "all": {str(k): round(v, 3) for k, v in times.items()},
+                    per_class.append((k, label(pick), round(cur, 3)))
+            out.append({"knob": name, "all": {str(label(k)): round(v, 3) for k, v in times.items()},
                         "per_class": per_class})
         return {"knobs": out, "ms": round(cur, 3)}
 

@@ -1110,6 +1110,20 @@ extern "C" int ps_plan_tune_class(ps_plan *plan, int knob, int cls, int value) {
   return PS_OK;
 }
 
+extern "C" int ps_plan_tune_default(ps_plan *plan, int knob, int cls) {
+  if (!plan) return set_error(PS_ERR_INVALID_ARG, "plan is NULL");
+  if (knob != PS_TUNE_MFMA_ROWS && knob != PS_TUNE_FP32_ROW_THREADS && knob != PS_TUNE_FP32_COL_ROWS)
+    return set_error(PS_ERR_INVALID_ARG, "unknown tuning knob " + std::to_string(knob));
+  std::vector<WidthClass *> v = tune_classes(plan);
+  if (cls < -1 || cls >= (int)v.size()) return set_error(PS_ERR_INVALID_ARG, "no launch class " + std::to_string(cls));
+  drop_graph(plan);
+  if (cls < 0 && knob == PS_TUNE_MFMA_ROWS) plan->mfma_rows = 0;
+  const int value = cls >= 0 && knob == PS_TUNE_MFMA_ROWS ? -1 : 0;
+  for (size_t k = 0; k < v.size(); ++k)
+    if (cls < 0 || (int)k == cls) set_knob(plan, (int)k, *v[k], knob, value);
+  return PS_OK;
+}
+
 extern "C" int ps_plan_classes(const ps_plan *plan, int *n_classes, int *info, int max_classes) {
   if (!plan || !n_classes) return set_error(PS_ERR_INVALID_ARG, "null argument");
   int n = 0, level = 0;
@@ -1215,7 +1229,7 @@ static hipError_t sweep(ps_plan *pl, const Bases &b, int terms, int col_terms, p
       const long ev2 = profile_begin(pp, 2, s);
       if (mf)
         e = launch_rowpass_mfma(b, jobs + c.start, c.count, pl->taps, pl->shifts, pl->frags, pl->R, terms,
-                                c.mfma_rows > 0 ? c.mfma_rows : pl->mfma_rows, c.max_h, c.max_w,
+                                c.mfma_rows != 0 ? std::max(c.mfma_rows, 0) : pl->mfma_rows, c.max_h, c.max_w,
                                 L.mfma_row_lds[ti], c.leaf, s);
       else
         e = launch_rowpass(b, jobs + c.start, c.count, pl->taps, pl->shifts, pl->R, c.max_h, c.max_w, L.lds, L.lds4,
