@@ -365,7 +365,8 @@ int ps_load_joint_mat(const char *path, int flip, ps_joint *out, int *type);
 /* The library keeps up to 1 GiB per device of the memory that destroyed plans
  * and finished calls held, for the next ones (and gives it back by itself when
  * an allocation of its own fails).  This frees what it keeps on the current
- * device.  No reference counterpart. */
+ * device; other allocators cannot reach it before, and it has to be called
+ * before hipDeviceReset.  No reference counterpart. */
 int ps_release_memory(void);
 const char *ps_last_error_string(void);
 const char *ps_version(void);

@@ -44,10 +44,21 @@ inline void check_hip(hipError_t e, const char *where) {
   if (e != hipSuccess) throw std::runtime_error(std::string(where) + ": " + hipGetErrorString(e));
 }
 
+// The memory that the library keeps on the current device between calls, back
+// to the device (ps_release_memory).
+inline void releaseMemory() { check(ps_release_memory(), "ps_release_memory"); }
+
 // RAII device buffer
 struct DeviceBuffer {
   void *p = nullptr;
-  explicit DeviceBuffer(size_t bytes) { check_hip(hipMalloc(&p, bytes ? bytes : 1), "hipMalloc"); }
+  explicit DeviceBuffer(size_t bytes) {
+    hipError_t e = hipMalloc(&p, bytes ? bytes : 1);
+    if (e == hipErrorOutOfMemory && ps_release_memory() == PS_OK) {  // the library keeps up to 1 GiB
+      (void)hipGetLastError();
+      e = hipMalloc(&p, bytes ? bytes : 1);
+    }
+    check_hip(e, "hipMalloc");
+  }
   ~DeviceBuffer() { (void)hipFree(p); }
   DeviceBuffer(const DeviceBuffer &) = delete;
   DeviceBuffer &operator=(const DeviceBuffer &) = delete;

@@ -162,6 +162,13 @@ def _stream_handle(stream):
     return stream.cuda_stream
 
 
+def release_memory():
+    """Give the memory that the library keeps on the current device between
+    calls (up to 1 GiB of what finished calls and closed plans held) back to
+    the device, where torch can allocate it."""
+    check(lib().ps_release_memory(), "ps_release_memory")
+
+
 class Plan:
     """A batch of instances, packed back to back: unary and marginal buffers
     hold [inst][P][S][R][H_i][W_i] floats, the root posterior [inst][S][H_i][W_i]."""
