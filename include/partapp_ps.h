@@ -294,7 +294,7 @@ int ps_find_local_max(const float *grids_dev, const long long *offsets, const in
  * or bilinear gather (TM_BILINEAR), with NO_CLASS_VALUE 0 where nothing
  * lands; then scores < 0 become 1e-4 and the log is taken (0 -> LOG_ZERO).
  * Writes log_unary_dev [n][height][width].  Synchronous.  Allocates device
- * memory only for more than 1440 slices (their warps) and for nearest warps
+ * memory only for more than 80 slices (their warps) and for nearest warps
  * that cannot be inverted or shrink extremely (8 bytes per output cell).
  * A nearest warp may write onto its own input (that too takes 8 bytes per
  * output cell); the buffers of a bilinear one must not overlap. */

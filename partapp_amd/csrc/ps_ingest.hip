@@ -16,6 +16,7 @@
 #include <cmath>
 #include <functional>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/partapp_ps.h"
@@ -91,6 +92,11 @@ struct IngestSlices {
   static constexpr int kMax = 80;  // 48 bytes each, below the 4 KB of kernel arguments
   IngestWarp one[kMax];
 };
+struct IngestTable {
+  const IngestWarp *__restrict__ one;
+};
+template <bool TAB>
+using IngestWarps = std::conditional_t<TAB, IngestTable, IngestSlices>;
 
 constexpr int kTile = 32;                    // output pixels per side of a block
 constexpr int kPix = kTile * kTile / kIngThreads;  // pixels of a thread, kTile / kPix rows apart
@@ -118,63 +124,71 @@ enum IngestMode : int { kIngBilinear = 0, kIngDirect = 1, kIngDirect4 = 2 };
 // reaches 5.2), the rest being vector work on the warp (147 us with every test
 // in double).  The scatter into 64-bit keys took 575 us, with clearing and
 // reading the keys 646 us, and several ms of allocating 172 MB for them.
-template <int MODE>
-__global__ __launch_bounds__(kIngThreads) void k_ingest_tile(const float *__restrict__ grid, IngestSlices sl,
-                                                             const IngestWarp *__restrict__ tab, int first, int gh,
-                                                             int gw, int H, int W, int tile0, int xtiles,
-                                                             float *__restrict__ out) {
+//
+// TAB: the warps come from a table (a choice at run time leaves them in vector
+// registers, and 4 KB of arguments cost a launch a microsecond).  FLAT: 1024 pixels in a row instead of 32 x 32, for slices that
+// fill few such tiles.
+template <int MODE, bool TAB, bool FLAT>
+__global__ __launch_bounds__(kIngThreads) void k_ingest_tile(const float *__restrict__ grid, IngestWarps<TAB> warps,
+                                                             int first, int gh, int gw, int H, int W, int tile0,
+                                                             int xtiles, float *__restrict__ out) {
   unsigned bx, by;
   xcd_block(bx, by);
-  IngestWarp S;  // from the arguments, or from the table where a call has very many slices
-  if (tab) S = tab[by];
-  else S = sl.one[by];
+  double m[6];
+#pragma unroll
+  for (int i = 0; i < 6; ++i) m[i] = warps.one[by].m[i];
   const int s = first + (int)by;
   const int ty = (tile0 + (int)bx) / xtiles;
-  const unsigned x = (unsigned)(tile0 + (int)bx - ty * xtiles) * kTile + (threadIdx.x & 31);
+  const unsigned x0 = (unsigned)(tile0 + (int)bx - ty * xtiles) * kTile + (threadIdx.x & 31);
   const unsigned y0 = (unsigned)ty * kTile + (threadIdx.x >> 5);
-  if (x >= (unsigned)W) return;
+  const unsigned p0 = (unsigned)(tile0 + (int)bx) * (kTile * kTile) + threadIdx.x;
+  if (!FLAT && x0 >= (unsigned)W) return;
+  // pixel k of the thread
+  auto row = [&](int k) { return FLAT ? (p0 + k * kIngThreads) / (unsigned)W : y0 + k * (kTile / kPix); };
+  auto col = [&](int k, unsigned y) { return FLAT ? p0 + k * kIngThreads - y * (unsigned)W : x0; };
   const float *src = grid + (long long)s * gh * gw;
-  float *dst = out + (long long)s * H * W + x;
-  const double m0 = S.m[0], m1 = S.m[1], m2 = S.m[2], m3 = S.m[3], m4 = S.m[4], m5 = S.m[5];
-  const double xd = (double)x;
+  float *dst = out + (long long)s * H * W;
   if (MODE == kIngDirect4) {
-    const CellWarp cell(S.m);
+    const CellWarp cell(m);
     float c[kPix][4];
 #pragma unroll
-    for (int k = 0; k < kPix; ++k) cell.load4((int)x, (int)(y0 + k * (kTile / kPix)), gw, gh, src, gw, c[k]);
+    for (int k = 0; k < kPix; ++k) {
+      const unsigned y = row(k);
+      cell.load4((int)col(k, y), (int)y, gw, gh, src, gw, c[k]);
+    }
 #pragma unroll
     for (int k = 0; k < kPix; ++k) {
-      const unsigned y = y0 + k * (kTile / kPix);
-      if (y < (unsigned)H) dst[(long long)y * W] = clip_log(last_cell(c[k]));
+      const unsigned y = row(k);
+      if (y < (unsigned)H) dst[(long long)y * W + col(k, y)] = clip_log(last_cell(c[k]));
     }
   } else if (MODE == kIngDirect) {
-    const CellWarp cell(S.m);
+    const CellWarp cell(m);
     for (int k = 0; k < kPix; ++k) {
-      const unsigned y = y0 + k * (kTile / kPix);
+      const unsigned y = row(k), x = col(k, y);
       if (y >= (unsigned)H) break;
-      const double yd = (double)y;
+      const double xd = (double)x, yd = (double)y;
       const double cx = cell.a[0] * xd + cell.a[1] * yd + cell.a[2], cy = cell.a[3] * xd + cell.a[4] * yd + cell.a[5];
       const int x_hi = (int)fmin(floor(cx + cell.ex), (double)(gw - 1)), x_lo = (int)fmax(ceil(cx - cell.ex), 0.0);
       const int y_hi = (int)fmin(floor(cy + cell.ey), (double)(gh - 1)), y_lo = (int)fmax(ceil(cy - cell.ey), 0.0);
       float v = 0.0f;
       for (int x1 = x_hi; x1 >= x_lo && v == 0.0f; --x1) {
-        const double p = m0 * (double)x1, q = m3 * (double)x1;
+        const double p = m[0] * (double)x1, q = m[3] * (double)x1;
         for (int y1 = y_hi; y1 >= y_lo; --y1)
           if (cell.lands(p, q, (double)y1, xd, yd)) {
             v = src[(long long)y1 * gw + x1];
             if (v != 0.0f) break;  // NO_CLASS_VALUE is not written
           }
       }
-      dst[(long long)y * W] = clip_log(v);
+      dst[(long long)y * W + x] = clip_log(v);
     }
   } else {
     const float eps10 = 10.0f * FLT_EPSILON;
 #pragma unroll
     for (int k = 0; k < kPix; ++k) {
-      const unsigned y = y0 + k * (kTile / kPix);
+      const unsigned y = row(k), x = col(k, y);
       if (y >= (unsigned)H) break;
-      const double x1 = m0 * xd + m1 * (double)y + m2;
-      const double y1 = m3 * xd + m4 * (double)y + m5;
+      const double x1 = m[0] * (double)x + m[1] * (double)y + m[2];
+      const double y1 = m[3] * (double)x + m[4] * (double)y + m[5];
       const int ix = (int)floor(x1);
       const int iy = (int)floor(y1);
       float r = 0.0f;
@@ -192,7 +206,7 @@ __global__ __launch_bounds__(kIngThreads) void k_ingest_tile(const float *__rest
           r = t0 + t1 + t2 + t3;
         }
       }
-      dst[(long long)y * W] = clip_log(r);
+      dst[(long long)y * W + x] = clip_log(r);
     }
   }
 }
@@ -243,11 +257,9 @@ extern "C" int ps_ingest_scores(const float *score_grid_dev, int n, int grid_hei
   int devcount = 0;
   if (hipGetDeviceCount(&devcount) != hipSuccess || devcount == 0)
     return set_error(PS_ERR_NO_DEVICE, "no HIP device");
-  std::vector<double> mats(6 * (size_t)n);
-  for (int s = 0; s < n; ++s) warp_matrix(Tig + 9 * s, interpolate != 0, mats.data() + 6 * s);
-  hipStream_t st = static_cast<hipStream_t>(stream);
   std::vector<IngestWarp> warps(n);
-  for (int s = 0; s < n; ++s) std::copy(&mats[6 * (size_t)s], &mats[6 * (size_t)s] + 6, warps[s].m);
+  for (int s = 0; s < n; ++s) warp_matrix(Tig + 9 * s, interpolate != 0, warps[s].m);
+  hipStream_t st = static_cast<hipStream_t>(stream);
   // a nearest warp onto its own input (log_unary_dev overlapping the grid) is
   // the scatter's, whose keys hold every value before the first is written
   const float *grid_end = score_grid_dev + (long long)n * grid_height * grid_width;
@@ -261,32 +273,48 @@ extern "C" int ps_ingest_scores(const float *score_grid_dev, int n, int grid_hei
     four = four && f;
   }
   if (gather) {
-    // up to 1440 slices (10 parts x 3 scales x 48 rotations) ride in the
-    // arguments of at most 18 launches; more come from a table
+    // the warps of one launch ride in its arguments, those of more slices come
+    // from a table (in the arguments of several launches, 4 to 6 us each, 1440
+    // slices of 128 x 128 pixels took 152 us sampled and 212 us direct)
     IngestWarp *tab = nullptr;
     hipError_t eg = hipSuccess;
-    if (n > 18 * IngestSlices::kMax) {
+    if (n > IngestSlices::kMax) {
       if (pool_get(&tab, sizeof(IngestWarp) * n) != hipSuccess)
         return set_error(PS_ERR_OUT_OF_MEMORY, "ingest workspace");
       eg = hipMemcpyAsync(tab, warps.data(), sizeof(IngestWarp) * n, hipMemcpyHostToDevice, st);
     }
     const int xtiles = (width + kTile - 1) / kTile, step = tab ? 32768 : IngestSlices::kMax;
-    const long long tiles = (long long)xtiles * ((height + kTile - 1) / kTile);
+    const long long square = (long long)xtiles * ((height + kTile - 1) / kTile);
+    const long long row = ((long long)height * width + kTile * kTile - 1) / (kTile * kTile);
+    // tiles keep a rotated block's cells in its CU's cache, unless a third of
+    // their pixels or more lie outside the slice (2000 slices of 40 x 40 pixels:
+    // 4 of them each, 2 rows)
+    const bool flat = 3 * row <= 2 * square;
+    const long long tiles = flat ? row : square;
     constexpr long long kTiles = 1ll << 22;  // tiles of one launch
     for (int s0 = 0; s0 < n; s0 += step) {
-      IngestSlices sl;
       const int ns = std::min(n - s0, step);
-      if (!tab) std::copy(warps.begin() + s0, warps.begin() + s0 + ns, sl.one);
       for (long long t0 = 0; t0 < tiles && eg == hipSuccess; t0 += kTiles) {
         const dim3 grid((unsigned)std::min(kTiles, tiles - t0), (unsigned)ns), blk(kIngThreads);
-        const IngestWarp *t = tab ? tab + s0 : nullptr;
-        auto launch = [&](auto kernel) {
-          hipLaunchKernelGGL(kernel, grid, blk, 0, st, score_grid_dev, sl, t, s0, grid_height, grid_width, height,
-                             width, (int)t0, xtiles, log_unary_dev);
+        auto launch = [&](auto tabc, auto flatc) {
+          constexpr bool T = decltype(tabc)::value, F = decltype(flatc)::value;
+          IngestWarps<T> w;
+          if constexpr (T) w.one = tab + s0;
+          else std::copy(warps.begin() + s0, warps.begin() + s0 + ns, w.one);
+          auto mode = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, blk, 0, st, score_grid_dev, w, s0, grid_height, grid_width, height, width,
+                               (int)t0, xtiles, log_unary_dev);
+          };
+          if (interpolate) mode(k_ingest_tile<kIngBilinear, T, F>);
+          else if (four) mode(k_ingest_tile<kIngDirect4, T, F>);
+          else mode(k_ingest_tile<kIngDirect, T, F>);
         };
-        if (interpolate) launch(k_ingest_tile<kIngBilinear>);
-        else if (four) launch(k_ingest_tile<kIngDirect4>);
-        else launch(k_ingest_tile<kIngDirect>);
+        const std::true_type yes;
+        const std::false_type no;
+        if (tab && flat) launch(yes, yes);
+        else if (tab) launch(yes, no);
+        else if (flat) launch(no, yes);
+        else launch(no, no);
         eg = hipGetLastError();
       }
     }
@@ -298,13 +326,13 @@ extern "C" int ps_ingest_scores(const float *score_grid_dev, int n, int grid_hei
   // the buffers overlap, or some slice's warp is singular, too ill-conditioned
   // or shrinks too much for the gather: scatter with last-writer keys
   const long long out_n = (long long)n * height * width;
-  const size_t mat_bytes = (mats.size() * sizeof(double) + 255) & ~(size_t)255;
+  const size_t mat_bytes = (sizeof(IngestWarp) * (size_t)n + 255) & ~(size_t)255;
   void *ws = nullptr;
   hipError_t e = pool_get(&ws, mat_bytes + (size_t)out_n * sizeof(unsigned long long));
   if (e != hipSuccess) return set_error(PS_ERR_OUT_OF_MEMORY, "ingest workspace");
   double *mats_dev = static_cast<double *>(ws);
   unsigned long long *keys = reinterpret_cast<unsigned long long *>(static_cast<char *>(ws) + mat_bytes);
-  e = hipMemcpyAsync(mats_dev, mats.data(), mats.size() * sizeof(double), hipMemcpyHostToDevice, st);
+  e = hipMemcpyAsync(mats_dev, warps.data(), sizeof(IngestWarp) * (size_t)n, hipMemcpyHostToDevice, st);
   auto blocks = [](long long m) {
     long long g = (m + kIngThreads - 1) / kIngThreads;
     return (unsigned)(g < 8192 ? (g < 1 ? 1 : g) : 8192);
