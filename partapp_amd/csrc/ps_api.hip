@@ -13,7 +13,6 @@
 #include <cmath>
 #include <cstdint>
 #include <cstring>
-#include <map>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -918,25 +917,6 @@ struct OutsideCapture {
   ~OutsideCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
 };
 
-// A stream of the library's own on the current device, made on first use and
-// kept (making one for a plan's tables took 45 us, forming them 25): a launch
-// on the default stream would join the capture of a stream that waits for it.
-hipError_t own_stream(int device, hipStream_t *s) {
-  static std::mutex mu;
-  static std::map<int, hipStream_t> streams;
-  std::lock_guard<std::mutex> lock(mu);
-  hipStream_t &st = streams[device];
-  if (!st) {
-    const hipError_t e = hipStreamCreateWithFlags(&st, hipStreamNonBlocking);
-    if (e != hipSuccess) {
-      st = nullptr;
-      return e;
-    }
-  }
-  *s = st;
-  return hipSuccess;
-}
-
 // the operand tables of the BF16 passes, complete on return (the plan may be
 // executed on any stream)
 int ensure_fragments(ps_plan *pl) {
@@ -946,10 +926,19 @@ int ensure_fragments(ps_plan *pl) {
   uint4 *f = nullptr;
   if (pool_get(&f, pl->frag_units * 16) != hipSuccess)
     return set_error(PS_ERR_OUT_OF_MEMORY, "fragment tables (" + std::to_string(pl->frag_units * 16) + " bytes)");
-  hipStream_t s = nullptr;
-  hipError_t e = own_stream(pl->device, &s);
-  if (e == hipSuccess) e = launch_fragments(pl->jobs, (int)pl->h_jobs.size(), pl->taps, pl->R, f, s);
-  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  // on the default stream, unless that would join the capture of a stream that
+  // waits for it: then on one of its own (made and destroyed, 45 us; kept, it
+  // takes a hardware queue that the caller's streams would have shared out)
+  hipStream_t own = nullptr;
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  hipError_t e = hipSuccess;
+  if (hipStreamIsCapturing(nullptr, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    e = hipStreamCreateWithFlags(&own, hipStreamNonBlocking);
+  }
+  if (e == hipSuccess) e = launch_fragments(pl->jobs, (int)pl->h_jobs.size(), pl->taps, pl->R, f, own);
+  if (e == hipSuccess) e = hipStreamSynchronize(own);
+  if (own) (void)hipStreamDestroy(own);
   if (e != hipSuccess) {
     pool_put(f, false);
     return hip_error(e, "fragment tables");

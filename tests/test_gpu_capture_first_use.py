@@ -1,7 +1,9 @@
 """The first choice of a BF16 method and the first MAP guard of a plan while a
-stream is being captured (on its thread, and on another): both make tables,
+stream is being captured (on its thread, and on another; a stream that waits for
+the default one, and one that does not): both make tables,
 none of which belongs in the graph, and the graph's replays equal the eager
 sweep."""
+import ctypes
 import threading
 
 import pytest
@@ -24,9 +26,15 @@ def outputs(bufs):
     return [b.clone() for b in bufs[1:]]
 
 
+@pytest.mark.parametrize("blocking", [False, True])
 @pytest.mark.parametrize("what", ["method", "guard", "method in another thread"])
-def test_first_use(gpu, what):
+def test_first_use(gpu, what, blocking):
     import torch
+    stream = None
+    if blocking:  # torch's own streams do not wait for the default one
+        made = ctypes.c_void_p()
+        assert ctypes.CDLL("libamdhip64.so").hipStreamCreate(ctypes.byref(made)) == 0
+        stream = torch.cuda.ExternalStream(made.value)
     ref_plan, ref = setup(gpu)
     ref_plan.set_method("fp32" if what == "guard" else "bf16mix")
     ref_plan.execute(*ref)
@@ -44,7 +52,7 @@ def test_first_use(gpu, what):
 
     x = torch.zeros(8, device=gpu)
     g = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(g):
+    with torch.cuda.graph(g, stream=stream):
         x.add_(1)
         if what.endswith("thread"):
             raised = []
