@@ -102,18 +102,21 @@ __device__ __forceinline__ f32x4_t mfma4(float a, float b, f32x4_t c) {
 // copies' 16-byte units start in different LDS banks (an odd pitch).
 __host__ __device__ __forceinline__ int tap4_chunks(int k) { return (2 * k + 1 + 3 + 3) >> 2; }
 __host__ __device__ __forceinline__ int tap4_pitch(int k) { return 4 * (tap4_chunks(k) | 1); }
-// A thread's first element is loaded ahead, to wait beside the row pass's
-// gather (a launch of 112x128x24: 13.6 -> 12.9 us, of 32 300x300x24: 757 -> 743).
+// A thread takes a tap to its place in the four copies; its first one is loaded
+// ahead, to wait beside the pass's other loads (a launch of 112x128x24: 13.6 ->
+// 12.9 us, of 32 300x300x24: 757 -> 743).
 __device__ __forceinline__ float tap4_load(const float *__restrict__ f, int k) {
-  const int i = (int)threadIdx.x, t = (i >> 2) - (i & 3);
-  return f[min(max(t, 0), 2 * k)];
+  return f[min(max((int)threadIdx.x - 3, 0), 2 * k)];
 }
-__device__ __forceinline__ void tap4_store(float *t4, float first, const float *__restrict__ f, int k) {
+__device__ __forceinline__ void tap4_store(float *t4, float first, const float *__restrict__ f, int k, int nt) {
   const int L = 2 * k + 1, n4 = 4 * tap4_chunks(k), pitch = tap4_pitch(k);
-  for (int i = threadIdx.x; i < 4 * n4; i += blockDim.x) {
-    const int n = i & 3, e = i >> 2, t = e - n;
-    const float v = i == (int)threadIdx.x ? first : f[min(max(t, 0), 2 * k)];
-    t4[n * pitch + e] = t >= 0 && t < L ? v : 0.0f;
+  for (int i = threadIdx.x; i < n4 + 3; i += nt) {
+    const int t = i - 3;
+    float v = i == (int)threadIdx.x ? first : f[min(max(t, 0), 2 * k)];
+    v = t >= 0 && t < L ? v : 0.0f;
+#pragma unroll
+    for (int n = 0; n < 4; ++n)
+      if (t + n >= 0 && t + n < n4) t4[n * pitch + t + n] = v;
   }
 }
 
@@ -240,7 +243,7 @@ __host__ __device__ __forceinline__ size_t row4_lds_bytes(int rg, int W, int k) 
 // four steps' taps serves the S groups of slices.
 template <int RG>
 __device__ __forceinline__ void xfilter4(const float *P, const float *t4, int kx, float *T, int tp, long long plane,
-                                         int y, int W) {
+                                         int y, int W, int nt) {
   static_assert(RG % 4 == 0, "rows in groups of four");
   constexpr int S = RG / 4, Q = row4_pitch(RG);
   constexpr bool kPairs = row4_pairs(RG);
@@ -249,7 +252,7 @@ __device__ __forceinline__ void xfilter4(const float *P, const float *t4, int kx
   const int NT = tap4_chunks(kx), tiles = (W + 63) >> 6;
   char *trow = reinterpret_cast<char *>(T + (long long)y * tp);
   const long long plane_b = plane * 4;
-  for (int j = wave; j < tiles; j += (int)(blockDim.x >> 6)) {
+  for (int j = wave; j < tiles; j += nt >> 6) {
     const float4 *tv = reinterpret_cast<const float4 *>(t4 + m * tap4_pitch(kx));
     const float *d = P + min(64 * j + (lane & ~3), ((W + 3) & ~3) - 4) * Q + (kPairs ? m * S : m);
     f32x4_t acc[S];
@@ -292,16 +295,52 @@ __device__ __forceinline__ void xfilter4(const float *P, const float *t4, int kx
   }
 }
 
-// The same filter of rows holding a non-finite value, one output at a time
-// (the taps padded to a multiple of four with zeros, as the pool holds them).
-__device__ __forceinline__ void xfilter_plain(const float *P, int rg, const float *__restrict__ f, int kx, float *T,
-                                              int tp, long long plane, int y, int W) {
-  const int Lp = (2 * kx + 1 + 3) & ~3;
-  for (int i = threadIdx.x; i < rg * W; i += blockDim.x) {
-    const int r = i / W, x = i - r * W;
-    float a = 0.0f;
-    for (int t = 0; t < Lp; ++t) a = fmaf(P[(x + t) * row4_pitch(rg) + r], f[t], a);
-    T[r * plane + (long long)y * tp + x] = a;
+// Four taps of a filter on the vector unit: acc[i] += win[i + u] f[u], u
+// ascending, the N values of the window and the four behind them, which become
+// its last.
+template <int N>
+__device__ __forceinline__ void plain_taps(float (&acc)[N], float (&win)[N], const float (&behind)[4], const float *f) {
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const float t = f[u];
+#pragma unroll
+    for (int i = 0; i < N; ++i) acc[i] = fmaf(i + u < N ? win[(i + u) % N] : behind[(i + u) % 4], t, acc[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) win[i] = i + 4 < N ? win[(i + 4) % N] : behind[(i + 4) % 4];
+}
+
+// The same filter of rows holding a non-finite value, each output over its own
+// taps (padded to a multiple of four with zeros, as the pool holds them): N
+// outputs of a slice per thread (eight of 24 slices; of 48, whose 48 values a
+// thread holds meanwhile, four: with eight the kernel takes 100 registers
+// instead of 77 and two waves of six per SIMD).
+template <int RG>
+__device__ __forceinline__ void xfilter_plain(const float *P, const float *__restrict__ f, int kx, float *T, int tp,
+                                              long long plane, int y, int W, int nt) {
+  constexpr int Q = row4_pitch(RG), N = RG == 24 ? 8 : 4;
+  const int Lp = (2 * kx + 1 + 3) & ~3, last = row4_len(W, kx) - 1;
+  for (int i = threadIdx.x; i < RG * ((W + N - 1) / N); i += nt) {
+    const int q = i / RG, r = i - q * RG;
+    int pos = N * q;
+    // (past the layout: its last position, for outputs past the row)
+    auto next = [&] { return P[min(pos++, last) * Q + r]; };
+    float a[N], win[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      a[j] = 0.0f;
+      win[j] = next();
+    }
+    for (int t = 0; t < Lp; t += 4) {
+      float behind[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) behind[j] = next();
+      plain_taps<N>(a, win, behind, f + t);
+    }
+    float *o = T + r * plane + (long long)y * tp + N * q;
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+      if (N * q + j < W) o[j] = a[j];
   }
 }
 
@@ -564,7 +603,7 @@ enum RowKind : int { kRowVector = 0, kRowMfma = 1, kRowMfmaWide = 2 };
 
 template <int R, bool SPLIT, int KIND>
 __device__ __forceinline__ void rowpass_body(const Bases &b, const MsgJob &J, const float *__restrict__ taps,
-                                             const int *__restrict__ shifts, float *P, int y) {
+                                             const int *__restrict__ shifts, float *P, int y, int nt) {
   const int H = J.H, W = J.W;
   const int kx = J.kx;
   const RowGeom g = row_geom(W, kx);
@@ -576,8 +615,8 @@ __device__ __forceinline__ void rowpass_body(const Bases &b, const MsgJob &J, co
     // zeros before the row and as far behind it as a window reaches whose
     // first output is inside
     const int tail = (kx + W) * Q, end = (W + 4 * tap4_chunks(kx)) * Q;
-    for (int i = threadIdx.x; i < kx * Q; i += blockDim.x) P[i] = 0.0f;
-    for (int i = tail + (int)threadIdx.x; i < end; i += blockDim.x) P[i] = 0.0f;
+    for (int i = threadIdx.x; i < kx * Q; i += nt) P[i] = 0.0f;
+    for (int i = tail + (int)threadIdx.x; i < end; i += nt) P[i] = 0.0f;
     if (threadIdx.x == 0) *bad = 0u;
   } else {
     zero_halo(P, RG, W, kx, g.Pw);
@@ -590,7 +629,7 @@ __device__ __forceinline__ void rowpass_body(const Bases &b, const MsgJob &J, co
   const float *src = cptr(b, J.src);
   float *T = mptr(b, J.tmp);
   const long long plane = (long long)H * J.tpitch;
-  const bool one = MFMA && W <= (int)blockDim.x;
+  const bool one = MFMA && W <= nt;
   const float tap0 = MFMA ? tap4_load(taps + J.taps_x, kx) : 0.0f;
   float e[R];
   unsigned bits = 0u;
@@ -606,7 +645,7 @@ __device__ __forceinline__ void rowpass_body(const Bases &b, const MsgJob &J, co
   auto group = [&](auto gc) {
     constexpr int G = decltype(gc)::value;
     if (G > 0) __syncthreads();  // every item of the group before is filtered
-    for (int x0 = 0; x0 < W; x0 += (int)blockDim.x) {
+    for (int x0 = 0; x0 < W; x0 += nt) {
       const int x = x0 + (int)threadIdx.x;
       if (KIND != kRowMfma && __builtin_amdgcn_readfirstlane(x) >= W) break;
       if (!one || G == 0) values(min(x, W - 1));  // past the row: its last column again
@@ -616,15 +655,15 @@ __device__ __forceinline__ void rowpass_body(const Bases &b, const MsgJob &J, co
       }
     }
     if (MFMA && G == 0) {
-      tap4_store(t4, tap0, taps + J.taps_x, kx);
+      tap4_store(t4, tap0, taps + J.taps_x, kx, nt);
       __syncthreads();  // the flag is clear
     }
     if (MFMA && bits >= kRowNonFinite) *bad = 1u;
     __syncthreads();
     float *Tg = T + G * RG * plane;
     if (!MFMA) xfilter_rows(P, taps + J.taps_x, Tg, RG, J.tpitch, plane, y, g);
-    else if (__builtin_amdgcn_readfirstlane(*bad) == 0u) xfilter4<RG>(P, t4, kx, Tg, J.tpitch, plane, y, W);
-    else xfilter_plain(P, RG, taps + J.taps_x, kx, Tg, J.tpitch, plane, y, W);
+    else if (__builtin_amdgcn_readfirstlane(*bad) == 0u) xfilter4<RG>(P, t4, kx, Tg, J.tpitch, plane, y, W, nt);
+    else xfilter_plain<RG>(P, taps + J.taps_x, kx, Tg, J.tpitch, plane, y, W, nt);
   };
   group(std::integral_constant<int, 0>{});
   if constexpr (NG > 1) group(std::integral_constant<int, 1>{});
@@ -634,11 +673,17 @@ __device__ __forceinline__ void rowpass_body(const Bases &b, const MsgJob &J, co
   }
 }
 
+// 24 slices on the matrix cores: at most 96 scalar registers, which the register
+// count that seven waves a SIMD allow comes to.  More are allotted as 112, for
+// seven waves instead of eight, and the first SIMD of a CU then takes no fourth
+// block of five waves, two of which each block puts there: 2703 instead of 2835
+// us of all row passes of 32 images of 300x300.
 template <int R, bool SPLIT, int KIND>
-__global__ __launch_bounds__(512) void k_rowpass_r(Bases b, const MsgJob *__restrict__ jobs,
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(R == 24 && KIND != kRowVector ? 7 : 2))) void k_rowpass_r(Bases b, const MsgJob *__restrict__ jobs,
                                                    const float *__restrict__ taps, const int *__restrict__ shifts) {
   extern __shared__ float4 lds4[];
   float *P = reinterpret_cast<float *>(lds4);
+  const int nt = (int)blockDim.x;
   unsigned bx, by;
   xcd_block(bx, by);
   const MsgJob &J = jobs[by];
@@ -646,8 +691,8 @@ __global__ __launch_bounds__(512) void k_rowpass_r(Bases b, const MsgJob *__rest
   const int y = (int)bx;
   if (y >= J.H) return;
   // a warp whose offset changes along an axis takes the SPLIT variants
-  if (SPLIT && J.split != 0) rowpass_body<R, SPLIT, KIND>(b, J, taps, shifts, P, y);
-  else rowpass_body<R, false, KIND>(b, J, taps, shifts, P, y);
+  if (SPLIT && J.split != 0) rowpass_body<R, SPLIT, KIND>(b, J, taps, shifts, P, y, nt);
+  else rowpass_body<R, false, KIND>(b, J, taps, shifts, P, y, nt);
 }
 
 // Row pass for any rotation count: the exponentiated column goes through an
@@ -824,6 +869,28 @@ __device__ __forceinline__ void yfilter4(const float *col, int row, int n, const
   for (int i = 0; i < ROWS; ++i) a[i] = acc[i >> 2][i & 3];
 }
 
+// The same of a tile holding a non-finite value, each row over its own taps
+// (padded to a multiple of four, Lp, with zeros).
+template <int ROWS>
+__device__ __forceinline__ void yfilter_plain(const float *col, int row, int n, const float *__restrict__ fy, int Lp,
+                                              float (&a)[ROWS]) {
+  auto next = [&] {
+    const float v = col[row * kColTileX];
+    if (++row == n) row = 0;
+    return v;
+  };
+  float win[ROWS];
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i) win[i] = next();
+#pragma unroll 2
+  for (int t = 0; t < Lp; t += 4) {
+    float behind[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) behind[j] = next();
+    plain_taps<ROWS>(a, win, behind, fy + t);
+  }
+}
+
 // The caller's accumulation is a template (EPI, one variant per destination
 // kind), so every load of a tile is unconditional straight-line code: the
 // epilogue operands first, then the next tile's rows (always loaded, clamped
@@ -862,12 +929,12 @@ __device__ __forceinline__ void colpass_strip(const Bases &b, const MsgJob &J, c
   const int nrows = col_tile_rows(ky, ROWS);
   const float *fy = taps + J.taps_y;
   // MFMA: the tap operand and a flag (a non-finite value was staged: the
-  // strip goes on a tap at a time) behind the tile
+  // strip goes on on the vector unit) behind the tile
   float *t4 = tile + nrows * kColTileX;
   unsigned *bad = reinterpret_cast<unsigned *>(t4 + 4 * tap4_pitch(ky));
   unsigned bits = 0u;
   if (MFMA) {
-    tap4_store(t4, tap4_load(fy, ky), fy, ky);
+    tap4_store(t4, tap4_load(fy, ky), fy, ky, kColWaves * 64);
     if (threadIdx.x == 0) *bad = 0u;
     __syncthreads();
   }
@@ -956,16 +1023,7 @@ __device__ __forceinline__ void colpass_strip(const Bases &b, const MsgJob &J, c
       if (MFMA && __builtin_amdgcn_readfirstlane(*bad) == 0u) {
         yfilter4<ROWS>(tile + lane, row0, nrows, t4, ky, a);
       } else if (MFMA) {
-        for (int i = 0; i < kColRows; ++i) {
-          float v = 0.0f;
-          for (int t = 0; t < Lp; ++t) {
-            int rr = row0 + i + t;
-            if (rr >= nrows) rr -= nrows;
-            v = fmaf(tile[rr * kColTileX + lane], fy[t], v);
-          }
-#pragma unroll
-          for (int j = 0; j < kColRows; ++j) a[j] = j == i ? v : a[j];
-        }
+        yfilter_plain<ROWS>(tile + lane, row0, nrows, fy, Lp, a);
       } else {
         float buf[kColRows];
 #pragma unroll
@@ -1413,8 +1471,10 @@ static void launch_rowpass_r(int R, bool split, dim3 grid, dim3 blk, size_t lds_
 //   48 slices, 4 images: 1343 / 838 (W 500, a column a thread), 1502 / 1821
 //     (W 600, 2 / 3 blocks per CU), 2873 / 2197 (W 800, 1 / 2), 4268 / 5302
 //     (W 1480, 1 / 1); three columns a thread 4049 / 4154 (W 1400, 1 / 2)
+// Of rows of up to 16 columns a wave's tile of 64 is mostly empty (24 slices, 16
+// images 300 rows high: 291 / 321 us at W 16, 293 / 285 at W 20).
 static bool row_on_mfma(int R, int W, size_t lds, size_t lds4, long long blocks) {
-  if (lds4 == 0) return false;
+  if (lds4 == 0 || (R == 24 && W <= 16)) return false;
   const int waves = std::min(512, (W + 63) / 64 * 64) / 64;
   // blocks per CU by LDS and by registers (waves of the kernel per CU), and no
   // more than there are
@@ -1495,7 +1555,11 @@ hipError_t launch_colpass(const Bases &b, const MsgJob *jobs, int n_jobs, const 
   if (rows == 0 || split) rows = kColRowsDefault;
   if (epi_hi < kEpiUpRoot || epi_hi > kEpiDownMid || (rows != 8 && rows != 16)) return hipErrorInvalidValue;
   const int xtiles = (max_w + kColTileX - 1) / kColTileX;
-  const int tile_y = kColWaves * rows;
+  // few rows of a tile to filter do not pay for the tap operand (us of all column
+  // passes of 16 images of 300 columns x 24, half width 9, vector unit / matrix
+  // cores: 107 / 115 at 4 rows, 121 / 122 at 12)
+  if (max_h <= 12) lds4_bytes_16 = 0;
+  const int tile_y = kColWaves * (lds4_bytes_16 == 0 ? kColRowsDefault : rows);
   dim3 grid(R * xtiles, n_jobs, col_parts(R * xtiles * n_jobs, (max_h + tile_y - 1) / tile_y));
   const size_t less = sizeof(float) * kColWaves * 8 * kColTileX;
   if (lds4_bytes_16 == 0 && split)

@@ -1,6 +1,7 @@
-"""The FP32 row pass's three routes around the rule that chooses between them
-(blocks per CU, columns per thread) and where waves lie past the row: single
-messages against the float32 oracle, at its bar for messages."""
+"""The routes of the FP32 row and column pass around the rules that choose
+between them (blocks per CU, columns per thread, narrow and short grids) and
+where waves lie past the row: single messages against the float32 oracle, at its
+bar for messages."""
 import numpy as np
 import pytest
 
@@ -17,6 +18,7 @@ pytestmark = pytest.mark.gpu
     (24, 260, 690), (24, 260, 730), (24, 250, 730), (24, 260, 810),  # matrix cores, vector, too few blocks, matrix cores
     (48, 5, 512), (48, 5, 513), (48, 5, 640), (48, 5, 1025),      # matrix cores, vector
     (48, 260, 810), (48, 260, 1024), (48, 260, 1030),             # matrix cores, matrix cores, vector
+    (24, 40, 16), (24, 40, 17), (24, 12, 100), (24, 13, 100),     # narrow rows, and a column pass of few rows, vector
 ])
 def test_routes(gpu, R, H, W):
     import torch
