@@ -273,7 +273,7 @@ int ps_message_noalloc(const ps_model *model, const float *child_dev, float *par
  * grid: in scan order (d, then x, then y) when there are at most max_n,
  * otherwise the max_n largest by value, in decreasing order (ties in scan
  * order).  out_dev: [n_grids][max_n] records, count_dev: [n_grids].
- * max_n <= 4096.  Allocates a workspace (88 KB per grid and a bit per point,
+ * max_n <= 4096.  Allocates a workspace (112 KB per grid and a bit per point,
  * each row rounded up to 64; for 1024 grids at a time); synchronous.
  * Feeds best_part_hyp (objectdetect_findrot.cpp:280-283) and the root
  * HypothesisList (:1037-1048). */

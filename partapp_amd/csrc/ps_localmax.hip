@@ -15,13 +15,13 @@
 //                   when there are at most max_n)
 //   k_lmax_select   one workgroup per grid sorts those few in LDS
 // Where some grid has more of those keys than LDS takes (k_lmax_select tells
-// the host), all of it runs again with a third histogram (the last 10 bits);
-// where too many values equal that threshold, k_lmax_collect takes the keys
-// above it and k_lmax_select the first of the equal ones in the scan.
-// Grids near LOG_ZERO do it (the bin spans 64 units of value there) and plateaus.
-// Selected by one workgroup from every mark, byte by byte, such a grid of
-// 24 x 300 x 300 took 7.6 ms, now 0.67 (0.18 without the second run), a
-// plateau of 1000 x 1000 6.2 and now 3.0 ms.
+// the host), it goes on with a third histogram (the last 10 bits) and, where too
+// many values equal that threshold, with three more of their scan indices, and
+// collects again.
+// Grids near LOG_ZERO do it (the bin spans 64 units of value there), grids of few
+// distinct values, plateaus.  Selected by one workgroup from every mark, byte by
+// byte, such a grid of 24 x 300 x 300 took 7.6 ms, now 0.62 (0.17 without the second
+// part), a plateau of 1000 x 1000 6.2 and now 0.40 ms.
 // key = (order key of value) << 32 | (2^32-1 - scan index): distinct, so the
 // result does not depend on the order in which the keys were collected.
 //
@@ -67,15 +67,19 @@ constexpr int kCap = 8192;      // keys collected per grid (64 KB, sorted in LDS
 constexpr int kMarkRows = 16;   // rows of a wave's 64-column tile
 constexpr int kTabGrids = 1024; // grids of one set of launches that reads a table
 
-// per grid: the histograms, the marked points and the collected keys; the second
-// run's: whether the third histogram is needed, the 32-bit threshold where only
-// values above it are collected (tie)
+// per grid: the histograms of the first part, the marked points and the
+// collected keys; from the second part's kernels the 22-bit threshold, the 32-bit
+// one and the leading bits of the scan threshold, each with the max_n-th largest's
+// place in its bin, and whether they were needed; its histograms
 struct LmState {
-  unsigned hist[3][kBins];
-  unsigned marked, collected;
-  unsigned third, tie, tie_key;
-  unsigned pad_[59];
+  unsigned hist[2][kBins];
+  unsigned marked;
+  unsigned collected, third, thr22, need2, tie, thr32, need3, scan11, need4, scan22, need5;
+  unsigned pad_[52];
+  unsigned more[4][kBins];
 };
+constexpr int kStateWords = sizeof(LmState) / 4, kFirstWords = 2 * kBins + 64;  // the first part clears those
+constexpr int kSecondFrom = 2 * kBins + 1;                                     // the second part from there on
 
 __device__ __forceinline__ unsigned okey(float f) {
   unsigned u = __float_as_uint(f);
@@ -86,9 +90,11 @@ __device__ __forceinline__ float okey_inv(unsigned k) {
   return __uint_as_float(u);
 }
 
-__global__ __launch_bounds__(256) void k_lmax_clear(unsigned *__restrict__ p, long long n) {
+// words [from, to) of each of n states
+__global__ __launch_bounds__(256) void k_lmax_clear(LmState *__restrict__ st, int n, int from, int to) {
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0u;
+  const int per = to - from, g = (int)(i / per);
+  if (g < n) reinterpret_cast<unsigned *>(st + g)[from + (int)(i - (long long)g * per)] = 0u;
 }
 
 // grid i of a launch: from the arguments, or (TAB) from the table.  Two
@@ -255,7 +261,9 @@ __device__ __forceinline__ void lm_marked(const float *__restrict__ grids, const
   }
 }
 
-// DIGIT 1: the next 11 bits, 2: the last 10.
+// One more histogram, of the values (DIGIT 1: bits 20 to 10, 2: 9 to 0) or, of
+// values equal to the threshold, of 2^32-1 - scan (3: bits 31 to 21, 4: 20 to 10,
+// 5: 9 to 0) whose leading bits are those that hold the max_n-th largest.
 template <int DIGIT, bool TAB>
 __global__ __launch_bounds__(256) void k_lmax_refine(const float *__restrict__ grids, LmBatch gd,
                                                      const LmGrid *__restrict__ tab,
@@ -263,32 +271,56 @@ __global__ __launch_bounds__(256) void k_lmax_refine(const float *__restrict__ g
                                                      LmState *__restrict__ st, int max_n) {
   __shared__ unsigned hist[kBins], part[4];
   LmState &S = st[blockIdx.y];
-  if (S.marked <= (unsigned)max_n) return;
-  unsigned need = (unsigned)max_n;
-  unsigned top = (unsigned)lm_bin(S.hist[0], need, part);  // the leading bits of the values counted
-  if (DIGIT == 2) {
-    const unsigned b = (unsigned)lm_bin(S.hist[1], need, part);
-    top = top << 11 | b;
-    // the keys at or above the 22-bit threshold
-    const bool third = (unsigned)max_n - need + S.hist[1][b] > (unsigned)kCap;
-    if (blockIdx.x == 0 && threadIdx.x == 0) S.third = third;
-    if (!third) return;
+  const bool first = blockIdx.x == 0 && threadIdx.x == 0;
+  unsigned top, v0 = 0u;  // leading bits of what is counted; of what value
+  if (DIGIT <= 2) {
+    if (S.marked <= (unsigned)max_n) return;
+    unsigned need = (unsigned)max_n;
+    top = (unsigned)lm_bin(S.hist[0], need, part);
+    if (DIGIT == 2) {
+      const unsigned b = (unsigned)lm_bin(S.hist[1], need, part);
+      top = top << 11 | b;
+      // the keys at or above the 22-bit threshold
+      const bool third = (unsigned)max_n - need + S.hist[1][b] > (unsigned)kCap;
+      if (first) S.third = third, S.thr22 = top, S.need2 = need;
+      if (!third) return;
+    }
+  } else if (DIGIT == 3) {
+    if (!S.third) return;
+    unsigned need = S.need2;
+    const unsigned b = (unsigned)lm_bin(S.more[0], need, part);
+    const bool tie = (unsigned)max_n - need + S.more[0][b] > (unsigned)kCap;
+    v0 = S.thr22 << 10 | b;
+    if (first) S.tie = tie, S.thr32 = v0, S.need3 = need;
+    if (!tie) return;
+    top = 0u;
+  } else {
+    if (!S.tie) return;
+    v0 = S.thr32;
+    unsigned need = DIGIT == 4 ? S.need3 : S.need4;
+    const unsigned b = (unsigned)lm_bin(S.more[DIGIT - 3], need, part);
+    top = DIGIT == 4 ? b : S.scan11 << 11 | b;
+    if (first && DIGIT == 4) S.scan11 = top, S.need4 = need;
+    if (first && DIGIT == 5) S.scan22 = top, S.need5 = need;
   }
-  constexpr int kShift = DIGIT == 1 ? 10 : 0, kTop = DIGIT == 1 ? 21 : 10;
+  constexpr int kShift = DIGIT == 1 || DIGIT == 4 ? 10 : DIGIT == 3 ? 21 : 0;
+  constexpr int kBits = DIGIT == 2 || DIGIT == 5 ? 10 : 11;
   for (int i = threadIdx.x; i < kBins; i += 256) hist[i] = 0u;
   __syncthreads();
   const LmGrid &G = lm_grid<TAB>(gd, tab, blockIdx.y);
   const unsigned wave = (unsigned)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  lm_marked(grids, G, mask, blockIdx.x * 4 + wave, gridDim.x * 4, [&](bool on, float v, int, int, int) {
-    const unsigned k = okey(v);
-    if (on && (k >> kTop) == top) atomicAdd(&hist[(k >> kShift) & ((1u << (kTop - kShift)) - 1u)], 1u);
+  lm_marked(grids, G, mask, blockIdx.x * 4 + wave, gridDim.x * 4, [&](bool on, float v, int d, int y, int x) {
+    const unsigned k = DIGIT <= 2 ? okey(v) : (unsigned)lm_key(G, v, d, y, x);
+    const bool in = on && (DIGIT <= 2 || okey(v) == v0) && (DIGIT == 3 || (k >> (kShift + kBits) % 32) == top);
+    if (in) atomicAdd(&hist[(k >> kShift) & ((1u << kBits) - 1u)], 1u);
   });
   __syncthreads();
+  unsigned *h = DIGIT == 1 ? S.hist[1] : S.more[DIGIT - (DIGIT == 1 ? 1 : 2)];
   for (int i = threadIdx.x; i < kBins; i += 256)
-    if (hist[i]) atomicAdd(&S.hist[DIGIT][i], hist[i]);
+    if (hist[i]) atomicAdd(h + i, hist[i]);
 }
 
-template <bool TAB>
+template <bool SECOND, bool TAB>
 __global__ __launch_bounds__(256) void k_lmax_collect(const float *__restrict__ grids, LmBatch gd,
                                                       const LmGrid *__restrict__ tab,
                                                       const unsigned long long *__restrict__ mask,
@@ -297,30 +329,28 @@ __global__ __launch_bounds__(256) void k_lmax_collect(const float *__restrict__ 
   __shared__ unsigned part[4];
   LmState &S = st[blockIdx.y];
   const LmGrid &G = lm_grid<TAB>(gd, tab, blockIdx.y);
-  unsigned thr = 0u;  // least value key that is collected
-  const unsigned marked = S.marked, third = S.third;
-  if (marked > (unsigned)max_n) {
+  unsigned thr = 0u, thr_scan = 0u;  // least value key that is collected; of its ties the least 2^32-1 - scan
+  const unsigned marked = S.marked;
+  bool tie = false;
+  if (SECOND && S.third) {
+    tie = S.tie != 0u;
+    thr = S.thr32;
+    if (tie) {
+      unsigned need = S.need5;
+      thr_scan = S.scan22 << 10 | (unsigned)lm_bin(S.more[3], need, part);
+    }
+  } else if (marked > (unsigned)max_n) {
     unsigned need = (unsigned)max_n;
     const unsigned b1 = (unsigned)lm_bin(S.hist[0], need, part);
     const unsigned b2 = (unsigned)lm_bin(S.hist[1], need, part);
     thr = b1 << 21 | b2 << 10;
-    if (third) {
-      const unsigned b3 = (unsigned)lm_bin(S.hist[2], need, part);
-      thr |= b3;
-      if ((unsigned)max_n - need + S.hist[2][b3] > (unsigned)kCap) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-          S.tie = 1u;
-          S.tie_key = thr;
-        }
-        if (++thr == 0u) return;  // only what lies above: nothing does
-      }
-    }
   }
   unsigned long long *out = keys + (long long)blockIdx.y * kCap;
   const int lane = threadIdx.x & 63;
   const unsigned wave = (unsigned)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   lm_marked(grids, G, mask, blockIdx.x * 4 + wave, gridDim.x * 4, [&](bool on, float v, int d, int y, int x) {
-    const bool take = on && okey(v) >= thr;
+    bool take = on && okey(v) >= thr;
+    if (SECOND && tie) take = take && (okey(v) > thr || (unsigned)lm_key(G, v, d, y, x) >= thr_scan);
     const unsigned long long w = __ballot(take);
     if (w == 0ull) return;
     unsigned at = 0u;
@@ -350,80 +380,9 @@ __device__ void bitonic_desc(unsigned long long *s, int n) {
 
 __device__ __forceinline__ unsigned long long swap_halves(unsigned long long k) { return (k << 32) | (k >> 32); }
 
-template <bool TAB>
-__global__ __launch_bounds__(kSelThreads) void k_lmax_select(const float *__restrict__ grids, LmBatch gd,
-                                                             const LmGrid *__restrict__ tab,
-                                                             const unsigned long long *__restrict__ mask,
-                                                             const LmState *__restrict__ st,
-                                                             const unsigned long long *__restrict__ keys, int max_n,
-                                                             ps_local_max *__restrict__ out, int *__restrict__ out_n,
-                                                             unsigned *more_host) {
-  __shared__ unsigned long long s[kCap];
-  __shared__ unsigned hist[256];
-  __shared__ unsigned prefix_s, need_s, fill_s;
-  const LmGrid &G = lm_grid<TAB>(gd, tab, blockIdx.x);
-  const LmState &S = st[blockIdx.x];
-  const unsigned long long *c = keys + (long long)blockIdx.x * kCap;
-  const unsigned marked = S.marked, n = S.collected;
-  const int keep = (int)min(marked, (unsigned)max_n);
-  if (n > (unsigned)kCap) {  // the first run only
-    if (threadIdx.x == 0) __hip_atomic_store(more_host, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    return;
-  }
-  const bool tie = S.tie != 0u;
-  // all of them in scan order (by 2^32-1 - scan descending), or the largest
-  const bool all = marked <= (unsigned)max_n;
-  const int size = tie ? keep : (int)n;
-  int n2 = 1;
-  while (n2 < size) n2 <<= 1;
-  for (int i = threadIdx.x; i < n2; i += blockDim.x) s[i] = i < (int)n ? (all ? swap_halves(c[i]) : c[i]) : 0ull;
-  if (tie) {
-    // fewer than max_n values above the threshold, more than LDS holds equal
-    // to it: radix select of the first in the scan, the most significant byte
-    // of 2^32-1 - scan first
-    const unsigned v0 = S.tie_key;
-    if (threadIdx.x == 0) {
-      prefix_s = 0u;
-      need_s = (unsigned)max_n - n;
-      fill_s = n;
-    }
-    const unsigned wave = (unsigned)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    unsigned m = 0u;
-    for (int shift = 24; shift >= 0; shift -= 8) {
-      if (threadIdx.x < 256) hist[threadIdx.x] = 0u;
-      __syncthreads();
-      const unsigned prefix = prefix_s;
-      lm_marked(grids, G, mask, wave, kSelThreads / 64, [&](bool on, float v, int d, int y, int x) {
-        const unsigned k = (unsigned)lm_key(G, v, d, y, x);
-        if (on && okey(v) == v0 && (k & m) == prefix) atomicAdd(&hist[(k >> shift) & 255u], 1u);
-      });
-      __syncthreads();
-      if (threadIdx.x == 0) {
-        unsigned need = need_s, acc = 0u;
-        int bin = 255;
-        for (; bin > 0; --bin) {
-          if (acc + hist[bin] >= need) break;
-          acc += hist[bin];
-        }
-        need_s = need - acc;
-        prefix_s = prefix | ((unsigned)bin << shift);
-      }
-      m |= 0xffu << shift;
-      __syncthreads();
-    }
-    // scan indices are distinct: exactly max_n - n of them are >= the selected one
-    const unsigned thr = prefix_s;
-    lm_marked(grids, G, mask, wave, kSelThreads / 64, [&](bool on, float v, int d, int y, int x) {
-      const unsigned long long k = lm_key(G, v, d, y, x);
-      if (on && okey(v) == v0 && (unsigned)k >= thr) s[atomicAdd(&fill_s, 1u)] = k;
-    });
-  }
-  bitonic_desc(s, n2);
-  if (all) {
-    for (int i = threadIdx.x; i < keep; i += blockDim.x) s[i] = swap_halves(s[i]);
-    __syncthreads();
-  }
-  ps_local_max *o = out + (long long)blockIdx.x * max_n;
+// the first `keep` keys of s as records; every thread of the block calls it
+__device__ __forceinline__ void lm_write(const LmGrid &G, const unsigned long long *s, int keep,
+                                         ps_local_max *__restrict__ o, int *__restrict__ o_n) {
   for (int i = threadIdx.x; i < keep; i += blockDim.x) {
     const unsigned long long k = s[i];
     const unsigned scan = 0xffffffffu - (unsigned)(k & 0xffffffffull);
@@ -436,7 +395,36 @@ __global__ __launch_bounds__(kSelThreads) void k_lmax_select(const float *__rest
     r.score = okey_inv((unsigned)(k >> 32));
     o[i] = r;
   }
-  if (threadIdx.x == 0) out_n[blockIdx.x] = keep;
+  if (threadIdx.x == 0) *o_n = keep;
+}
+
+template <bool TAB>
+__global__ __launch_bounds__(kSelThreads) void k_lmax_select(LmBatch gd, const LmGrid *__restrict__ tab,
+                                                             const LmState *__restrict__ st,
+                                                             const unsigned long long *__restrict__ keys, int max_n,
+                                                             ps_local_max *__restrict__ out, int *__restrict__ out_n,
+                                                             unsigned *more_host) {
+  __shared__ unsigned long long s[kCap];
+  const LmGrid &G = lm_grid<TAB>(gd, tab, blockIdx.x);
+  const LmState &S = st[blockIdx.x];
+  const unsigned long long *c = keys + (long long)blockIdx.x * kCap;
+  const unsigned marked = S.marked, n = S.collected;
+  const int keep = (int)min(marked, (unsigned)max_n);
+  if (n > (unsigned)kCap) {  // the first part only
+    if (threadIdx.x == 0) __hip_atomic_store(more_host, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    return;
+  }
+  // all of them in scan order (by 2^32-1 - scan descending), or the largest
+  const bool all = marked <= (unsigned)max_n;
+  int n2 = 1;
+  while (n2 < (int)n) n2 <<= 1;
+  for (int i = threadIdx.x; i < n2; i += blockDim.x) s[i] = i < (int)n ? (all ? swap_halves(c[i]) : c[i]) : 0ull;
+  bitonic_desc(s, n2);
+  if (all) {
+    for (int i = threadIdx.x; i < keep; i += blockDim.x) s[i] = swap_halves(s[i]);
+    __syncthreads();
+  }
+  lm_write(G, s, keep, out + (long long)blockIdx.x * max_n, out_n + blockIdx.x);
 }
 
 }  // namespace
@@ -490,7 +478,7 @@ extern "C" int ps_find_local_max(const float *grids_dev, const long long *offset
   if (e == hipSuccess) *more = 0u;
   if (table && e == hipSuccess)
     e = hipMemcpyAsync(tab, gd.data(), sizeof(LmGrid) * (size_t)n_grids, hipMemcpyHostToDevice, s);
-  for (const bool third : {false, true}) {
+  for (const bool second : {false, true}) {
     for (int g0 = 0; g0 < n_grids && e == hipSuccess; g0 += step) {
       const int n = std::min(n_grids - g0, step);
       const LmGrid *one = gd.data() + g0, *t = table ? tab + g0 : nullptr;
@@ -501,23 +489,37 @@ extern "C" int ps_find_local_max(const float *grids_dev, const long long *offset
         tiles = std::max(tiles, (long long)one[i].D * ((one[i].H + kMarkRows - 1) / kMarkRows) * one[i].wq);
         most = std::max(most, (long long)one[i].D * one[i].H * one[i].wq);
       }
-      // counters cleared by a small kernel (this entry point synchronizes and is
-      // not capturable)
-      const long long n_state = (long long)(sizeof(LmState) / sizeof(unsigned)) * n;
-      hipLaunchKernelGGL(k_lmax_clear, dim3((unsigned)((n_state + 255) / 256)), dim3(256), 0, s,
-                         reinterpret_cast<unsigned *>(st), n_state);
+      // cleared by a small kernel (this entry point synchronizes and is not
+      // capturable)
+      auto clear = [&](int from, int to) {
+        const long long words = (long long)n * (to - from);
+        hipLaunchKernelGGL(k_lmax_clear, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, s, st, n, from, to);
+      };
       const dim3 blk(256);
       // the marked points again: 8 words per wave and turn, at most 128 blocks a grid
       const dim3 again((unsigned)std::min<long long>(128, (most + 31) / 32), (unsigned)n);
       const dim3 mark((unsigned)std::min<long long>(1 << 20, (tiles + 3) / 4), (unsigned)n);
       auto launch = [&](auto tabc) {
         constexpr bool T = decltype(tabc)::value;
-        hipLaunchKernelGGL((k_lmax_mark<T>), mark, blk, 0, s, grids_dev, b, t, mask, st);
-        hipLaunchKernelGGL((k_lmax_refine<1, T>), again, blk, 0, s, grids_dev, b, t, mask, st, max_n);
-        if (third) hipLaunchKernelGGL((k_lmax_refine<2, T>), again, blk, 0, s, grids_dev, b, t, mask, st, max_n);
-        hipLaunchKernelGGL((k_lmax_collect<T>), again, blk, 0, s, grids_dev, b, t, mask, st, max_n, keys);
-        hipLaunchKernelGGL((k_lmax_select<T>), dim3((unsigned)n), dim3(kSelThreads), 0, s, grids_dev, b, t, mask, st, keys,
-                           max_n, out_dev + (long long)g0 * max_n, count_dev + g0, more);
+        // the second part goes on from the first where its marks are still there
+        if (!second || n < n_grids) {
+          clear(0, kFirstWords);
+          hipLaunchKernelGGL((k_lmax_mark<T>), mark, blk, 0, s, grids_dev, b, t, mask, st);
+          hipLaunchKernelGGL((k_lmax_refine<1, T>), again, blk, 0, s, grids_dev, b, t, mask, st, max_n);
+        }
+        if (second) {
+          clear(kSecondFrom, kStateWords);
+          hipLaunchKernelGGL((k_lmax_refine<2, T>), again, blk, 0, s, grids_dev, b, t, mask, st, max_n);
+          hipLaunchKernelGGL((k_lmax_refine<3, T>), again, blk, 0, s, grids_dev, b, t, mask, st, max_n);
+          hipLaunchKernelGGL((k_lmax_refine<4, T>), again, blk, 0, s, grids_dev, b, t, mask, st, max_n);
+          hipLaunchKernelGGL((k_lmax_refine<5, T>), again, blk, 0, s, grids_dev, b, t, mask, st, max_n);
+        }
+        if (second)
+          hipLaunchKernelGGL((k_lmax_collect<true, T>), again, blk, 0, s, grids_dev, b, t, mask, st, max_n, keys);
+        else
+          hipLaunchKernelGGL((k_lmax_collect<false, T>), again, blk, 0, s, grids_dev, b, t, mask, st, max_n, keys);
+        hipLaunchKernelGGL((k_lmax_select<T>), dim3((unsigned)n), dim3(kSelThreads), 0, s, b, t, st, keys, max_n,
+                           out_dev + (long long)g0 * max_n, count_dev + g0, more);
       };
       if (table) launch(std::true_type());
       else launch(std::false_type());
