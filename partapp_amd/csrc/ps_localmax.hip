@@ -14,6 +14,7 @@
 //   k_lmax_collect  the keys at or above that 22-bit threshold (all of them
 //                   when there are at most max_n)
 //   k_lmax_select   one workgroup per grid sorts those few in LDS
+// (k_lmax_small does all that for grids of no more points than LDS takes.)
 // Where some grid has more of those keys than LDS takes (k_lmax_select tells
 // the host), it goes on with a third histogram (the last 10 bits) and, where too
 // many values equal that threshold, with three more of their scan indices, and
@@ -427,6 +428,49 @@ __global__ __launch_bounds__(kSelThreads) void k_lmax_select(LmBatch gd, const L
   lm_write(G, s, keep, out + (long long)blockIdx.x * max_n, out_n + blockIdx.x);
 }
 
+// All of it for a grid of at most kCap points, one workgroup each: five launches
+// take such a call longer than their work (six grids of 24x25x2: 97 us a call with
+// them, 80 with one).
+template <bool TAB>
+__global__ __launch_bounds__(kSelThreads) void k_lmax_small(const float *__restrict__ grids, LmBatch gd,
+                                                            const LmGrid *__restrict__ tab, int max_n,
+                                                            ps_local_max *__restrict__ out, int *__restrict__ out_n) {
+  __shared__ unsigned long long s[kCap];
+  __shared__ unsigned fill_s;
+  const LmGrid &G = lm_grid<TAB>(gd, tab, blockIdx.x);
+  const int D = G.D, H = G.H, W = G.W, HW = H * W, n = D * HW;
+  const float *g = grids + G.off;
+  if (threadIdx.x == 0) fill_s = 0u;
+  __syncthreads();
+  for (int e = threadIdx.x; e < n; e += kSelThreads) {
+    const int d = e / HW, rem = e - d * HW, y = rem / W, x = rem - y * W;
+    const float *p = g + d * HW;
+    const int xl = max(x - 1, 0), xr = min(x + 1, W - 1);
+    // (a neighbour outside the grid is one inside the neighbourhood again;
+    // fmaxf leaves a NaN out, as the comparison with one does)
+    auto row = [&](int yy) {
+      const float *q = p + min(max(yy, 0), H - 1) * W;
+      return fmaxf(fmaxf(q[xl], q[xr]), q[x]);
+    };
+    const float c = p[rem], above = row(y - 1), below = row(y + 1), side = fmaxf(p[y * W + xl], p[y * W + xr]);
+    const float vp = d > 0 ? g[e - HW] : c, vn = d < D - 1 ? g[e + HW] : c;
+    if (!(above > c) && !(below > c) && !(side > c) && (d == 0 || vp < c) && (d == D - 1 || vn < c))
+      s[atomicAdd(&fill_s, 1u)] = lm_key(G, c, d, y, x);
+  }
+  __syncthreads();
+  const int marked = (int)fill_s, keep = min(marked, max_n);
+  const bool all = marked <= max_n;
+  int n2 = 1;
+  while (n2 < marked) n2 <<= 1;
+  for (int i = threadIdx.x; i < n2; i += kSelThreads) s[i] = i < marked ? (all ? swap_halves(s[i]) : s[i]) : 0ull;
+  bitonic_desc(s, n2);
+  if (all) {
+    for (int i = threadIdx.x; i < keep; i += kSelThreads) s[i] = swap_halves(s[i]);
+    __syncthreads();
+  }
+  lm_write(G, s, keep, out + (long long)blockIdx.x * max_n, out_n + blockIdx.x);
+}
+
 }  // namespace
 
 }  // namespace ps
@@ -484,10 +528,21 @@ extern "C" int ps_find_local_max(const float *grids_dev, const long long *offset
       const LmGrid *one = gd.data() + g0, *t = table ? tab + g0 : nullptr;
       LmBatch b;
       if (!table) std::copy(one, one + n, b.g);
-      long long tiles = 0, most = 0;
+      long long tiles = 0, most = 0, points = 0;
       for (int i = 0; i < n; ++i) {
+        points = std::max(points, (long long)one[i].D * one[i].H * one[i].W);
         tiles = std::max(tiles, (long long)one[i].D * ((one[i].H + kMarkRows - 1) / kMarkRows) * one[i].wq);
         most = std::max(most, (long long)one[i].D * one[i].H * one[i].wq);
+      }
+      if (points <= kCap) {
+        auto small = [&](auto tabc) {
+          hipLaunchKernelGGL((k_lmax_small<decltype(tabc)::value>), dim3((unsigned)n), dim3(kSelThreads), 0, s, grids_dev,
+                             b, t, max_n, out_dev + (long long)g0 * max_n, count_dev + g0);
+        };
+        if (table) small(std::true_type());
+        else small(std::false_type());
+        e = hipGetLastError();
+        continue;
       }
       // cleared by a small kernel (this entry point synchronizes and is not
       // capturable)

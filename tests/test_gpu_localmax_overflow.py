@@ -62,3 +62,33 @@ def test_many_grids(gpu, n):
     res = find_local_max([torch.from_numpy(g).to(gpu) for g in gs], 12)
     for g, r in zip(gs, res):
         assert [(int(a["d"]), int(a["x"]), int(a["y"]), float(a["score"])) for a in r] == ref(g, 12)
+
+
+# 8192 points at most: one workgroup a grid; one more, or one such grid among them: the general kernels
+@pytest.mark.parametrize("shapes", [[(2, 64, 64)], [(1, 8192, 1), (8192, 1, 1), (1, 1, 8192)], [(3, 2731, 1)],
+                                    [(2, 64, 64), (1, 1, 1), (1, 90, 92)], [(24, 18, 18), (5, 3, 40)]])
+@pytest.mark.parametrize("kind", ["noise", "few_values", "equal", "nan"])
+@pytest.mark.parametrize("max_n", [1, 25, 4096])
+def test_small_grids(gpu, shapes, kind, max_n):
+    import torch
+    rng = np.random.default_rng(len(shapes) * 10 + max_n)
+    gs = [rng.normal(0, 1, s).astype(np.float32) for s in shapes]
+    if kind == "few_values":
+        gs = [np.round(g) for g in gs]
+    elif kind == "equal":
+        gs = [np.full_like(g, -1e6) for g in gs]
+    elif kind == "nan":  # (one slice: a NaN's place among neighbours in other slices is the comparison's)
+        for g in gs:
+            g[0].flat[::13] = np.nan
+    res = find_local_max([torch.from_numpy(g).to(gpu) for g in gs], max_n)
+    for g, r in zip(gs, res):
+        if kind == "nan":
+            p = np.pad(g, ((1, 1), (1, 1), (1, 1)), constant_values=np.nan)
+            n = [p[1, 1 + dy:1 + dy + g.shape[1], 1 + dx:1 + dx + g.shape[2]] for dy in (-1, 0, 1) for dx in (-1, 0, 1)
+                 if dy or dx] if g.shape[0] == 1 else None
+            if n is None:
+                continue
+            keep = ~np.any([m > g[0] for m in n], axis=0)
+            assert len(r) == min(max_n, int(keep.sum())) and all(keep[a["y"], a["x"]] for a in r)
+        else:
+            assert [(int(a["d"]), int(a["x"]), int(a["y"]), float(a["score"])) for a in r] == ref(g, max_n)
