@@ -170,7 +170,9 @@ int ps_plan_set_method(ps_plan *plan, int method);
  *                            multiple of 64 up to 512; 0 = one per column,
  *                            the default);
  *   PS_TUNE_FP32_COL_ROWS    output rows per lane of the FP32 column pass
- *                            (8 or 16; 0 = 8, the default).
+ *                            (8 or 16; 0 = 8, the default; 8 in any case for
+ *                            grids of up to 12 rows, filters too long for the
+ *                            matrix cores and warps whose offset changes).
  * ps_plan_tune sets a knob for every launch class; ps_plan_tune_class for
  * one class; ps_plan_tune_default takes it back to its default, for one class
  * or, with cls = -1, for all.  A class is one (level, width class) row-pass launch of the
@@ -256,7 +258,7 @@ int ps_message(const ps_model *model, const float *child_dev, float *parent_dev,
  * PS_MESSAGE_NOALLOC_BYTES that the library holds on every GPU it runs on
  * until the process ends; a message that needs more (about
  * R * height * ceil32(width) * 4 bytes plus a few KB of tables, plus
- * 12 * R * th * tw bytes of eigenbasis grids for an off-diagonal C) returns
+ * 8 * R * th * ceil4(tw) bytes of eigenbasis grids for an off-diagonal C) returns
  * PS_ERR_UNSUPPORTED.  Same arguments, results and errors as ps_message;
  * synchronous.  Calls on one GPU share the array: the library serialises
  * them with a process-wide lock (overlapping calls would race on it). */

@@ -981,9 +981,10 @@ __device__ __forceinline__ void colpass_strip(const Bases &b, const MsgJob &J, c
 
   // The output rows [ya, yb) run in segments of one inverse row offset oy: up
   // to ybrk and, for a split warp, from it on.  Within a segment, tile t holds source
-  // rows s_t + [0, nrows), s_t = ylo + 64 t + oy - ky.  Tile t+1 shares rows
-  // [64, nrows) of tile t (moved to [0, Lp) in LDS) and needs 64 new rows,
-  // fetched into registers while tile t is filtered.
+  // rows s_t + [0, nrows), s_t = ylo + kColTileY t + oy - ky.  Tile t+1 shares rows
+  // [kColTileY, nrows) of tile t, which stay where they are in the ring (MFMA) or
+  // move to [0, Lp) in LDS, and needs kColTileY new rows, fetched into registers
+  // while tile t is filtered; in the ring they take the place of the oldest.
   constexpr int kNew = kColTileY / kColWaves;  // new rows per thread
   Epi<EPI> acc;
   // (the padding columns of the plan's grids are left unwritten here: the
@@ -1304,7 +1305,8 @@ __device__ __forceinline__ void root_pixels(const Bases &b, const RootJob &J, in
 // 8 waves per SIMD), not those of the widest tree
 template <int KC, bool LSE64>
 __global__ __launch_bounds__(64 * kRootWaves * kRootTiles) void k_root(Bases b, const RootJob *__restrict__ jobs, int R) {
-  extern __shared__ float4 lds4[];  // [R][64]: beliefs (FP32 sum: their exponentials)
+  // [R][64 kRootTiles] beliefs (FP32 sum: their exponentials), then the waves' keys
+  extern __shared__ float4 lds4[];
   unsigned bx, by;
   xcd_block(bx, by);
   const RootJob &J = jobs[by];

@@ -9,7 +9,7 @@
 // looks up that device's address of the array with hipGetSymbolAddress, with
 // the device current, and every later call on it reuses the stored address.
 // All calls on one GPU share its array, which keeps the last call's contents;
-// the kernels clear the two keys they accumulate into before using them, and
+// the two keys that the kernels raise arrive as zeros with the call's tables, and
 // every other byte they read was written earlier in the same call.  Calls
 // are serialised by a process-wide lock (each call is synchronous), so calls
 // from several host threads do not overlap on the array; two processes each
